@@ -179,7 +179,7 @@ int oal_selftest(int* device_errors, void* stream);
  * Same operator and layouts as oal_forward with every tensor float64: q, k, v
  * (padded to 64 features), c0 [Hq], lam [Hq][groups], gam [Hq][groups][groups]
  * (symmetric), out and num [B][Hq][N][64], den [B][Hq][N]; out = num / den, no
- * floor. Evaluated over token pairs in 32-token tiles (O(N^2) per head), for
+ * floor. Evaluated over token pairs in tiles (O(N^2) per head), for
  * validation in double precision rather than speed. No saved state: the
  * backward recomputes from q, k, v.
  */

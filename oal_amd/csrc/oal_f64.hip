@@ -23,10 +23,14 @@
 // (dgam is d/dgam of sum_{g,h} gam_gh s_g s_h, the convention of the fp32 and
 // bf16 routes; a factor's gradient is the same under the reference's gather).
 //
-// The cost is O(N^2 (64 + 64 * 64 / 4)) per head in the forward: this route is
-// for validation in double precision (gradcheck, quality sessions in float64),
-// not for speed. Tiles of 32 queries x 32 keys; a block's 128 threads are 32
-// tokens x 4 quarters, each quarter owning 16 of the 64 dimensions.
+// Up to 8 groups (kGroups) the pair values come from group sums on the fp64
+// matrix cores (the k64g_* kernels below): O(N^2 (64 + G^2)) per head. More
+// groups take the per-dimension kernels (k64_*): 64 * 64 terms a pair whatever the
+// labels, tiles of 32 queries x 32 keys, a block's 128 threads being 32 tokens x
+// 4 quarters, each quarter owning 16 of the 64 dimensions. Kernel time of one
+// forward and backward at B=1, Hq=14, Hkv=2, N=256 and 8 groups: 43.4 ms from
+// per-dimension sums (32.8 in k64_dkv's 16 blocks), 0.20 ms from group sums
+// (k64g_fwd 44, k64g_dq 76, k64g_dkv 75 us).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -460,18 +464,471 @@ __global__ __launch_bounds__(256) void k64_coef_grad(const double* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
+// Up to kGroups groups: group sums on the matrix cores.
+//
+// v_mfma_f64_16x16x4_f64 runs at the rate of the fp64 VALU, so what it buys is
+// operand traffic: one operand register per lane and k-step feeds 16 products,
+// where the per-dimension form reads 64 x 64 coefficients from LDS for every
+// pair. What bounds these kernels is fp64 issue (64 cycles a product, 4 a VALU
+// instruction): about 23 products for the group sums of a 16 x 16 tile, 16 each
+// for a contraction over the 64 dimensions or value columns, and 64 G-by-G FMAs
+// per entry.
+//
+// A wave takes 16 x 16 token tiles. The dimensions are in group-sorted order
+// (perm), 16 k-steps of 4, so a group is a range of positions: its sum takes the
+// k-steps that its range touches, with the first operand zero outside the
+// group. A tile's accumulator register r of lane l is entry
+// [4 r + l / 16][l % 16], which is, as it stands, the first operand of a product
+// over the tile's rows: k-step r, row l % 16 of the result. So a kernel that
+// sums over keys forms the tiles transposed ([key][query]) and one that sums
+// over queries forms them straight, and no tile passes through LDS.
+// A block's four waves share one row of tiles, taken in turn (tile index mod 4),
+// and add their sums in wave order at the end: a fixed order whatever the
+// device does. 14 heads of 256 tokens are 224 blocks of four waves.
+// ---------------------------------------------------------------------------
+namespace {
+
+constexpr int kG64 = 8;          // groups of these kernels
+constexpr int kM = 16;           // tile edge
+constexpr int kWv = 4;           // waves per block
+constexpr int kPairs64 = kG64 * (kG64 + 1) / 2;
+constexpr int kCo = 1 + kG64 + kPairs64;  // coefficient sums: 1, s_g, s_g s_h (g >= h)
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ d4 mma64(double a, double b, d4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// A head's coefficients and its dimensions in group order.
+struct HeadTab {
+  double c0, lam[kG64], gam[kG64][kG64];  // zero beyond the given groups
+  int perm[kD], grp[kD];                  // position -> dimension, group
+  int first[kG64 + 1];                    // group g holds positions [first[g], first[g + 1])
+};
+
+__device__ void stage_head(HeadTab& tab, const int32_t* __restrict__ labels, const double* __restrict__ c0,
+                           const double* __restrict__ lam, const double* __restrict__ gam, int G, int h) {
+  const int t = threadIdx.x;
+  if (t < kD) {
+    const int own = labels[h * kD + t], g = own < 0 ? 0 : (own >= G ? G - 1 : own);
+    int pos = 0;
+    for (int d = 0; d < kD; ++d) {
+      const int x = labels[h * kD + d], o = x < 0 ? 0 : (x >= G ? G - 1 : x);
+      pos += o < g || (o == g && d < t);
+    }
+    tab.perm[pos] = t;
+    tab.grp[pos] = g;
+  }
+  if (t < kG64 * kG64) {
+    const int a = t / kG64, b = t % kG64;
+    tab.gam[a][b] = a < G && b < G ? gam[((size_t)h * G + a) * G + b] : 0.0;
+  }
+  if (t < kG64) tab.lam[t] = t < G ? lam[(size_t)h * G + t] : 0.0;
+  if (t == 0) tab.c0 = c0 ? c0[h] : 0.0;
+  __syncthreads();
+  if (t <= kG64) {
+    int n = 0;
+    for (int d = 0; d < kD; ++d) n += tab.grp[d] < t;
+    tab.first[t] = n;
+  }
+  __syncthreads();
+}
+
+// The wave's operand of 16 rows in group order: x[s] = row (row0 + l % 16),
+// position 4 s + l / 16. Rows past N repeat row N - 1 (their entries are masked).
+__device__ __forceinline__ void load_sorted(double (&x)[16], const double* __restrict__ src, int row0, int N,
+                                            const HeadTab& tab, int lane) {
+  const int row = row0 + (lane & 15);
+  const double* p = src + (size_t)(row < N ? row : N - 1) * kD;
+#pragma unroll
+  for (int s = 0; s < 16; ++s) x[s] = p[tab.perm[4 * s + (lane >> 4)]];
+}
+
+// The same in the natural order of the dimensions (value columns, G).
+__device__ __forceinline__ void load_rows(double (&x)[16], const double* __restrict__ src, int row0, int N, int lane) {
+  const int row = row0 + (lane & 15);
+  const double* p = src + (size_t)(row < N ? row : N - 1) * kD;
+#pragma unroll
+  for (int s = 0; s < 16; ++s) x[s] = p[4 * s + (lane >> 4)];
+}
+
+// Makes the compiler read a head's table again: kept in registers over the tile
+// loop it is 144 coefficient and 256 mask registers, which spill.
+__device__ __forceinline__ void reread() { asm volatile("" ::: "memory"); }
+
+// s[g] = scale * sum over the group's positions of a[row] b[col].
+__device__ __forceinline__ void group_sums(d4 (&s)[kG64], const double (&a)[16], const double (&b)[16], double scale,
+                                           const HeadTab& tab, int lane) {
+  reread();
+  int lab[16];
+#pragma unroll
+  for (int k = 0; k < 16; ++k) lab[k] = tab.grp[4 * k + (lane >> 4)];
+#pragma unroll
+  for (int g = 0; g < kG64; ++g) {
+    const int lo = tab.first[g], hi = tab.first[g + 1];
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+      if (lo < 4 * k + 4 && hi > 4 * k) acc = mma64(lab[k] == g ? a[k] : 0.0, b[k], acc);
+    s[g] = acc * scale;
+  }
+}
+
+// t[g] = sum_h gam[g][h] s[h]
+__device__ __forceinline__ d4 quadratic_row(const d4 (&s)[kG64], const HeadTab& tab, int g) {
+  d4 t = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int h = 0; h < kG64; ++h) t += tab.gam[g][h] * s[h];
+  return t;
+}
+
+__device__ __forceinline__ d4 kappa_tile(const d4 (&s)[kG64], const HeadTab& tab) {
+  d4 kap = {tab.c0, tab.c0, tab.c0, tab.c0};
+#pragma unroll
+  for (int g = 0; g < kG64; ++g) kap += s[g] * (tab.lam[g] + quadratic_row(s, tab, g));
+  return kap;
+}
+
+// sum over the four lane groups of a column (lanes l, l + 16, l + 32, l + 48)
+__device__ __forceinline__ double column_sum(double x) {
+  x += __shfl_xor(x, 16, 64);
+  x += __shfl_xor(x, 32, 64);
+  return x;
+}
+
+// acc[cb] += sum over the tile's rows of (ds d kappa / d s_g)[row][.] y[row][.] for the
+// positions 16 cb + l % 16 of each group: the query or key gradient's products
+// in group order. tile ds, operand rows y from memory; rows past N repeat row N - 1.
+__device__ __forceinline__ void gradient_products(d4 (&acc)[4], const d4 (&s)[kG64], const d4& ds,
+                                                  const double* __restrict__ src, int row0, int N,
+                                                  const HeadTab& tab, int lane) {
+  const double* rows[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = row0 + 4 * r + (lane >> 4);
+    rows[r] = src + (size_t)(row < N ? row : N - 1) * kD;
+  }
+  reread();
+  double y[4][4];
+  int lab[4];
+#pragma unroll
+  for (int cb = 0; cb < 4; ++cb) {
+    const int pos = 16 * cb + (lane & 15), d = tab.perm[pos];
+    lab[cb] = tab.grp[pos];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) y[cb][r] = rows[r][d];
+  }
+#pragma unroll
+  for (int g = 0; g < kG64; ++g) {
+    const int lo = tab.first[g], hi = tab.first[g + 1];
+    const d4 x = ds * (tab.lam[g] + 2.0 * quadratic_row(s, tab, g));
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+      if (lo < 16 * cb + 16 && hi > 16 * cb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[cb] = mma64(x[r], lab[cb] == g ? y[cb][r] : 0.0, acc[cb]);
+      }
+  }
+}
+
+// acc[cb] += sum over the tile's rows of t[row][.] y[row][16 cb + l % 16].
+__device__ __forceinline__ void value_products(d4 (&acc)[4], const d4& t, const double* __restrict__ src, int row0,
+                                               int N, int lane) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = row0 + 4 * r + (lane >> 4);
+    const double* p = src + (size_t)(row < N ? row : N - 1) * kD + (lane & 15);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) acc[cb] = mma64(t[r], p[16 * cb], acc[cb]);
+  }
+}
+
+// The block's four accumulator sets summed in wave order through LDS; wave 0 holds the result.
+__device__ __forceinline__ void add_waves(d4 (&acc)[4], double* red, int wave, int lane) {
+  __syncthreads();
+  if (wave) {
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[((wave - 1) * 16 + 4 * cb + r) * 64 + lane] = acc[cb][r];
+  }
+  __syncthreads();
+  if (!wave) {
+    for (int w = 0; w < kWv - 1; ++w)
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[cb][r] += red[(w * 16 + 4 * cb + r) * 64 + lane];
+  }
+}
+
+constexpr int kRed = (kWv - 1) * 16 * 64;  // doubles of add_waves' scratch
+
+}  // namespace
+
+__global__ __launch_bounds__(64 * kWv) void k64g_fwd(const double* __restrict__ q, const double* __restrict__ k,
+                                                     const double* __restrict__ v,
+                                                     const int32_t* __restrict__ labels,
+                                                     const double* __restrict__ c0, const double* __restrict__ lam,
+                                                     const double* __restrict__ gam, int G, int Hq, int Hkv, int N,
+                                                     double scale, double* __restrict__ out,
+                                                     double* __restrict__ num, double* __restrict__ den) {
+  __shared__ HeadTab tab;
+  __shared__ double red[kRed];
+  __shared__ double zred[kWv][kM];
+  const int it = blockIdx.x, bh = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
+  stage_head(tab, labels, c0, lam, gam, G, h);
+  const int tq = it * kM + (lane & 15);
+  const double* ku = k + (size_t)u * N * kD;
+  const double* vu = v + (size_t)u * N * kD;
+  double qr[16];
+  load_sorted(qr, q + (size_t)bh * N * kD, it * kM, N, tab, lane);
+  d4 acc[4] = {};
+  double z = 0.0;
+  for (int jt = wave; jt <= it; jt += kWv) {
+    double kr[16];
+    load_sorted(kr, ku, jt * kM, N, tab, lane);
+    d4 s[kG64];
+    group_sums(s, kr, qr, scale, tab, lane);
+    d4 kap = kappa_tile(s, tab);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tk = jt * kM + 4 * r + (lane >> 4);
+      kap[r] = tk <= tq && tk < N ? kap[r] : 0.0;
+      z += kap[r];
+    }
+    value_products(acc, kap, vu, jt * kM, N, lane);
+  }
+  z = column_sum(z);
+  if (lane < kM) zred[wave][lane] = z;
+  add_waves(acc, red, wave, lane);
+  if (wave) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = 4 * r + (lane >> 4), row = it * kM + i;
+    if (row >= N) continue;
+    double zz = 0.0;
+    for (int w = 0; w < kWv; ++w) zz += zred[w][i];
+    const size_t o = ((size_t)bh * N + row) * kD + (lane & 15);
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      num[o + 16 * cb] = acc[cb][r];
+      out[o + 16 * cb] = acc[cb][r] / zz;
+    }
+    if ((lane & 15) == 0) den[(size_t)bh * N + row] = zz;
+  }
+}
+
+// dq of one query tile (dq may be null) and, with part given, the tile's
+// coefficient sums part[bh][it][kCo] = sum of ds {1, s_g, s_g s_h (g >= h)}.
+__global__ __launch_bounds__(64 * kWv) void k64g_dq(const double* __restrict__ q, const double* __restrict__ k,
+                                                    const double* __restrict__ v, const int32_t* __restrict__ labels,
+                                                    const double* __restrict__ lam, const double* __restrict__ gam,
+                                                    int G, int Hq, int Hkv, int N, double scale,
+                                                    const double* __restrict__ Gv, const double* __restrict__ Gz,
+                                                    double* __restrict__ dq, double* __restrict__ part) {
+  __shared__ HeadTab tab;
+  __shared__ double red[kRed];
+  __shared__ double cred[kWv][kCo];
+  const int it = blockIdx.x, bh = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
+  stage_head(tab, labels, nullptr, lam, gam, G, h);
+  const int tq = it * kM + (lane & 15);
+  const double* ku = k + (size_t)u * N * kD;
+  const double* vu = v + (size_t)u * N * kD;
+  double qr[16], gr[16];
+  load_sorted(qr, q + (size_t)bh * N * kD, it * kM, N, tab, lane);
+  load_rows(gr, Gv + (size_t)bh * N * kD, it * kM, N, lane);
+  const double gz = Gz[(size_t)bh * N + (tq < N ? tq : N - 1)];
+  d4 acc[4] = {};
+  double co[kCo];
+#pragma unroll
+  for (int c = 0; c < kCo; ++c) co[c] = 0.0;
+  for (int jt = wave; jt <= it; jt += kWv) {
+    double kr[16], vr[16];
+    load_sorted(kr, ku, jt * kM, N, tab, lane);
+    load_rows(vr, vu, jt * kM, N, lane);
+    d4 s[kG64], ds = {gz, gz, gz, gz};
+    group_sums(s, kr, qr, scale, tab, lane);
+#pragma unroll
+    for (int x = 0; x < 16; ++x) ds = mma64(vr[x], gr[x], ds);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tk = jt * kM + 4 * r + (lane >> 4);
+      ds[r] = tk <= tq && tk < N && tq < N ? ds[r] : 0.0;
+    }
+    if (dq) gradient_products(acc, s, ds * scale, ku, jt * kM, N, tab, lane);
+    if (part) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        co[0] += ds[r];
+#pragma unroll
+        for (int g = 0; g < kG64; ++g) {
+          const double x = ds[r] * s[g][r];
+          co[1 + g] += x;
+#pragma unroll
+          for (int e = 0; e <= g; ++e)
+            co[1 + kG64 + g * (g + 1) / 2 + e] = fma(x, s[e][r], co[1 + kG64 + g * (g + 1) / 2 + e]);
+        }
+      }
+    }
+  }
+  if (part) {
+#pragma unroll
+    for (int c = 0; c < kCo; ++c) {
+      double x = co[c];
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) x += __shfl_xor(x, off, 64);
+      if (lane == 0) cred[wave][c] = x;
+    }
+  }
+  add_waves(acc, red, wave, lane);
+  if (part && threadIdx.x < kCo) {
+    double x = 0.0;
+    for (int w = 0; w < kWv; ++w) x += cred[w][threadIdx.x];
+    part[((size_t)bh * gridDim.x + it) * kCo + threadIdx.x] = x;
+  }
+  if (wave || !dq) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = it * kM + 4 * r + (lane >> 4);
+    if (row >= N) continue;
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) dq[((size_t)bh * N + row) * kD + tab.perm[16 * cb + (lane & 15)]] = acc[cb][r];
+  }
+}
+
+// dk and dv of one key tile for one query head, into [B][Hq][N][64] (the heads
+// of a unit are summed by k64g_headsum). Either may be null.
+__global__ __launch_bounds__(64 * kWv) void k64g_dkv(const double* __restrict__ q, const double* __restrict__ k,
+                                                     const double* __restrict__ v,
+                                                     const int32_t* __restrict__ labels,
+                                                     const double* __restrict__ c0, const double* __restrict__ lam,
+                                                     const double* __restrict__ gam, int G, int Hq, int Hkv, int N,
+                                                     double scale, const double* __restrict__ Gv,
+                                                     const double* __restrict__ Gz, double* __restrict__ dkh,
+                                                     double* __restrict__ dvh) {
+  __shared__ HeadTab tab;
+  __shared__ double red[kRed];
+  const int jt = blockIdx.x, bh = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
+  const int NT = gridDim.x;
+  stage_head(tab, labels, c0, lam, gam, G, h);
+  const int tk = jt * kM + (lane & 15);
+  const double* qh = q + (size_t)bh * N * kD;
+  const double* gh = Gv + (size_t)bh * N * kD;
+  double kr[16], vr[16];
+  load_sorted(kr, k + (size_t)u * N * kD, jt * kM, N, tab, lane);
+  load_rows(vr, v + (size_t)u * N * kD, jt * kM, N, lane);
+  d4 ak[4] = {}, av[4] = {};
+  for (int it = jt + wave; it < NT; it += kWv) {
+    double qr[16], gr[16];
+    load_sorted(qr, qh, it * kM, N, tab, lane);
+    load_rows(gr, gh, it * kM, N, lane);
+    d4 s[kG64], ds;
+    group_sums(s, qr, kr, scale, tab, lane);
+    d4 kap = kappa_tile(s, tab);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tq = it * kM + 4 * r + (lane >> 4);
+      ds[r] = Gz[(size_t)bh * N + (tq < N ? tq : N - 1)];
+    }
+#pragma unroll
+    for (int x = 0; x < 16; ++x) ds = mma64(gr[x], vr[x], ds);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int tq = it * kM + 4 * r + (lane >> 4);
+      const bool ok = tk <= tq && tq < N && tk < N;
+      kap[r] = ok ? kap[r] : 0.0;
+      ds[r] = ok ? ds[r] * scale : 0.0;
+    }
+    if (dvh) value_products(av, kap, gh, it * kM, N, lane);
+    if (dkh) gradient_products(ak, s, ds, qh, it * kM, N, tab, lane);
+  }
+  add_waves(ak, red, wave, lane);
+  add_waves(av, red, wave, lane);
+  if (wave) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = jt * kM + 4 * r + (lane >> 4);
+    if (row >= N) continue;
+    const size_t o = ((size_t)bh * N + row) * kD;
+#pragma unroll
+    for (int cb = 0; cb < 4; ++cb) {
+      const int c = 16 * cb + (lane & 15);
+      if (dkh) dkh[o + tab.perm[c]] = ak[cb][r];
+      if (dvh) dvh[o + c] = av[cb][r];
+    }
+  }
+}
+
+// dst[b][kv head][n][d] = sum over the unit's R query heads, in head order, of
+// src[b][head][n][d]; blockIdx.y 0: (src0, dst0), 1: (src1, dst1).
+__global__ __launch_bounds__(256) void k64g_headsum(const double* __restrict__ src0, const double* __restrict__ src1,
+                                                    int R, size_t per_head, size_t total, double* __restrict__ dst0,
+                                                    double* __restrict__ dst1) {
+  const double* src = blockIdx.y ? src1 : src0;
+  double* dst = blockIdx.y ? dst1 : dst0;
+  const size_t x = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (!dst || x >= total) return;
+  const double* p = src + (x / per_head) * R * per_head + x % per_head;
+  double acc = 0.0;
+  for (int r = 0; r < R; ++r) acc += p[(size_t)r * per_head];
+  dst[x] = acc;
+}
+
+// dc0, dlam, dgam of head h from the tiles' sums, added over (batch, tile): each
+// wave a fixed share of them, lane by lane, then lanes and waves in a fixed order.
+__global__ __launch_bounds__(256) void k64g_coef_grad(const double* __restrict__ part, int B, int Hq, int NT, int G,
+                                                      double* __restrict__ dc0, double* __restrict__ dlam,
+                                                      double* __restrict__ dgam) {
+  __shared__ double w[kCo];
+  const int h = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int c = wave; c < kCo; c += 4) {
+    double x = 0.0;
+    for (int i = lane; i < B * NT; i += 64) {
+      const int b = i / NT, it = i % NT;
+      x += part[((size_t)(b * Hq + h) * NT + it) * kCo + c];
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) x += __shfl_xor(x, off, 64);
+    if (lane == 0) w[c] = x;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) dc0[h] = w[0];
+  for (int e = threadIdx.x; e < G; e += 256) dlam[(size_t)h * G + e] = w[1 + e];
+  for (int e = threadIdx.x; e < G * G; e += 256) {
+    const int a = e / G, c = e % G, hi = a > c ? a : c, lo = a > c ? c : a;
+    dgam[(size_t)h * G * G + e] = w[1 + kG64 + hi * (hi + 1) / 2 + lo];
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Host launches.
 // ---------------------------------------------------------------------------
-size_t f64_workspace_bytes(int B, int Hq, int N) {
+size_t f64_workspace_bytes(int B, int Hq, int N, int G) {
   const size_t rows = (size_t)B * Hq * N;
-  const size_t NT = (size_t)(N + kT - 1) / kT;
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
-  return al(sizeof(double) * rows * kD) + al(sizeof(double) * rows) + al(sizeof(double) * B * Hq * NT * kFP);
+  const size_t grads = al(sizeof(double) * rows * kD) + al(sizeof(double) * rows);
+  // group sums: dk and dv per query head, coefficient sums per 16-token tile
+  if (G <= kG64)
+    return grads + 2 * al(sizeof(double) * rows * kD) + al(sizeof(double) * B * Hq * ((N + kM - 1) / kM) * kCo);
+  const size_t NT = (size_t)(N + kT - 1) / kT;
+  return grads + al(sizeof(double) * B * Hq * NT * kFP);
 }
 
 void launch_f64_forward(const F64Geom& g, const double* q, const double* k, const double* v, const int32_t* labels,
                         const double* c0, const double* lam, const double* gam, int G, double scale, double* out,
                         double* num, double* den, hipStream_t st, const Timer& timed) {
+  if (G <= kG64) {
+    timed("k64g_fwd", st, [&] {
+      hipLaunchKernelGGL(k64g_fwd, dim3((g.N + kM - 1) / kM, g.B * g.Hq), dim3(64 * kWv), 0, st, q, k, v, labels, c0,
+                         lam, gam, G, g.Hq, g.Hkv, g.N, scale, out, num, den);
+    });
+    return;
+  }
   const int NT = (g.N + kT - 1) / kT;
   timed("k64_fwd", st, [&] {
     hipLaunchKernelGGL(k64_fwd, dim3(NT, g.B * g.Hq), dim3(kNT), 0, st, q, k, v, labels, c0, lam, gam, G, g.Hq,
@@ -484,19 +941,56 @@ void launch_f64_backward(const F64Geom& g, const double* q, const double* k, con
                          double scale, const double* num, const double* den, const double* dout,
                          const double* dnum, const double* dden, double* dq, double* dk, double* dv, double* dc0,
                          double* dlam, double* dgam, void* workspace, hipStream_t st, const Timer& timed) {
-  const int NT = (g.N + kT - 1) / kT;
   const size_t rows = (size_t)g.B * g.Hq * g.N;
-  auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
   char* p = static_cast<char*>(workspace);
-  double* Gv = reinterpret_cast<double*>(p);
-  p += al(sizeof(double) * rows * kD);
-  double* Gz = reinterpret_cast<double*>(p);
-  p += al(sizeof(double) * rows);
-  double* part = reinterpret_cast<double*>(p);
+  auto take = [&](size_t n) {
+    double* x = reinterpret_cast<double*>(p);
+    p += (n * sizeof(double) + 255) & ~size_t(255);
+    return x;
+  };
+  double* Gv = take(rows * kD);
+  double* Gz = take(rows);
   timed("k64_gvec", st, [&] {
     hipLaunchKernelGGL(k64_gvec, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, dout, dnum, dden, num, den,
                        (long)rows, Gv, Gz);
   });
+  if (G <= kG64) {
+    const int NM = (g.N + kM - 1) / kM, R = g.Hq / g.Hkv;
+    double* dkh = take(rows * kD);
+    double* dvh = take(rows * kD);
+    double* part = take((size_t)g.B * g.Hq * NM * kCo);
+    const dim3 grid(NM, g.B * g.Hq), block(64 * kWv);
+    if (dq || dc0) {
+      timed("k64g_dq", st, [&] {
+        hipLaunchKernelGGL(k64g_dq, grid, block, 0, st, q, k, v, labels, lam, gam, G, g.Hq, g.Hkv, g.N, scale, Gv, Gz,
+                           dq, dc0 ? part : nullptr);
+      });
+    }
+    if (dk || dv) {
+      // one query head per KV head: the head's sums are the results
+      double* dk1 = R == 1 ? dk : dk ? dkh : nullptr;
+      double* dv1 = R == 1 ? dv : dv ? dvh : nullptr;
+      timed("k64g_dkv", st, [&] {
+        hipLaunchKernelGGL(k64g_dkv, grid, block, 0, st, q, k, v, labels, c0, lam, gam, G, g.Hq, g.Hkv, g.N, scale,
+                           Gv, Gz, dk1, dv1);
+      });
+      if (R > 1) {
+        const size_t per_head = (size_t)g.N * kD, total = (size_t)g.B * g.Hkv * per_head;
+        timed("k64g_headsum", st, [&] {
+          hipLaunchKernelGGL(k64g_headsum, dim3((unsigned)((total + 255) / 256), 2), dim3(256), 0, st, dkh, dvh, R,
+                             per_head, total, dk, dv);
+        });
+      }
+    }
+    if (dc0) {
+      timed("k64g_coef_grad", st, [&] {
+        hipLaunchKernelGGL(k64g_coef_grad, dim3(g.Hq), dim3(256), 0, st, part, g.B, g.Hq, NM, G, dc0, dlam, dgam);
+      });
+    }
+    return;
+  }
+  const int NT = (g.N + kT - 1) / kT;
+  double* part = take((size_t)g.B * g.Hq * NT * kFP);
   if (dq) {
     timed("k64_dq", st, [&] {
       hipLaunchKernelGGL(k64_dq, dim3(NT, g.B * g.Hq), dim3(kNT), 0, st, q, k, v, labels, lam, gam, G, g.Hq, g.Hkv,

@@ -296,7 +296,7 @@ int run_mfma_selftest(int* dev_errors, hipStream_t st);
 struct F64Geom {
   int B, Hq, Hkv, N;
 };
-size_t f64_workspace_bytes(int B, int Hq, int N);
+size_t f64_workspace_bytes(int B, int Hq, int N, int G);
 void launch_f64_forward(const F64Geom& g, const double* q, const double* k, const double* v, const int32_t* labels,
                         const double* c0, const double* lam, const double* gam, int G, double scale, double* out,
                         double* num, double* den, hipStream_t st, const Timer& timed);

@@ -215,6 +215,33 @@ def test_grouped_function_fwd_bwd_multi_tile_ragged_gqa(groups):
         assert e <= 1e-11, (name, e)
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 65, 129])
+@pytest.mark.parametrize("hq,hkv,sizes", [(3, 1, (64,)), (2, 2, (1, 62, 1)), (2, 1, (3, 5, 1, 20, 16, 2, 9, 8))])
+def test_group_sum_tiles_at_their_edges(n, hq, hkv, sizes):
+    """Lengths around the 16-token tile and its four-wave turn; one group, groups
+    that share k-steps, one of them spanning several column blocks; the sums of
+    a unit's heads. The bound: 64 N terms a sum, each to 1.1e-16, is 9e-13 at
+    N = 129; 1e-11 leaves the quotients their conditioning."""
+    from oal_amd.hd_block_gemm_autograd import grouped_oal_f64
+
+    dev = _dev()
+    q, k, v, labels, c0, lam, gam = _grouped_case(
+        2, hq, hkv, n, lambda gen: torch.stack([go.seeded_groups(64, sizes, gen) for _ in range(hq)]), len(sizes), seed=n)
+    leaves = [t.to(dev).requires_grad_() for t in (q, k, v, c0, lam, gam)]
+    out, num, den = grouped_oal_f64(leaves[0], leaves[1], leaves[2], labels.to(dev), *leaves[3:], scale=0.125)
+    gen = torch.Generator().manual_seed(n)
+    dout, dden = (torch.randn(t.shape, generator=gen, dtype=torch.float64) for t in (out, den))
+    torch.autograd.backward((out, den), (dout.to(dev), dden.to(dev)))
+    ref = [t.clone().requires_grad_() for t in (q, k, v, c0, lam, gam)]
+    num_r, den_r = go.dense_forward_coefficients(ref[0], ref[1], ref[2], labels, *ref[3:], scale=0.125)
+    torch.autograd.backward((num_r / den_r, den_r), (dout, dden))
+    want = [num_r / den_r, num_r, den_r] + [t.grad for t in ref[:5]] + [go.symmetrize_gamma_gradient(ref[5].grad)]
+    for name, a, r in zip(("out", "num", "den", "dq", "dk", "dv", "dc0", "dlam", "dgam"),
+                          [out, num, den] + [t.grad for t in leaves], want):
+        err = float((a.detach().cpu() - r.detach()).norm() / r.detach().norm())
+        assert err <= 1e-11, (name, err)
+
+
 def test_partial_requests_and_reruns_are_bitwise_identical():
     from oal_amd import _native
     from oal_amd.hd_block_gemm_autograd import pad_labels
