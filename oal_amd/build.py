@@ -19,13 +19,13 @@ SOURCES = [os.path.join(PKG, "csrc", "oal_kernels.hip"), os.path.join(PKG, "csrc
            os.path.join(PKG, "csrc", "oal_mfma_bwd.hip"), os.path.join(PKG, "csrc", "oal_mfma_local.hip"),
            os.path.join(PKG, "csrc", "oal_mfma_scan.hip"), os.path.join(PKG, "csrc", "oal_mfma_den.hip"),
            os.path.join(PKG, "csrc", "oal_mfma_pair.hip"), os.path.join(PKG, "csrc", "oal_f32_mma.hip"),
-           os.path.join(PKG, "csrc", "oal_f64.hip")]
+           os.path.join(PKG, "csrc", "oal_f64.hip"), os.path.join(PKG, "csrc", "oal_direct.hip")]
 # Sources whose matrix-core accumulators the compiler would otherwise place in
 # the accumulation registers (AGPRs): there every VALU use of a group sum needs
 # a v_accvgpr_read copy first (256 of them per tile in the intra-chunk forward).
 # In VGPRs the VALU reads them directly; each kernel in these files stays
 # within 256 VGPRs without spilling.
-VGPR_FORM = {"oal_mfma_fwd.hip", "oal_mfma_local.hip"}
+VGPR_FORM = {"oal_mfma_fwd.hip", "oal_mfma_local.hip", "oal_direct.hip"}
 HEADERS = [os.path.join(PKG, "csrc", "oal_common.hpp"), os.path.join(ROOT, "include", "oal_amd.h")]
 OUTPUT = os.path.join(PKG, "liboal_amd.so")
 OBJDIR = os.path.join(PKG, "_build")

@@ -1,0 +1,49 @@
+// The direct route: evaluation over token pairs for short sequences
+// (oal_direct.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "oal_internal.hpp"
+
+namespace oal {
+
+constexpr int kDirectTile = 16;  // tokens per tile edge
+
+// Whether a call takes the direct route: where a model of both routes' forward
+// and backward time on MI355X (microseconds, kernels alone) says that it is the
+// shorter one. A function of the geometry alone, so that the size queries and
+// both directions agree. A direct call costs its launches and the longest row,
+// its 16 x 16 tiles and its blocks of 16 rows; the state route its longer chain
+// of launches and its rows. Measured, bf16, 14/2 heads and 8 groups, direct
+// against state: B=1 N=128 49 / 216, N=512 87 / 237, N=1024 190 / 255, N=1536
+// 334 / 266; B=2 N=800 210 / 276, N=1000 297 / 269; B=8 N=512 413 / 319; B=64
+// N=128 393 / 458. fp32: B=1 N=256 90 / 438, N=1024 400 / 581, N=1536 744 / 674;
+// B=4 N=512 502 / 800, N=1024 1343 / 1241; B=64 N=256 2440 / 3818. Up to 4
+// groups: bf16 B=4 N=512 170 / 257, fp32 B=4 N=1024 777 / 1159.
+inline bool direct_route(bool f32, int groups, int B, int Hq, int N) {
+  if (groups > 8 || (long)B * Hq > 65535) return false;
+  const double nt = (N + kDirectTile - 1) / kDirectTile, blocks = (double)B * Hq * nt, tiles = blocks * (nt + 1) / 2,
+               rows = (double)B * Hq * N;
+  const bool few = groups <= 4;
+  if (f32) return 60 + 0.03 * N + (few ? 0.0042 : 0.0082) * tiles + (few ? 0.06 : 0.085) * blocks < 420 + 0.0145 * rows;
+  return 30 + 0.03 * N + (few ? 0.0029 : 0.0042) * tiles + 0.031 * blocks < 200 + 0.0028 * rows;
+}
+
+// Workspace of a direct backward.
+size_t direct_work_bytes(bool f32, int B, int Hq, int N);
+
+// F32: fp32 arithmetic, else bf16 operands with fp32 accumulation.
+template <typename T, bool F32>
+void launch_direct_forward(const LaunchGeom& g, const T* q, const T* k, const T* v, const int32_t* labels,
+                           const float* c0, const float* lam, const float* gam, int groups, float scale, float floor,
+                           T* out, float* num, float* den, hipStream_t st, const Timer& timed);
+template <typename T, bool F32>
+void launch_direct_backward(const LaunchGeom& g, const T* q, const T* k, const T* v, const int32_t* labels,
+                            const float* c0, const float* lam, const float* gam, int groups, float scale, float floor,
+                            const float* num, const float* den, const T* dout, const float* dnum, const float* dden,
+                            T* dq, T* dk, T* dv, float* dc0, float* dlam, float* dgam, void* workspace, hipStream_t st,
+                            const Timer& timed);
+
+}  // namespace oal

@@ -30,6 +30,7 @@
 
 #include "oal_amd.h"
 #include "oal_common.hpp"
+#include "oal_direct.hpp"
 #include "oal_internal.hpp"
 
 namespace oal {
@@ -798,6 +799,10 @@ bool use_mfma(int precision, int groups, const Geometry& g) {
   return precision == OAL_PRECISION_BF16 && groups <= 64 && g.R <= 8;
 }
 
+bool use_direct(int precision, int groups, const Geometry& g) {
+  return oal::direct_route(!use_mfma(precision, groups, g), groups, g.B, g.Hq, g.N);
+}
+
 oal::LaunchGeom launch_geom(const Geometry& g) { return oal::LaunchGeom{g.B, g.Hq, g.Hkv, g.N, g.NB, g.U, g.R}; }
 
 // Second stream and fork/join events per device, created on first use and kept
@@ -884,6 +889,27 @@ namespace {
 
 oal::Timer make_timer() {
   return [](const char* name, hipStream_t st, const std::function<void()>& launch) { timed(name, st, launch); };
+}
+
+// The direct route of both entry points (oal_direct.hip): every kernel on the
+// caller's stream.
+template <typename T, bool F32>
+void direct_forward(const Geometry& g, const void* q, const void* k, const void* v, const int32_t* labels,
+                    const float* c0, const float* lam, const float* gam, int groups, float scale, float floor, void* out,
+                    float* num, float* den, hipStream_t st) {
+  oal::launch_direct_forward<T, F32>(launch_geom(g), static_cast<const T*>(q), static_cast<const T*>(k),
+                                     static_cast<const T*>(v), labels, c0, lam, gam, groups, scale, floor,
+                                     static_cast<T*>(out), num, den, st, make_timer());
+}
+template <typename T, bool F32>
+void direct_backward(const Geometry& g, const void* q, const void* k, const void* v, const int32_t* labels,
+                     const float* c0, const float* lam, const float* gam, int groups, float scale, float floor,
+                     const float* num, const float* den, const void* dout, const float* dnum, const float* dden, void* dq,
+                     void* dk, void* dv, float* dc0, float* dlam, float* dgam, void* workspace, hipStream_t st) {
+  oal::launch_direct_backward<T, F32>(launch_geom(g), static_cast<const T*>(q), static_cast<const T*>(k),
+                                      static_cast<const T*>(v), labels, c0, lam, gam, groups, scale, floor, num, den,
+                                      static_cast<const T*>(dout), dnum, dden, static_cast<T*>(dq), static_cast<T*>(dk),
+                                      static_cast<T*>(dv), dc0, dlam, dgam, workspace, st, make_timer());
 }
 
 template <typename T, int GMAX>
@@ -1087,6 +1113,8 @@ size_t oal_forward_saved_bytes(int batch, int q_heads, int kv_heads, int seq_len
                                int precision) {
   Geometry g;
   if (check_geometry(batch, q_heads, kv_heads, seq_len, dtype, &g) || check_common(groups, precision)) return 0;
+  // the direct route's backward starts from q, k, v, num and den alone; a byte count of 0 means an error
+  if (use_direct(precision, groups, g)) return 256;
   if (use_mfma(precision, groups, g)) return oal::mfma_saved_bytes(g.Hq, g.U, g.NB, g.R);
   return saved_bytes(g);
 }
@@ -1095,6 +1123,7 @@ size_t oal_backward_workspace_bytes(int batch, int q_heads, int kv_heads, int se
                                     int precision) {
   Geometry g;
   if (check_geometry(batch, q_heads, kv_heads, seq_len, dtype, &g) || check_common(groups, precision)) return 0;
+  if (use_direct(precision, groups, g)) return oal::direct_work_bytes(!use_mfma(precision, groups, g), g.B, g.Hq, g.N);
   if (use_mfma(precision, groups, g))
     return oal::mfma_work_view(nullptr, g.B, g.Hq, g.U, g.N, g.NB, groups > 8).bytes;
   return work_view(g, nullptr, f32_mma(groups)).bytes;
@@ -1114,6 +1143,20 @@ int oal_forward(const void* q, const void* k, const void* v, const int32_t* labe
     if (!aligned16(p)) return fail("oal_forward: tensor pointers must be 16-byte aligned");
   if (check_common(groups, precision)) return 1;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (use_direct(precision, groups, g)) {
+    if (use_mfma(precision, groups, g)) {
+      if (dtype == OAL_DTYPE_F32)
+        direct_forward<float, false>(g, q, k, v, labels, c0, lam, gam, groups, scale, floor, out, num, den, st);
+      else
+        direct_forward<uint16_t, false>(g, q, k, v, labels, c0, lam, gam, groups, scale, floor, out, num, den, st);
+    } else {
+      if (dtype == OAL_DTYPE_F32)
+        direct_forward<float, true>(g, q, k, v, labels, c0, lam, gam, groups, scale, floor, out, num, den, st);
+      else
+        direct_forward<uint16_t, true>(g, q, k, v, labels, c0, lam, gam, groups, scale, floor, out, num, den, st);
+    }
+    return launch_status("oal_forward launch");
+  }
   if (use_mfma(precision, groups, g)) {
     const oal::LaunchGeom lg = launch_geom(g);
     if (dtype == OAL_DTYPE_F32)
@@ -1158,6 +1201,27 @@ int backward_entry(const void* q, const void* k, const void* v, const int32_t* l
   // argument combinations the kernels cannot serve are refused before anything is enqueued
   if ((dc0 || dlam || dgam) && !(dc0 && dlam && dgam)) return fail("dc0, dlam and dgam must be given together");
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (use_direct(precision, groups, g)) {
+    const bool mfma = use_mfma(precision, groups, g);
+    if (mfma && (dk != nullptr) != (dv != nullptr))
+      return fail("oal_backward: dk and dv must be requested together on the matrix-core path");
+#define OAL_DIRECT_ARGS                                                                                             \
+  g, q, k, v, labels, c0, lam, gam, groups, scale, floor, num, den, dout, dnum, dden, dq, dk, dv, dc0, dlam, dgam, \
+      workspace, st
+    if (mfma) {
+      if (dtype == OAL_DTYPE_F32)
+        direct_backward<float, false>(OAL_DIRECT_ARGS);
+      else
+        direct_backward<uint16_t, false>(OAL_DIRECT_ARGS);
+    } else {
+      if (dtype == OAL_DTYPE_F32)
+        direct_backward<float, true>(OAL_DIRECT_ARGS);
+      else
+        direct_backward<uint16_t, true>(OAL_DIRECT_ARGS);
+    }
+#undef OAL_DIRECT_ARGS
+    return launch_status("oal_backward launch");
+  }
   if (use_mfma(precision, groups, g)) {
     if ((dk != nullptr) != (dv != nullptr))
       return fail("oal_backward: dk and dv must be requested together on the matrix-core path");
