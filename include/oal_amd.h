@@ -205,6 +205,40 @@ int oal_backward_f64(const double* q, const double* k, const double* v,
                      double* dq, double* dk, double* dv, double* dc0, double* dlam, double* dgam,
                      void* workspace, void* stream);
 
+/*
+ * What a call around the operator needs besides it, one launch each; wide:
+ * float64 instead of float32 operands.
+ *
+ * oal_expand_factor: packed lower-triangular factors L (row-major, side groups
+ * + 1; [P], or [Hq][P] with per_head) -> c0 [Hq] = M_00 + eps, lam [Hq][groups] =
+ * 2 M_0,1.., gam [Hq][groups][groups] = M_1..,1.., M = L L^T (reference
+ * grouped_quadratic.py:184-218); gam comes out exactly symmetric.
+ * oal_expand_factor_backward: its VJP into dfactor (the factor's shape); each
+ * of dc0, dlam and dgam may be NULL.
+ */
+int oal_expand_factor(const void* factor, int wide, int per_head, int q_heads, int groups, double eps,
+                      void* c0, void* lam, void* gam, void* stream);
+int oal_expand_factor_backward(const void* factor, int wide, int per_head, int q_heads, int groups,
+                               const void* dc0, const void* dlam, const void* dgam, void* dfactor, void* stream);
+
+/*
+ * Checks that report into *flag, an int that the device can write and the
+ * caller zeroed (host-mapped memory serves): bits are only ever set, so the
+ * caller reads them once after synchronizing the stream.
+ *
+ * oal_check_labels: labels [head_dim], or [Hq][head_dim] with per_head, int32
+ * (int64 when wide) -> table [Hq][64] int32, padded with zeros; bit 0: an id
+ * outside [0, groups), bit 1: a row's ids are not 0 .. some maximum.
+ * oal_check_outputs: num and out (each may be NULL) of rows x width values with
+ * their row strides, den [rows]; out_kind 0 float32, 1 bfloat16, 2 float16, 3
+ * float64. Bit 0: num or den not finite, bit 1: a den not positive, bit 2: out
+ * not finite.
+ */
+int oal_check_labels(const void* labels, int wide, int per_head, int head_dim, int q_heads, int groups,
+                     int32_t* table, int* flag, void* stream);
+int oal_check_outputs(int wide, int out_kind, const void* num, const void* den, const void* out, size_t rows,
+                      int width, int num_stride, int out_stride, int* flag, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -70,6 +70,10 @@ _SIGNATURES = {
          _vp, _vp, _vp, _vp, _vp, _vp, _vp],
         _i,
     ),
+    "oal_expand_factor": ([_vp, _i, _i, _i, _i, ctypes.c_double, _vp, _vp, _vp, _vp], _i),
+    "oal_expand_factor_backward": ([_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp], _i),
+    "oal_check_labels": ([_vp, _i, _i, _i, _i, _i, _vp, _vp, _vp], _i),
+    "oal_check_outputs": ([_i, _i, _vp, _vp, _vp, _sz, _i, _i, _i, _vp, _vp], _i),
 }
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
@@ -479,3 +483,115 @@ def backward_f64(q, k, v, labels, c0, lam, gam, num, den, dout, dnum, dden, *, s
         )
         _check(rc, lib, "oal_backward_f64")
     return dq, dk, dv, dc0, dlam, dgam
+
+
+# ---------------------------------------------------------------------------
+# Adapter entry points: factor expansion and its VJP, checks of labels and outputs.
+# ---------------------------------------------------------------------------
+_OUT_KINDS = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2, torch.float64: 3}
+
+
+def expand_factor(factor: torch.Tensor, query_heads: int, groups: int, eps: float):
+    """(c0 [Hq], lam [Hq, G], gam [Hq, G, G]) of a contiguous float32 or float64
+    packed factor [P] or [Hq, P] on a ROCm device, in its dtype."""
+    lib = load_library()
+    _require_device(factor)
+    side = groups + 1
+    shape = (side * (side + 1) // 2,) if factor.ndim == 1 else (query_heads, side * (side + 1) // 2)
+    if factor.dtype not in (torch.float32, torch.float64):
+        raise RuntimeError("factor must be float32 or float64")
+    _check_tensor(factor, "factor", dtype=factor.dtype, shape=shape)
+    with torch.cuda.device(factor.device):
+        c0, lam, gam = (factor.new_empty(s) for s in ((query_heads,), (query_heads, groups),
+                                                      (query_heads, groups, groups)))
+        rc = lib.oal_expand_factor(_ptr(factor), int(factor.dtype == torch.float64), int(factor.ndim == 2), query_heads,
+                                   groups, float(eps), _ptr(c0), _ptr(lam), _ptr(gam), _stream(factor.device))
+        _check(rc, lib, "oal_expand_factor")
+    return c0, lam, gam
+
+
+def expand_factor_backward(factor: torch.Tensor, query_heads: int, groups: int, dc0, dlam, dgam) -> torch.Tensor:
+    """The VJP of :func:`expand_factor`; a gradient given as None counts as zero."""
+    lib = load_library()
+    _require_device(factor)
+    shapes = ((query_heads,), (query_heads, groups), (query_heads, groups, groups))
+    grads = []
+    for name, t, shape in zip(("dc0", "dlam", "dgam"), (dc0, dlam, dgam), shapes):
+        if t is not None:
+            t = t.to(factor.dtype).contiguous()
+            _check_tensor(t, name, dtype=factor.dtype, shape=shape, device=factor.device)
+        grads.append(t)
+    with torch.cuda.device(factor.device):
+        dfactor = torch.empty_like(factor)
+        rc = lib.oal_expand_factor_backward(_ptr(factor), int(factor.dtype == torch.float64), int(factor.ndim == 2),
+                                            query_heads, groups, *(_ptr(t) for t in grads), _ptr(dfactor),
+                                            _stream(factor.device))
+        _check(rc, lib, "oal_expand_factor_backward")
+    return dfactor
+
+
+class Verdict:
+    """Host-mapped words that checks enqueued on the current stream of a device
+    set bits in; :meth:`read` synchronizes that stream. One per call: the words
+    live until the kernels that may write them are done."""
+
+    def __init__(self, device: torch.device):
+        self._pending = False
+        self._words = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+        self._stream = torch.cuda.current_stream(device)
+        self._device = device
+
+    def check_labels(self, labels: torch.Tensor, query_heads: int, groups: int) -> torch.Tensor:
+        """Enqueue the check of [D] or [Hq, D] int32 or int64 labels (D <= 64);
+        returns the int32 [Hq, 64] table that the kernels read."""
+        lib = load_library()
+        labels = labels.contiguous()
+        with torch.cuda.device(self._device):
+            table = torch.empty((query_heads, HEAD_DIM), dtype=torch.int32, device=self._device)
+            self._pending = True
+            rc = lib.oal_check_labels(_ptr(labels), int(labels.dtype == torch.int64), int(labels.ndim == 2),
+                                      labels.shape[-1], query_heads, groups, _ptr(table), self._words.data_ptr(),
+                                      self._stream.cuda_stream)
+            _check(rc, lib, "oal_check_labels")
+        return table
+
+    def check_outputs(self, num, den: torch.Tensor, out) -> None:
+        """Enqueue the check of den and, where given, of num and out ([..., DV])."""
+        lib = load_library()
+        width, strides = 1, []
+        tensors = []
+        for t in (num, out):
+            if t is not None:
+                t = t.detach()
+                width = t.shape[-1]
+                # rows one stride apart: contiguous, or a slice of wider rows
+                row = t.stride(-2) if t.ndim > 1 else width
+                regular = t.stride(-1) == 1 and all(
+                    t.stride(i) == t.stride(i + 1) * t.shape[i + 1] for i in range(t.ndim - 2))
+                if not regular:
+                    t, row = t.contiguous(), width
+                strides.append(row)
+            else:
+                strides.append(0)
+            tensors.append(t)
+        den = den.detach().contiguous()
+        kind = 0 if out is None else _OUT_KINDS[out.dtype]
+        with torch.cuda.device(self._device):
+            self._pending = True
+            rc = lib.oal_check_outputs(int(den.dtype == torch.float64), kind, _ptr(tensors[0]), _ptr(den),
+                                       _ptr(tensors[1]), den.numel(), width, strides[0], strides[1],
+                                       self._words.data_ptr() + 4, self._stream.cuda_stream)
+            _check(rc, lib, "oal_check_outputs")
+
+    def __del__(self):
+        # an abandoned check (an error in between) may still write its words
+        if self._pending:
+            self._stream.synchronize()
+
+    def read(self) -> tuple[int, int]:
+        """(label bits, output bits) of the checks enqueued so far."""
+        if self._pending:
+            self._stream.synchronize()
+            self._pending = False
+        labels, outputs = self._words.tolist()
+        return labels, outputs

@@ -19,7 +19,8 @@ SOURCES = [os.path.join(PKG, "csrc", "oal_kernels.hip"), os.path.join(PKG, "csrc
            os.path.join(PKG, "csrc", "oal_mfma_bwd.hip"), os.path.join(PKG, "csrc", "oal_mfma_local.hip"),
            os.path.join(PKG, "csrc", "oal_mfma_scan.hip"), os.path.join(PKG, "csrc", "oal_mfma_den.hip"),
            os.path.join(PKG, "csrc", "oal_mfma_pair.hip"), os.path.join(PKG, "csrc", "oal_f32_mma.hip"),
-           os.path.join(PKG, "csrc", "oal_f64.hip"), os.path.join(PKG, "csrc", "oal_direct.hip")]
+           os.path.join(PKG, "csrc", "oal_f64.hip"), os.path.join(PKG, "csrc", "oal_direct.hip"),
+           os.path.join(PKG, "csrc", "oal_adapter.hip")]
 # Sources whose matrix-core accumulators the compiler would otherwise place in
 # the accumulation registers (AGPRs): there every VALU use of a group sum needs
 # a v_accvgpr_read copy first (256 of them per tile in the intra-chunk forward).

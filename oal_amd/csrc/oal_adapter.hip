@@ -1,0 +1,255 @@
+// Small kernels around the operator for gfx950: what a call of the public entry
+// points needs besides the attention itself, each in one launch.
+//
+//   k_expand_factor      packed lower-triangular factor L -> c0 = M_00 + eps,
+//                        lam = 2 M_0,1.., gam = M_1..,1.. with M = L L^T
+//                        (reference grouped_quadratic.py:184-218)
+//   k_expand_factor_bwd  its VJP, dL = (dM + dM^T) L on the lower triangle
+//   k_check_labels       group labels -> int32 [Hq][64], and whether they are valid
+//                        (reference grouped_quadratic.py:136-181)
+//   k_check_outputs      whether num, den and out are finite and den positive
+//                        (reference grouped_quadratic.py:379-397,
+//                        hd_block_gemm_runtime.py:392-408)
+//
+// All are bound by their launch: a few hundred values, or one pass over the
+// outputs. As torch operations the expansion took 14 launches and its VJP about 20,
+// the checks 3 to 14 launches with 2 to 5 host synchronizations, 190 us of host
+// time in a forward of 266 us at N = 128. A check writes its verdict into a
+// host-mapped word only when something is wrong, so the host needs one
+// synchronization and no copy.
+
+#include <hip/hip_fp16.h>
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <algorithm>
+
+#include "oal_common.hpp"
+#include "oal_internal.hpp"
+
+namespace oal {
+
+namespace {
+
+constexpr int kSideMax = kD + 1;
+constexpr int kPackMax = kSideMax * (kSideMax + 1) / 2;
+constexpr int kThreads = 256;
+
+__device__ __forceinline__ int packed(int i, int m) { return i * (i + 1) / 2 + m; }
+
+}  // namespace
+
+// One block per query head, the sums in fp64 (a few hundred terms, no time). M[i][j] and M[j][i] are the same sum in the same
+// order, so gam is exactly symmetric (the intra-chunk kernels rely on it).
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_expand_factor(const T* __restrict__ factor, bool per_head, int G, T eps,
+                                                            T* __restrict__ c0, T* __restrict__ lam,
+                                                            T* __restrict__ gam) {
+  __shared__ T L[kPackMax];
+  const int h = blockIdx.x, side = G + 1, P = side * (side + 1) / 2;
+  const T* src = factor + (per_head ? (size_t)h * P : 0);
+  for (int x = threadIdx.x; x < P; x += kThreads) L[x] = src[x];
+  __syncthreads();
+  for (int x = threadIdx.x; x < side * side; x += kThreads) {
+    const int i = x / side, j = x % side, n = i < j ? i : j;
+    double acc = 0;
+    for (int m = 0; m <= n; ++m) acc += (double)L[packed(i, m)] * L[packed(j, m)];
+    if (x == 0)
+      c0[h] = (T)(acc + eps);
+    else if (i == 0)
+      lam[(size_t)h * G + j - 1] = (T)(2 * acc);
+    else if (j > 0)
+      gam[((size_t)h * G + i - 1) * G + j - 1] = (T)acc;
+  }
+}
+
+// dL_im = sum_{j >= m} (dM_ij + dM_ji) L_jm; a shared factor's gradient is the
+// sum over the heads in order, in one block. Any of dc0, dlam, dgam may be null.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_expand_factor_bwd(const T* __restrict__ factor, bool per_head, int Hq,
+                                                                int G, const T* __restrict__ dc0,
+                                                                const T* __restrict__ dlam,
+                                                                const T* __restrict__ dgam, T* __restrict__ dfactor) {
+  __shared__ T L[kPackMax];
+  __shared__ T S[kSideMax * kSideMax];
+  const int side = G + 1, P = side * (side + 1) / 2;
+  const int first = per_head ? blockIdx.x : 0, last = per_head ? blockIdx.x + 1 : Hq;
+  for (int x = threadIdx.x; x < P; x += kThreads) L[x] = factor[(per_head ? (size_t)first * P : 0) + x];
+  constexpr int kOwn = (kPackMax + kThreads - 1) / kThreads;  // entries per thread, at most
+  double sum[kOwn] = {};
+  for (int h = first; h < last; ++h) {
+    __syncthreads();
+    for (int x = threadIdx.x; x < side * side; x += kThreads) {
+      const int i = x / side, j = x % side;
+      T s = 0;
+      if (x == 0)
+        s = dc0 ? 2 * dc0[h] : T(0);
+      else if (i == 0 || j == 0)
+        s = dlam ? 2 * dlam[(size_t)h * G + i + j - 1] : T(0);
+      else if (dgam)
+        s = dgam[((size_t)h * G + i - 1) * G + j - 1] + dgam[((size_t)h * G + j - 1) * G + i - 1];
+      S[x] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < kOwn; ++n) {
+      const int x = threadIdx.x + n * kThreads;
+      if (x >= P) break;
+      int i = 0;
+      while (packed(i + 1, 0) <= x) ++i;
+      const int m = x - packed(i, 0);
+      double acc = 0;
+      for (int j = m; j < side; ++j) acc += (double)S[i * side + j] * L[packed(j, m)];
+      sum[n] += acc;
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < kOwn; ++n) {
+    const int x = threadIdx.x + n * kThreads;
+    if (x < P) dfactor[(size_t)first * (per_head ? P : 0) + x] = (T)sum[n];
+  }
+}
+
+// One wave per label row (one row shared by all heads, or one per head): ids in
+// [0, G) forming a prefix. flag |= 1: an id out of range, |= 2: not a prefix.
+template <typename I>
+__global__ __launch_bounds__(64) void k_check_labels(const I* __restrict__ labels, bool per_head, int D, int Hq, int G,
+                                                     int32_t* __restrict__ table, int* flag) {
+  const int row = blockIdx.x, l = threadIdx.x;
+  const I id = l < D ? labels[(size_t)row * D + l] : 0;
+  const bool in = id >= 0 && id < (I)G;
+  uint64_t used = l < D && in && id < 64 ? 1ull << id : 0;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) used |= __shfl_xor(used, off, 64);
+  const bool wild = __any(l < D && !in), far = __any(l < D && in && id >= 64);
+  if (l == 0 && (wild || far || (used & (used + 1)) || !used)) atomicOr_system(flag, wild ? 1 : 2);
+  const int32_t v = l < D && in ? (int32_t)id : 0;
+  if (per_head) {
+    table[(size_t)row * kD + l] = v;
+  } else {
+    for (int h = 0; h < Hq; ++h) table[(size_t)h * kD + l] = v;
+  }
+}
+
+namespace {
+
+__device__ __forceinline__ bool finite(float x) { return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u; }
+__device__ __forceinline__ bool finite(double x) {
+  return ((uint64_t)__double_as_longlong(x) & 0x7ff0000000000000ull) != 0x7ff0000000000000ull;
+}
+struct Bf16 {
+  uint16_t x;
+};
+struct Fp16 {
+  uint16_t x;
+};
+__device__ __forceinline__ bool finite(Bf16 v) { return (v.x & 0x7f80) != 0x7f80; }
+__device__ __forceinline__ bool finite(Fp16 v) { return (v.x & 0x7c00) != 0x7c00; }
+
+// Whether a thread's share of rows x width values (row stride in elements) is
+// finite; 16 bytes at a time where the rows are contiguous and aligned.
+template <typename T>
+__device__ __forceinline__ bool all_finite(const T* __restrict__ p, size_t rows, int width, int stride, size_t t,
+                                           size_t n) {
+  constexpr int V = 16 / sizeof(T);
+  const size_t total = rows * width;
+  bool ok = true;
+  size_t done = 0;
+  if (stride == width && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+    struct alignas(16) Vec {
+      T v[V];
+    };
+    const size_t vecs = total / V;
+#pragma unroll 4
+    for (size_t i = t; i < vecs; i += n) {
+      const Vec x = reinterpret_cast<const Vec*>(p)[i];
+#pragma unroll
+      for (int e = 0; e < V; ++e) ok &= finite(x.v[e]);
+    }
+    done = vecs * V;
+  }
+  for (size_t i = done + t; i < total; i += n) ok &= finite(p[i / width * stride + i % width]);
+  return ok;
+}
+
+}  // namespace
+
+// flag |= 1: num or den not finite, |= 2: den not positive, |= 4: out not
+// finite. num and out may be null.
+template <typename T, typename O>
+__global__ __launch_bounds__(kThreads) void k_check_outputs(const T* __restrict__ num, const T* __restrict__ den,
+                                                            const O* __restrict__ out, size_t rows, int width,
+                                                            int num_stride, int out_stride, int* flag) {
+  const size_t t = (size_t)blockIdx.x * kThreads + threadIdx.x, n = (size_t)gridDim.x * kThreads;
+  int bad = 0;
+  for (size_t i = t; i < rows; i += n) {
+    const T z = den[i];
+    bad |= (finite(z) ? 0 : 1) | (z > 0 ? 0 : 2);
+  }
+  if (num && !all_finite(num, rows, width, num_stride, t, n)) bad |= 1;
+  if (out && !all_finite(out, rows, width, out_stride, t, n)) bad |= 4;
+  const int any = (__any(bad & 1) ? 1 : 0) | (__any(bad & 2) ? 2 : 0) | (__any(bad & 4) ? 4 : 0);
+  if (any && (threadIdx.x & 63) == 0) atomicOr_system(flag, any);
+}
+
+template <typename T>
+void launch_expand_factor(const T* factor, bool per_head, int Hq, int G, double eps, T* c0, T* lam, T* gam,
+                          hipStream_t st) {
+  hipLaunchKernelGGL(k_expand_factor<T>, dim3(Hq), dim3(kThreads), 0, st, factor, per_head, G, (T)eps, c0, lam, gam);
+}
+template <typename T>
+void launch_expand_factor_bwd(const T* factor, bool per_head, int Hq, int G, const T* dc0, const T* dlam,
+                              const T* dgam, T* dfactor, hipStream_t st) {
+  hipLaunchKernelGGL(k_expand_factor_bwd<T>, dim3(per_head ? Hq : 1), dim3(kThreads), 0, st, factor, per_head, Hq, G,
+                     dc0, dlam, dgam, dfactor);
+}
+template void launch_expand_factor<float>(const float*, bool, int, int, double, float*, float*, float*, hipStream_t);
+template void launch_expand_factor<double>(const double*, bool, int, int, double, double*, double*, double*, hipStream_t);
+template void launch_expand_factor_bwd<float>(const float*, bool, int, int, const float*, const float*, const float*,
+                                              float*, hipStream_t);
+template void launch_expand_factor_bwd<double>(const double*, bool, int, int, const double*, const double*,
+                                               const double*, double*, hipStream_t);
+
+void launch_check_labels(const void* labels, bool wide, bool per_head, int D, int Hq, int G, int32_t* table, int* flag,
+                         hipStream_t st) {
+  const dim3 grid(per_head ? Hq : 1), block(64);
+  if (wide)
+    hipLaunchKernelGGL(k_check_labels<int64_t>, grid, block, 0, st, static_cast<const int64_t*>(labels), per_head, D, Hq,
+                       G, table, flag);
+  else
+    hipLaunchKernelGGL(k_check_labels<int32_t>, grid, block, 0, st, static_cast<const int32_t*>(labels), per_head, D, Hq,
+                       G, table, flag);
+}
+
+namespace {
+template <typename T, typename O>
+void check_outputs(const void* num, const void* den, const void* out, size_t rows, int width, int ns, int os, int* flag,
+                   hipStream_t st) {
+  // one pass at memory speed for large outputs, one block for a few rows
+  const size_t work = num || out ? rows * width / 16 : rows / 4;
+  const unsigned blocks = (unsigned)std::min<size_t>(2048, std::max<size_t>(1, (work + kThreads - 1) / kThreads));
+  hipLaunchKernelGGL((k_check_outputs<T, O>), dim3(blocks), dim3(kThreads), 0, st, static_cast<const T*>(num),
+                     static_cast<const T*>(den), static_cast<const O*>(out), rows, width, ns, os, flag);
+}
+}  // namespace
+
+// out_kind: 0 float32, 1 bfloat16, 2 float16, 3 float64.
+int launch_check_outputs(bool wide, int out_kind, const void* num, const void* den, const void* out, size_t rows,
+                         int width, int num_stride, int out_stride, int* flag, hipStream_t st) {
+#define OAL_CHECK(T, O) check_outputs<T, O>(num, den, out, rows, width, num_stride, out_stride, flag, st)
+  switch (out_kind + (wide ? 4 : 0)) {
+    case 0: OAL_CHECK(float, float); break;
+    case 1: OAL_CHECK(float, Bf16); break;
+    case 2: OAL_CHECK(float, Fp16); break;
+    case 3: OAL_CHECK(float, double); break;
+    case 4: OAL_CHECK(double, float); break;
+    case 5: OAL_CHECK(double, Bf16); break;
+    case 6: OAL_CHECK(double, Fp16); break;
+    case 7: OAL_CHECK(double, double); break;
+    default: return 1;
+  }
+#undef OAL_CHECK
+  return 0;
+}
+
+}  // namespace oal

@@ -292,6 +292,18 @@ void launch_den_bwd(const LaunchGeom& g, const uint16_t* QT16, const uint16_t* G
 
 int run_mfma_selftest(int* dev_errors, hipStream_t st);
 
+// Factor expansion, its VJP, and the checks of labels and outputs (oal_adapter.hip).
+template <typename T>
+void launch_expand_factor(const T* factor, bool per_head, int Hq, int G, double eps, T* c0, T* lam, T* gam,
+                          hipStream_t st);
+template <typename T>
+void launch_expand_factor_bwd(const T* factor, bool per_head, int Hq, int G, const T* dc0, const T* dlam,
+                              const T* dgam, T* dfactor, hipStream_t st);
+void launch_check_labels(const void* labels, bool wide, bool per_head, int D, int Hq, int G, int32_t* table, int* flag,
+                         hipStream_t st);
+int launch_check_outputs(bool wide, int out_kind, const void* num, const void* den, const void* out, size_t rows,
+                         int width, int num_stride, int out_stride, int* flag, hipStream_t st);
+
 // FP64 route (oal_f64.hip): pairwise evaluation over 32-token tiles.
 struct F64Geom {
   int B, Hq, Hkv, N;

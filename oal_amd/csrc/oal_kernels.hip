@@ -1362,4 +1362,60 @@ int oal_backward_f64(const double* q, const double* k, const double* v, const in
   return launch_status("oal_backward_f64 launch");
 }
 
+// Adapter entry points: factor expansion and checks (oal_adapter.hip).
+int oal_expand_factor(const void* factor, int wide, int per_head, int q_heads, int groups, double eps, void* c0,
+                      void* lam, void* gam, void* stream) {
+  Range range("oal_expand_factor");
+  if (!factor || !c0 || !lam || !gam) return fail("oal_expand_factor: null pointer argument");
+  if (q_heads <= 0 || groups < 1 || groups > 64) return fail("oal_expand_factor: heads must be positive, groups in [1, 64]");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (wide)
+    oal::launch_expand_factor<double>(static_cast<const double*>(factor), per_head, q_heads, groups, eps,
+                                      static_cast<double*>(c0), static_cast<double*>(lam), static_cast<double*>(gam), st);
+  else
+    oal::launch_expand_factor<float>(static_cast<const float*>(factor), per_head, q_heads, groups, eps,
+                                     static_cast<float*>(c0), static_cast<float*>(lam), static_cast<float*>(gam), st);
+  return launch_status("oal_expand_factor launch");
+}
+
+int oal_expand_factor_backward(const void* factor, int wide, int per_head, int q_heads, int groups, const void* dc0,
+                               const void* dlam, const void* dgam, void* dfactor, void* stream) {
+  Range range("oal_expand_factor_backward");
+  if (!factor || !dfactor) return fail("oal_expand_factor_backward: null pointer argument");
+  if (q_heads <= 0 || groups < 1 || groups > 64)
+    return fail("oal_expand_factor_backward: heads must be positive, groups in [1, 64]");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (wide)
+    oal::launch_expand_factor_bwd<double>(static_cast<const double*>(factor), per_head, q_heads, groups,
+                                          static_cast<const double*>(dc0), static_cast<const double*>(dlam),
+                                          static_cast<const double*>(dgam), static_cast<double*>(dfactor), st);
+  else
+    oal::launch_expand_factor_bwd<float>(static_cast<const float*>(factor), per_head, q_heads, groups,
+                                         static_cast<const float*>(dc0), static_cast<const float*>(dlam),
+                                         static_cast<const float*>(dgam), static_cast<float*>(dfactor), st);
+  return launch_status("oal_expand_factor_backward launch");
+}
+
+int oal_check_labels(const void* labels, int wide, int per_head, int head_dim, int q_heads, int groups, int32_t* table,
+                     int* flag, void* stream) {
+  Range range("oal_check_labels");
+  if (!labels || !table || !flag) return fail("oal_check_labels: null pointer argument");
+  if (q_heads <= 0 || groups < 1 || head_dim < 1 || head_dim > 64)
+    return fail("oal_check_labels: heads and groups must be positive, head_dim in [1, 64]");
+  oal::launch_check_labels(labels, wide, per_head, head_dim, q_heads, groups, table, flag,
+                           static_cast<hipStream_t>(stream));
+  return launch_status("oal_check_labels launch");
+}
+
+int oal_check_outputs(int wide, int out_kind, const void* num, const void* den, const void* out, size_t rows, int width,
+                      int num_stride, int out_stride, int* flag, void* stream) {
+  Range range("oal_check_outputs");
+  if (!den || !flag) return fail("oal_check_outputs: null pointer argument");
+  if ((num || out) && width <= 0) return fail("oal_check_outputs: width must be positive");
+  if (oal::launch_check_outputs(wide, out_kind, num, den, out, rows, width, num_stride, out_stride, flag,
+                                static_cast<hipStream_t>(stream)))
+    return fail("oal_check_outputs: unknown output type");
+  return launch_status("oal_check_outputs launch");
+}
+
 }  // extern "C"

@@ -2,7 +2,7 @@
 
 Mirrors the reference surface ``oal_attention/grouped_quadratic.py:277-397``:
 the same arguments, validation rules and error types, the same factor ->
-(c0, lam, Gam) expansion (kept in torch so autograd reaches the factor), the
+(c0, lam, Gam) expansion (differentiable, so autograd reaches the factor), the
 same return conventions. ``execution="triton"`` and ``"auto"`` run the
 hand-written gfx950 HIP kernels (there is no Triton here). ``"reference"`` -- in
 the original a pure-torch evaluation in the working dtype on any device
@@ -19,6 +19,7 @@ from typing import Literal
 
 import torch
 
+from . import _native
 from .hd_block_gemm_autograd import grouped_oal, grouped_oal_f64
 
 _SUPPORTED_FLOATING_DTYPES = frozenset({torch.float16, torch.bfloat16, torch.float32, torch.float64})
@@ -115,10 +116,12 @@ def _validate_factor(factor: object, *, query_heads: int, q_device: torch.device
     return factor, gmax
 
 
-def _canonicalize_dim_groups(
-    dim_groups: object, *, query_heads: int, head_dimension: int, gmax: int, q_device: torch.device
-) -> torch.Tensor:
-    """grouped_quadratic.py:136-181: ids in [0, Gmax) forming a continuous prefix per head."""
+def _on_device(t: torch.Tensor) -> bool:
+    return t.device.type == "cuda" and torch.version.hip is not None
+
+
+def _validate_dim_groups(dim_groups: object, *, query_heads: int, head_dimension: int, q_device: torch.device):
+    """Type, device and shape rules of grouped_quadratic.py:136-165."""
     if not isinstance(dim_groups, torch.Tensor):
         raise TypeError("dim_groups must be a torch.Tensor")
     if dim_groups.dtype not in {torch.int32, torch.int64}:
@@ -128,23 +131,65 @@ def _canonicalize_dim_groups(
     if dim_groups.ndim == 1:
         if dim_groups.shape[0] != head_dimension:
             raise ValueError("dim_groups last dimension must equal D")
-        heads = dim_groups.unsqueeze(0).expand(query_heads, -1)
     elif dim_groups.ndim == 2:
         if dim_groups.shape[0] != query_heads:
             raise ValueError("dim_groups first dimension must equal query-head count Hq")
         if dim_groups.shape[1] != head_dimension:
             raise ValueError("dim_groups last dimension must equal D")
-        heads = dim_groups
     else:
         raise ValueError("dim_groups must have shape [D] or [Hq, D]")
-    if not bool(((heads >= 0) & (heads < gmax)).all()):
+    return dim_groups
+
+
+def _raise_for_labels(bits: int) -> None:
+    """The errors of the device's label check (_native.Verdict)."""
+    if bits & 1:
         raise ValueError("dim_groups IDs must satisfy 0 <= id < Gmax")
+    if bits & 2:
+        raise ValueError("dim_groups IDs for every query head must form a continuous prefix")
+
+
+def _canonicalize_dim_groups(
+    dim_groups: object, *, query_heads: int, head_dimension: int, gmax: int, q_device: torch.device
+) -> torch.Tensor:
+    """grouped_quadratic.py:136-181: ids in [0, Gmax) forming a continuous prefix per head."""
+    dim_groups = _validate_dim_groups(dim_groups, query_heads=query_heads, head_dimension=head_dimension,
+                                      q_device=q_device)
+    if _on_device(dim_groups) and head_dimension <= _native.HEAD_DIM:
+        verdict = _native.Verdict(dim_groups.device)
+        verdict.check_labels(dim_groups, query_heads, gmax)
+        _raise_for_labels(verdict.read()[0])
+        return dim_groups.to(torch.int32).contiguous()
+    heads = dim_groups if dim_groups.ndim == 2 else dim_groups.unsqueeze(0).expand(query_heads, -1)
+    if not bool(((heads >= 0) & (heads < gmax)).all()):
+        _raise_for_labels(1)
     host = heads.detach().to("cpu", torch.int64)
     for row in host:
         used = torch.unique(row, sorted=True)
         if used.numel() == 0 or not torch.equal(used, torch.arange(used.numel(), dtype=used.dtype)):
-            raise ValueError("dim_groups IDs for every query head must form a continuous prefix")
+            _raise_for_labels(2)
     return dim_groups.to(torch.int32).contiguous()
+
+
+class _FactorExpansion(torch.autograd.Function):
+    """factor [P] or [Hq, P] -> (c0, lam, gam) on the device, one launch each way.
+
+    Not twice differentiable, as the operator that its results go to is not."""
+
+    @staticmethod
+    def forward(ctx, factor, query_heads: int, gmax: int, kernel_eps: float):
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(factor)
+        ctx.sizes = (query_heads, gmax)
+        return _native.expand_factor(factor.detach(), query_heads, gmax, kernel_eps)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dc0, dlam, dgam):
+        if dc0 is None and dlam is None and dgam is None:
+            return None, None, None, None
+        (factor,) = ctx.saved_tensors
+        return _native.expand_factor_backward(factor, *ctx.sizes, dc0, dlam, dgam), None, None, None
 
 
 def _expand_factor_coefficients(
@@ -155,7 +200,12 @@ def _expand_factor_coefficients(
     Same expansion as grouped_quadratic.py:184-218. M is formed as an
     elementwise product-sum, so M[i][j] and M[j][i] are the same floating-point
     sum and Gam is exactly symmetric (the HIP intra-chunk term relies on it).
+    On the device it is one kernel (oal_adapter.hip) for the group counts that
+    the operator takes.
     """
+    if _on_device(factor) and gmax <= 64 and working_dtype in (torch.float32, torch.float64):
+        fac = factor[0] if factor.ndim == 2 and factor.shape[0] == 1 else factor
+        return _FactorExpansion.apply(fac.to(dtype=working_dtype).contiguous(), query_heads, gmax, float(kernel_eps))
     fac = factor.unsqueeze(0) if factor.ndim == 1 else factor
     fac = fac.to(dtype=working_dtype)
     if fac.shape[0] == 1:
@@ -184,6 +234,39 @@ def _validate_public_options(*, causal, execution, output_dtype, return_unnormal
     if not isinstance(return_unnormalized, bool):
         raise TypeError("return_unnormalized must be a bool")
     return causal, execution
+
+
+def _resolve_attention_scale(scale: object, head_dimension: int) -> float:
+    """D^-1/2, or the caller's finite Python scalar."""
+    if scale is None:
+        return head_dimension ** -0.5
+    if isinstance(scale, bool) or not isinstance(scale, (int, float)):
+        raise TypeError("scale must be a finite Python scalar")
+    try:
+        resolved = float(scale)
+    except OverflowError:
+        raise ValueError("scale must be finite") from None
+    if not math.isfinite(resolved):
+        raise ValueError("scale must be finite")
+    return resolved
+
+
+def _validate_execution(q: torch.Tensor, v: torch.Tensor, factor: torch.Tensor, execution: str) -> None:
+    """Device, type and size rules of one execution."""
+    if not _on_device(q):
+        if execution == "reference":
+            raise RuntimeError(
+                "execution='reference' runs the fp32 HIP kernels and requires ROCm device input; oal_amd "
+                "ships no CPU compute path (the pure-torch formula is test infrastructure only)"
+            )
+        raise RuntimeError("grouped quadratic HIP execution requires ROCm device input")
+    if execution != "reference":
+        if q.dtype not in _HIP_INPUT_DTYPES:
+            raise TypeError("grouped quadratic HIP execution supports float16, bfloat16 and float32")
+        if factor.dtype != torch.float32:
+            raise TypeError("grouped quadratic HIP factor must use FP32")
+    if q.shape[-1] > 64 or v.shape[-1] > 64:
+        raise ValueError("grouped quadratic HIP execution supports D<=64")
 
 
 def oal_attention(
@@ -216,70 +299,56 @@ def oal_attention(
     factor, gmax = _validate_factor(factor, query_heads=q.shape[1], q_device=q.device)
     working_dtype = _resolve_working_dtype(q.dtype, factor.dtype)
     resolved_eps = _validate_kernel_eps(kernel_eps, working_dtype=working_dtype)
-    dim_groups = _canonicalize_dim_groups(
-        dim_groups, query_heads=q.shape[1], head_dimension=q.shape[-1], gmax=gmax, q_device=q.device
-    )
-    if scale is None:
-        resolved_scale = q.shape[-1] ** -0.5
-    elif isinstance(scale, bool) or not isinstance(scale, (int, float)):
-        raise TypeError("scale must be a finite Python scalar")
-    else:
-        try:
-            resolved_scale = float(scale)
-        except OverflowError:
-            raise ValueError("scale must be finite") from None
-        if not math.isfinite(resolved_scale):
-            raise ValueError("scale must be finite")
-
-    if q.device.type != "cuda" or torch.version.hip is None:
-        if execution == "reference":
-            raise RuntimeError(
-                "execution='reference' runs the fp32 HIP kernels and requires ROCm device input; oal_amd "
-                "ships no CPU compute path (the pure-torch formula is test infrastructure only)"
-            )
-        raise RuntimeError("grouped quadratic HIP execution requires ROCm device input")
-    if execution == "reference":
-        # the reference evaluates in the working dtype (:332-355): the fp32 HIP
-        # kernels for FP32, the FP64 route (oal_f64.hip) for FP64
-        if q.shape[-1] > 64 or v.shape[-1] > 64:
-            raise ValueError("grouped quadratic HIP execution supports D<=64")
-        q_work, k_work, v_work = (t.to(dtype=working_dtype) for t in (q, k, v))
-        constant, linear, quadratic = _expand_factor_coefficients(
-            factor, query_heads=q.shape[1], gmax=gmax, kernel_eps=resolved_eps, working_dtype=working_dtype
+    if not (_on_device(q) and q.shape[-1] <= _native.HEAD_DIM):
+        # refused below, after the labels' own errors
+        _canonicalize_dim_groups(
+            dim_groups, query_heads=q.shape[1], head_dimension=q.shape[-1], gmax=gmax, q_device=q.device
         )
-        if working_dtype == torch.float64:
-            output, numerator, denominator = grouped_oal_f64(
-                q_work, k_work, v_work, dim_groups, constant, linear, quadratic, scale=resolved_scale
-            )
+        _resolve_attention_scale(scale, q.shape[-1])
+        _validate_execution(q, v, factor, execution)
+        raise AssertionError("unreachable: the execution check refuses this call")
+    _validate_dim_groups(dim_groups, query_heads=q.shape[1], head_dimension=q.shape[-1], q_device=q.device)
+    # The labels' and the outputs' checks run on the device beside the operator
+    # and report at the end, in the order in which the reference makes them: one
+    # synchronization. (The kernels clamp labels, so bad ones are safe to run.)
+    verdict = _native.Verdict(q.device)
+    try:
+        groups = verdict.check_labels(dim_groups, q.shape[1], gmax)
+        resolved_scale = _resolve_attention_scale(scale, q.shape[-1])
+        _validate_execution(q, v, factor, execution)
+        reference = execution == "reference"
+        coefficients = _expand_factor_coefficients(
+            factor, query_heads=q.shape[1], gmax=gmax, kernel_eps=resolved_eps,
+            working_dtype=working_dtype if reference else torch.float32,
+        )
+        if reference:
+            # the reference evaluates in the working dtype (:332-355): the fp32 HIP
+            # kernels for FP32, the FP64 route (oal_f64.hip) for FP64
+            q, k, v_work = (t.to(dtype=working_dtype) for t in (q, k, v))
+        else:
+            v_work = v
+        if reference and working_dtype == torch.float64:
+            output, numerator, denominator = grouped_oal_f64(q, k, v_work, groups, *coefficients, scale=resolved_scale)
         else:
             output, numerator, denominator = grouped_oal(
-                q_work, k_work, v_work, dim_groups, constant, linear, quadratic, scale=resolved_scale, floor=0.0,
-                precision="fp32",
+                q, k, v_work, groups, *coefficients, scale=resolved_scale, floor=0.0, precision="fp32"
             )
-    else:
-        if q.dtype not in _HIP_INPUT_DTYPES:
-            raise TypeError("grouped quadratic HIP execution supports float16, bfloat16 and float32")
-        if factor.dtype != torch.float32:
-            raise TypeError("grouped quadratic HIP factor must use FP32")
-        if q.shape[-1] > 64 or v.shape[-1] > 64:
-            raise ValueError("grouped quadratic HIP execution supports D<=64")
-        constant, linear, quadratic = _expand_factor_coefficients(
-            factor, query_heads=q.shape[1], gmax=gmax, kernel_eps=resolved_eps, working_dtype=torch.float32
-        )
-        output, numerator, denominator = grouped_oal(
-            q, k, v, dim_groups, constant, linear, quadratic, scale=resolved_scale, floor=0.0
-        )
-
-    if not (bool(torch.isfinite(numerator).all()) and bool(torch.isfinite(denominator).all())):
+        target = v.dtype if output_dtype is None else output_dtype
+        if torch.finfo(target).bits > torch.finfo(output.dtype).bits:
+            # a wider output than the kernel's storage dtype: normalize the fp32 num/den
+            output = numerator / denominator
+        output = output.to(dtype=target)
+        verdict.check_outputs(numerator, denominator, output)
+    except Exception:
+        _raise_for_labels(verdict.read()[0])
+        raise
+    labels, outputs = verdict.read()
+    _raise_for_labels(labels)
+    if outputs & 1:
         raise RuntimeError("Grouped Quadratic result must be finite")
-    if not bool((denominator > 0).all()):
+    if outputs & 2:
         raise RuntimeError("Grouped Quadratic denominator must be finite and strictly positive")
-    target = v.dtype if output_dtype is None else output_dtype
-    if torch.finfo(target).bits > torch.finfo(output.dtype).bits:
-        # a wider output than the kernel's storage dtype: normalize the fp32 num/den
-        output = numerator / denominator
-    output = output.to(dtype=target)
-    if not bool(torch.isfinite(output).all()):
+    if outputs & 4:
         raise RuntimeError("Grouped Quadratic normalized output must be finite")
     if return_unnormalized:
         return output, numerator, denominator

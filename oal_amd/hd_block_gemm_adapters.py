@@ -2,8 +2,8 @@
 
 Same surface as ``oal_attention/hd_block_gemm_adapters.py:120-415``:
 ``prepare_grouped_hd_block_gemm`` freezes geometry, groups and plan once;
-``run_prepared_grouped_hd_block_gemm`` expands the live factor per call (in
-torch, so autograd reaches the factor) and runs the HIP operator;
+``run_prepared_grouped_hd_block_gemm`` expands the live factor per call
+(differentiably, so autograd reaches the factor) and runs the HIP operator;
 ``grouped_causal_attention`` does both. Callers (e.g. the reference's
 ``qwen_lora_experiment/attention/hd_runtime.py:200-224``) can resolve these
 names unchanged.

@@ -1,0 +1,121 @@
+"""Factor expansion and the device checks around the operator (oal_adapter.hip).
+
+The expansion and its VJP against the torch formula in float64 (a sum of at
+most 65 products: 65 x 6e-8 = 4e-6 in float32, 8e-15 in float64); the label check
+against the host's rule on every kind of bad label; the output check on a bad
+value at either end of each operand, in whole and in sliced outputs of every type.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch.device("cuda:0")
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 4e-6), (torch.float64, 8e-15)])
+@pytest.mark.parametrize("groups,shared", [(1, False), (8, False), (8, True), (22, False), (64, False), (64, True)])
+def test_factor_expansion_and_its_vjp(dtype, tol, groups, shared):
+    from oal_amd import grouped_quadratic as gq
+
+    dev, hq, side = _dev(), 3, groups + 1
+    gen = torch.Generator().manual_seed(groups)
+    shape = (side * (side + 1) // 2,) if shared else (hq, side * (side + 1) // 2)
+    host = torch.randn(shape, generator=gen, dtype=torch.float64).to(dtype)
+    factor = host.to(dev).requires_grad_()
+    got = gq._expand_factor_coefficients(factor, query_heads=hq, gmax=groups, kernel_eps=1e-3, working_dtype=dtype)
+    ref = host.double().requires_grad_()
+    want = gq._expand_factor_coefficients(ref, query_heads=hq, gmax=groups, kernel_eps=1e-3, working_dtype=torch.float64)
+    assert torch.equal(got[2], got[2].transpose(-1, -2))
+    # positive: a shared factor's gradient of c0 alone is a sum over the heads, and the
+    # bound holds relative to the terms' size (of random signs it cancelled to 2e-3 of
+    # them once, at an error of 6e-8 of them)
+    up = [0.5 + torch.rand(t.shape, generator=gen, dtype=torch.float64) for t in want]
+    for name, a, r in zip(("c0", "lam", "gam"), got, want):
+        assert a.dtype == dtype
+        assert float((a.detach().cpu().double() - r.detach()).norm() / r.detach().norm()) <= tol, name
+    for used in ((0, 1, 2), (0,), (1,), (2,)):
+        da = torch.autograd.grad([got[i] for i in used], factor, [up[i].to(dev, dtype) for i in used], retain_graph=True)
+        dr = torch.autograd.grad([want[i] for i in used], ref, [up[i].to(dtype).double() for i in used], retain_graph=True)
+        assert float((da[0].cpu().double() - dr[0]).norm() / dr[0].norm()) <= tol, used
+
+
+def _prefix(row, groups):
+    used = sorted(set(row))
+    return 1 if any(x < 0 or x >= groups for x in row) else 0 if used == list(range(len(used))) else 2
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_label_check(dtype):
+    from oal_amd import _native
+
+    dev = _dev()
+    rows = [[0], [1], [0, 1, 2], [0, 2], [2, 2, 2], [-1, 0], [0, 5], [63 - i for i in range(64)], [0] * 63 + [2],
+            list(range(63)) + [64], [0, 1 << 30], [3, 2, 1, 0]]
+    for row in rows:
+        for groups in (1, 3, 5, 64, 100):
+            labels = torch.tensor(row, dtype=dtype, device=dev)
+            for given, hq in ((labels, 2), (torch.stack([labels, torch.zeros_like(labels)]), 2)):
+                verdict = _native.Verdict(dev)
+                table = verdict.check_labels(given, hq, groups)
+                bits = verdict.read()[0]
+                assert bits == _prefix(row, groups), (row, groups, bits)
+                if bits == 0:
+                    assert table.shape == (hq, 64) and table[0].tolist() == row + [0] * (64 - len(row))
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("shape,width", [((1, 1, 1), 1), ((2, 3, 5), 64), ((2, 3, 5), 17), ((1, 7, 301), 48)])
+def test_output_check(out_dtype, wide, shape, width):
+    from oal_amd import _native
+
+    dev, dtype = _dev(), torch.float64 if wide else torch.float32
+    num = torch.ones((*shape, 64), dtype=dtype, device=dev)[..., :width]
+    out = torch.ones((*shape, 64), dtype=out_dtype, device=dev)[..., :width]
+    den = torch.ones((*shape, 1), dtype=dtype, device=dev)
+
+    def bits(n=num, d=den, o=out):
+        verdict = _native.Verdict(dev)
+        verdict.check_outputs(n, d, o)
+        return verdict.read()[1]
+
+    assert bits() == 0 and bits(n=num.contiguous(), o=out.contiguous()) == 0 and bits(n=None, o=None) == 0
+    for at in (0, -1):
+        for value in (float("inf"), float("nan")):
+            for sliced in (True, False):
+                bad = num.clone() if not sliced else num.new_ones((*shape, 64))[..., :width]
+                bad[at, at, at, at] = value
+                assert bits(n=bad) == 1
+                bad = out.clone() if not sliced else out.new_ones((*shape, 64))[..., :width]
+                bad[at, at, at, at] = -value
+                assert bits(o=bad) == 4
+        for value, want in ((0.0, 2), (-1.0, 2), (float("nan"), 3), (float("inf"), 1), (float("-inf"), 3)):
+            bad = den.clone()
+            bad[at, at, at] = value
+            assert bits(d=bad) == want
+
+
+def test_errors_come_in_the_reference_order():
+    """Bad labels are reported before a bad scale or a size that the kernels refuse."""
+    from oal_amd import oal_attention
+
+    dev = _dev()
+    q, k, v = (torch.randn(1, 2, 5, 4, device=dev) for _ in range(3))
+    factor = torch.eye(3, device=dev)[tuple(torch.tril_indices(3, 3))]
+    good, bad = torch.tensor([0, 1, 1, 0], device=dev), torch.tensor([1, 1, 1, 1], device=dev)
+    with pytest.raises(ValueError, match="continuous prefix"):
+        oal_attention(q, k, v, bad, factor, scale=float("nan"))
+    with pytest.raises(ValueError, match="continuous prefix"):
+        oal_attention(q, k, torch.randn(1, 2, 5, 70, device=dev), bad, factor)
+    with pytest.raises(ValueError, match="scale must be finite"):
+        oal_attention(q, k, v, good, factor, scale=float("nan"))
+    with pytest.raises(ValueError, match="0 <= id < Gmax"):
+        oal_attention(q, k, v, good + 2, factor)
+    with pytest.raises(RuntimeError, match="result must be finite"):
+        oal_attention(q * float("inf"), k, v, good, factor)
