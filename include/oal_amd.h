@@ -222,6 +222,17 @@ int oal_expand_factor_backward(const void* factor, int wide, int per_head, int q
                                const void* dc0, const void* dlam, const void* dgam, void* dfactor, void* stream);
 
 /*
+ * oal_expand_pairs: per-dimension b [Hq][D] and per-pair c [Hq][D (D + 1) / 2]
+ * (pair (r, c), r >= c, at r (r + 1) / 2 + c) -> one group per dimension: lam
+ * [Hq][64], the symmetric gam [Hq][64][64] and labels [Hq][64] = d, zero past D.
+ * oal_expand_pairs_backward: dgam [Hq][64][64] -> dc, an off-diagonal pair
+ * taking both of its entries. All float32.
+ */
+int oal_expand_pairs(const float* b, const float* c, int q_heads, int head_dim, float* lam, float* gam,
+                     int32_t* labels, void* stream);
+int oal_expand_pairs_backward(const float* dgam, int q_heads, int head_dim, float* dc, void* stream);
+
+/*
  * Checks that report into *flag, an int that the device can write and the
  * caller zeroed (host-mapped memory serves): bits are only ever set, so the
  * caller reads them once after synchronizing the stream.

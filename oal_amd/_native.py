@@ -72,6 +72,8 @@ _SIGNATURES = {
     ),
     "oal_expand_factor": ([_vp, _i, _i, _i, _i, ctypes.c_double, _vp, _vp, _vp, _vp], _i),
     "oal_expand_factor_backward": ([_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp], _i),
+    "oal_expand_pairs": ([_vp, _vp, _i, _i, _vp, _vp, _vp, _vp], _i),
+    "oal_expand_pairs_backward": ([_vp, _i, _i, _vp, _vp], _i),
     "oal_check_labels": ([_vp, _i, _i, _i, _i, _i, _vp, _vp, _vp], _i),
     "oal_check_outputs": ([_i, _i, _vp, _vp, _vp, _sz, _i, _i, _i, _vp, _vp], _i),
 }
@@ -528,6 +530,35 @@ def expand_factor_backward(factor: torch.Tensor, query_heads: int, groups: int, 
                                             _stream(factor.device))
         _check(rc, lib, "oal_expand_factor_backward")
     return dfactor
+
+
+def expand_pairs(b: torch.Tensor, c: torch.Tensor):
+    """(lam [Hq, 64], gam [Hq, 64, 64], labels [Hq, 64]) of contiguous float32
+    b [Hq, D] and c [Hq, D(D+1)/2]: one group per dimension, zero past D."""
+    lib = load_library()
+    _require_device(b, c)
+    hq, d = b.shape
+    _check_tensor(b, "b", dtype=torch.float32, shape=(hq, d))
+    _check_tensor(c, "c", dtype=torch.float32, shape=(hq, d * (d + 1) // 2), device=b.device)
+    with torch.cuda.device(b.device):
+        lam, gam = b.new_empty((hq, HEAD_DIM)), b.new_empty((hq, HEAD_DIM, HEAD_DIM))
+        labels = torch.empty((hq, HEAD_DIM), dtype=torch.int32, device=b.device)
+        rc = lib.oal_expand_pairs(_ptr(b), _ptr(c), hq, d, _ptr(lam), _ptr(gam), _ptr(labels), _stream(b.device))
+        _check(rc, lib, "oal_expand_pairs")
+    return lam, gam, labels
+
+
+def expand_pairs_backward(dgam: torch.Tensor, head_dim: int) -> torch.Tensor:
+    """dc [Hq, D(D+1)/2] of the contiguous float32 gradient of :func:`expand_pairs`'s gam."""
+    lib = load_library()
+    _require_device(dgam)
+    hq = dgam.shape[0]
+    _check_tensor(dgam, "dgam", dtype=torch.float32, shape=(hq, HEAD_DIM, HEAD_DIM))
+    with torch.cuda.device(dgam.device):
+        dc = dgam.new_empty((hq, head_dim * (head_dim + 1) // 2))
+        rc = lib.oal_expand_pairs_backward(_ptr(dgam), hq, head_dim, _ptr(dc), _stream(dgam.device))
+        _check(rc, lib, "oal_expand_pairs_backward")
+    return dc
 
 
 class Verdict:

@@ -5,12 +5,17 @@
 //                        lam = 2 M_0,1.., gam = M_1..,1.. with M = L L^T
 //                        (reference grouped_quadratic.py:184-218)
 //   k_expand_factor_bwd  its VJP, dL = (dM + dM^T) L on the lower triangle
+//   k_expand_pairs       per-pair coefficients c [Hq][D (D + 1) / 2] -> the symmetric
+//                        gam [Hq][64][64], b -> lam, and the labels d -> d
+//   k_expand_pairs_bwd   dgam -> dc (an off-diagonal pair has two entries)
 //   k_check_labels       group labels -> int32 [Hq][64], and whether they are valid
 //                        (reference grouped_quadratic.py:136-181)
 //   k_check_outputs      whether num, den and out are finite and den positive
 //                        (reference grouped_quadratic.py:379-397,
 //                        hd_block_gemm_runtime.py:392-408)
 //
+// The pair kernels took 12 launches as torch operations (index gathers and
+// scatters, 50 us of kernels beside 330 us for the operator at N = 1024).
 // All are bound by their launch: a few hundred values, or one pass over the
 // outputs. As torch operations the expansion took 14 launches and its VJP about 20,
 // the checks 3 to 14 launches with 2 to 5 host synchronizations, 190 us of host
@@ -107,6 +112,31 @@ __global__ __launch_bounds__(kThreads) void k_expand_factor_bwd(const T* __restr
   for (int n = 0; n < kOwn; ++n) {
     const int x = threadIdx.x + n * kThreads;
     if (x < P) dfactor[(size_t)first * (per_head ? P : 0) + x] = (T)sum[n];
+  }
+}
+
+// One block per query head; dimensions past D are zero.
+__global__ __launch_bounds__(kThreads) void k_expand_pairs(const float* __restrict__ b, const float* __restrict__ c,
+                                                           int D, float* __restrict__ lam, float* __restrict__ gam,
+                                                           int32_t* __restrict__ labels) {
+  const int h = blockIdx.x, P = D * (D + 1) / 2;
+  for (int x = threadIdx.x; x < kD * kD; x += kThreads) {
+    const int i = x / kD, j = x % kD, hi = i > j ? i : j, lo = i > j ? j : i;
+    gam[(size_t)h * kD * kD + x] = hi < D ? c[(size_t)h * P + packed(hi, lo)] : 0.f;
+  }
+  if (threadIdx.x < kD) {
+    const int d = threadIdx.x;
+    lam[h * kD + d] = d < D ? b[h * D + d] : 0.f;
+    labels[h * kD + d] = d;
+  }
+}
+__global__ __launch_bounds__(kThreads) void k_expand_pairs_bwd(const float* __restrict__ dgam, int D,
+                                                               float* __restrict__ dc) {
+  const int h = blockIdx.x, P = D * (D + 1) / 2;
+  const float* g = dgam + (size_t)h * kD * kD;
+  for (int x = threadIdx.x; x < kD * kD; x += kThreads) {
+    const int i = x / kD, j = x % kD;
+    if (i < D && j <= i) dc[(size_t)h * P + packed(i, j)] = i == j ? g[x] : g[x] + g[j * kD + i];
   }
 }
 
@@ -209,6 +239,14 @@ template void launch_expand_factor_bwd<float>(const float*, bool, int, int, cons
                                               float*, hipStream_t);
 template void launch_expand_factor_bwd<double>(const double*, bool, int, int, const double*, const double*,
                                                const double*, double*, hipStream_t);
+
+void launch_expand_pairs(const float* b, const float* c, int Hq, int D, float* lam, float* gam, int32_t* labels,
+                         hipStream_t st) {
+  hipLaunchKernelGGL(k_expand_pairs, dim3(Hq), dim3(kThreads), 0, st, b, c, D, lam, gam, labels);
+}
+void launch_expand_pairs_bwd(const float* dgam, int Hq, int D, float* dc, hipStream_t st) {
+  hipLaunchKernelGGL(k_expand_pairs_bwd, dim3(Hq), dim3(kThreads), 0, st, dgam, D, dc);
+}
 
 void launch_check_labels(const void* labels, bool wide, bool per_head, int D, int Hq, int G, int32_t* table, int* flag,
                          hipStream_t st) {

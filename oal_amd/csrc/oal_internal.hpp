@@ -299,6 +299,9 @@ void launch_expand_factor(const T* factor, bool per_head, int Hq, int G, double 
 template <typename T>
 void launch_expand_factor_bwd(const T* factor, bool per_head, int Hq, int G, const T* dc0, const T* dlam,
                               const T* dgam, T* dfactor, hipStream_t st);
+void launch_expand_pairs(const float* b, const float* c, int Hq, int D, float* lam, float* gam, int32_t* labels,
+                         hipStream_t st);
+void launch_expand_pairs_bwd(const float* dgam, int Hq, int D, float* dc, hipStream_t st);
 void launch_check_labels(const void* labels, bool wide, bool per_head, int D, int Hq, int G, int32_t* table, int* flag,
                          hipStream_t st);
 int launch_check_outputs(bool wide, int out_kind, const void* num, const void* den, const void* out, size_t rows,

@@ -1396,6 +1396,25 @@ int oal_expand_factor_backward(const void* factor, int wide, int per_head, int q
   return launch_status("oal_expand_factor_backward launch");
 }
 
+int oal_expand_pairs(const float* b, const float* c, int q_heads, int head_dim, float* lam, float* gam, int32_t* labels,
+                     void* stream) {
+  Range range("oal_expand_pairs");
+  if (!b || !c || !lam || !gam || !labels) return fail("oal_expand_pairs: null pointer argument");
+  if (q_heads <= 0 || head_dim < 1 || head_dim > 64)
+    return fail("oal_expand_pairs: heads must be positive, head_dim in [1, 64]");
+  oal::launch_expand_pairs(b, c, q_heads, head_dim, lam, gam, labels, static_cast<hipStream_t>(stream));
+  return launch_status("oal_expand_pairs launch");
+}
+
+int oal_expand_pairs_backward(const float* dgam, int q_heads, int head_dim, float* dc, void* stream) {
+  Range range("oal_expand_pairs_backward");
+  if (!dgam || !dc) return fail("oal_expand_pairs_backward: null pointer argument");
+  if (q_heads <= 0 || head_dim < 1 || head_dim > 64)
+    return fail("oal_expand_pairs_backward: heads must be positive, head_dim in [1, 64]");
+  oal::launch_expand_pairs_bwd(dgam, q_heads, head_dim, dc, static_cast<hipStream_t>(stream));
+  return launch_status("oal_expand_pairs_backward launch");
+}
+
 int oal_check_labels(const void* labels, int wide, int per_head, int head_dim, int q_heads, int groups, int32_t* table,
                      int* flag, void* stream) {
   Range range("oal_check_labels");

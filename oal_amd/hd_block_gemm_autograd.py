@@ -193,27 +193,17 @@ def grouped_oal_f64(q, k, v, labels, c0, lam, gam, *, scale: float):
     return out, num, den
 
 
-def _pair_rows_cols(d: int, device) -> tuple[torch.Tensor, torch.Tensor]:
-    rows, cols = torch.tril_indices(d, d, device=device)
-    return rows, cols
-
-
 def logical_to_grouped(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, head_dim: int):
     """Logical (a [Hq], b [Hq, D], c [Hq, D(D+1)/2]) -> one group per dimension.
 
     labels = d, lam = b, Gam[r][c] = Gam[c][r] = c_p(r, c) (D padded to 64).
     """
-    hq = a.shape[0]
-    dev = a.device
-    rows, cols = _pair_rows_cols(head_dim, dev)
-    gam = torch.zeros((hq, HEAD_DIM, HEAD_DIM), dtype=torch.float32, device=dev)
-    cf = c.to(torch.float32)
-    gam[:, rows, cols] = cf
-    gam[:, cols, rows] = cf
-    lam = torch.zeros((hq, HEAD_DIM), dtype=torch.float32, device=dev)
-    lam[:, :head_dim] = b.to(torch.float32)
-    labels = torch.arange(HEAD_DIM, dtype=torch.int32, device=dev).unsqueeze(0).expand(hq, -1).contiguous()
-    return a.to(torch.float32).contiguous(), lam.contiguous(), gam.contiguous(), labels
+    if head_dim > HEAD_DIM:
+        raise ValueError(f"the HIP kernels support head and value dimensions up to {HEAD_DIM}")
+    hq, pairs = a.shape[0], head_dim * (head_dim + 1) // 2
+    b, c = (t.to(device=a.device, dtype=torch.float32).expand(hq, n).contiguous() for t, n in ((b, head_dim), (c, pairs)))
+    lam, gam, labels = _native.expand_pairs(b, c)
+    return a.to(torch.float32).contiguous(), lam, gam, labels
 
 
 class _HDParallelBlockGemmFunction(torch.autograd.Function):
@@ -262,16 +252,13 @@ class _HDParallelBlockGemmFunction(torch.autograd.Function):
             scale=scale, floor=eps, need_q=need_q, need_k=need_k, need_v=need_v,
             need_coef=need_a or need_b or need_c, precision=precision,
         )
-        rows, cols = _pair_rows_cols(d, qp.device)
         grads = [
             dq[..., :d] if need_q else None,
             dk[..., :d] if need_k else None,
             dvv[..., :dv] if need_v else None,
             dc0 if need_a else None,
             dlam[:, :d] if need_b else None,
-            torch.where(rows == cols, dgam[:, rows, cols], dgam[:, rows, cols] + dgam[:, cols, rows])
-            if need_c
-            else None,
+            _native.expand_pairs_backward(dgam, d) if need_c else None,
         ]
         out = [g.to(dt) if g is not None else None for g, dt in zip(grads, ctx.input_dtypes)]
         return (*out, None, None, None, None)

@@ -45,6 +45,30 @@ def test_factor_expansion_and_its_vjp(dtype, tol, groups, shared):
         assert float((da[0].cpu().double() - dr[0]).norm() / dr[0].norm()) <= tol, used
 
 
+@pytest.mark.parametrize("d", [1, 5, 48, 64])
+def test_pair_expansion_and_its_vjp(d):
+    """Copies and sums of two values: the same bits as the indexed assignment."""
+    from oal_amd import _native
+    from oal_amd.hd_block_gemm_autograd import logical_to_grouped
+
+    dev, hq = _dev(), 3
+    gen = torch.Generator().manual_seed(d)
+    a, b, c = (torch.randn(s, generator=gen) for s in ((hq,), (hq, d), (hq, d * (d + 1) // 2)))
+    c0, lam, gam, labels = logical_to_grouped(a.to(dev), b.to(dev), c.to(dev), d)
+    rows, cols = torch.tril_indices(d, d)
+    want = torch.zeros(hq, 64, 64)
+    want[:, rows, cols] = c
+    want[:, cols, rows] = c
+    assert torch.equal(c0.cpu(), a) and torch.equal(gam.cpu(), want)
+    assert torch.equal(lam.cpu(), torch.nn.functional.pad(b, (0, 64 - d)))
+    assert torch.equal(labels.cpu(), torch.arange(64, dtype=torch.int32).expand(hq, -1))
+    dgam = torch.randn((hq, 64, 64), generator=gen)
+    dc = torch.where(rows == cols, dgam[:, rows, cols], dgam[:, rows, cols] + dgam[:, cols, rows])
+    assert torch.equal(_native.expand_pairs_backward(dgam.to(dev), d).cpu(), dc)
+    shared = logical_to_grouped(a.to(dev), b[0].to(dev), c[:1].to(dev), d)
+    assert torch.equal(shared[1][2].cpu()[:d], b[0]) and torch.equal(shared[2][2].cpu(), want[0])
+
+
 def _prefix(row, groups):
     used = sorted(set(row))
     return 1 if any(x < 0 or x >= groups for x in row) else 0 if used == list(range(len(used))) else 2
