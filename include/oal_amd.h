@@ -233,6 +233,17 @@ int oal_expand_pairs(const float* b, const float* c, int q_heads, int head_dim, 
 int oal_expand_pairs_backward(const float* dgam, int q_heads, int head_dim, float* dc, void* stream);
 
 /*
+ * Projections proj [B][N][heads][64] of q, k and v to the operator's head-first
+ * layout head [B][heads][N][64], q and k rotated by the rotate-half rotary
+ * embedding of cosine and sine [N][64]; with back, the transpose: gradients of
+ * head to gradients of proj. A NULL proj or head skips that tensor. All dtype
+ * (OAL_DTYPE_F32 or OAL_DTYPE_BF16), 16-byte aligned.
+ */
+int oal_rotary_heads(void* proj_q, void* proj_k, void* proj_v, void* head_q, void* head_k, void* head_v,
+                     const void* cosine, const void* sine, int back, int batch, int q_heads, int kv_heads,
+                     int seq_len, int dtype, void* stream);
+
+/*
  * Checks that report into *flag, an int that the device can write and the
  * caller zeroed (host-mapped memory serves): bits are only ever set, so the
  * caller reads them once after synchronizing the stream.

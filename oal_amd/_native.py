@@ -74,6 +74,7 @@ _SIGNATURES = {
     "oal_expand_factor_backward": ([_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp], _i),
     "oal_expand_pairs": ([_vp, _vp, _i, _i, _vp, _vp, _vp, _vp], _i),
     "oal_expand_pairs_backward": ([_vp, _i, _i, _vp, _vp], _i),
+    "oal_rotary_heads": ([_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp], _i),
     "oal_check_labels": ([_vp, _i, _i, _i, _i, _i, _vp, _vp, _vp], _i),
     "oal_check_outputs": ([_i, _i, _vp, _vp, _vp, _sz, _i, _i, _i, _vp, _vp], _i),
 }
@@ -559,6 +560,36 @@ def expand_pairs_backward(dgam: torch.Tensor, head_dim: int) -> torch.Tensor:
         rc = lib.oal_expand_pairs_backward(_ptr(dgam), hq, head_dim, _ptr(dc), _stream(dgam.device))
         _check(rc, lib, "oal_expand_pairs_backward")
     return dc
+
+
+def rotary_heads(tensors, cos: torch.Tensor, sin: torch.Tensor, q_heads: int, kv_heads: int, *, back: bool):
+    """q, k, v projections [B, N, heads * 64] -> head-first [B, heads, N, 64], q
+    and k rotated by cos, sin [N, 64]; or, with ``back``, head-first gradients ->
+    projection gradients. A tensor given as None comes back as None."""
+    lib = load_library()
+    given = next(t for t in tensors if t is not None)
+    _require_device(given)
+    code, dev = _dtype_code(given.dtype), given.device
+    b, n = given.shape[0], cos.shape[0]
+    _check_tensor(cos, "cos", dtype=given.dtype, shape=(n, HEAD_DIM), device=dev)
+    _check_tensor(sin, "sin", dtype=given.dtype, shape=(n, HEAD_DIM), device=dev)
+    cos, sin = _aligned(cos), _aligned(sin)
+    source, result = [], []
+    with torch.cuda.device(dev):
+        for name, t, heads in zip("qkv", tensors, (q_heads, kv_heads, kv_heads)):
+            if t is None:
+                source.append(None)
+                result.append(None)
+                continue
+            flat, split = (b, n, heads * HEAD_DIM), (b, heads, n, HEAD_DIM)
+            _check_tensor(t, name, dtype=given.dtype, shape=split if back else flat, device=dev)
+            source.append(_aligned(t))
+            result.append(t.new_empty(flat if back else split))
+        proj, head = (result, source) if back else (source, result)
+        rc = lib.oal_rotary_heads(*map(_ptr, proj), *map(_ptr, head), _ptr(cos), _ptr(sin), int(back), b, q_heads,
+                                  kv_heads, n, code, _stream(dev))
+        _check(rc, lib, "oal_rotary_heads")
+    return tuple(result)
 
 
 class Verdict:

@@ -14,7 +14,14 @@
 //                        (reference grouped_quadratic.py:379-397,
 //                        hd_block_gemm_runtime.py:392-408)
 //
-// The pair kernels took 12 launches as torch operations (index gathers and
+//   k_rotary_heads       projections [B][N][heads 64] of q, k, v -> head-first [B][heads]
+//                        [N][64], q and k rotated (rotate-half rotary embedding,
+//                        reference qwen_lora_experiment/attention/common.py:510-596);
+//                        and back, for the gradients
+//
+// The rotation and the three transposes took 13 launches forward and 16 backward,
+// several passes over q each; in one pass it is bound by memory at large sizes and by
+// its launch below. The pair kernels took 12 launches as torch operations (index gathers and
 // scatters, 50 us of kernels beside 330 us for the operator at N = 1024).
 // All are bound by their launch: a few hundred values, or one pass over the
 // outputs. As torch operations the expansion took 14 launches and its VJP about 20,
@@ -222,6 +229,79 @@ __global__ __launch_bounds__(kThreads) void k_check_outputs(const T* __restrict_
   if (any && (threadIdx.x & 63) == 0) atomicOr_system(flag, any);
 }
 
+namespace {
+
+// 8 consecutive values as floats.
+__device__ __forceinline__ void load8(float (&x)[8], const float* p) {
+  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+  x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+}
+__device__ __forceinline__ void load8(float (&x)[8], const uint16_t* p) {
+  const uint4 a = *reinterpret_cast<const uint4*>(p);
+  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    x[2 * e] = __uint_as_float(w[e] << 16);
+    x[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
+  }
+}
+__device__ __forceinline__ void store8(float* p, const float (&x)[8]) {
+  reinterpret_cast<float4*>(p)[0] = make_float4(x[0], x[1], x[2], x[3]);
+  reinterpret_cast<float4*>(p)[1] = make_float4(x[4], x[5], x[6], x[7]);
+}
+__device__ __forceinline__ void store8(uint16_t* p, const float (&x)[8]) {
+  uint32_t w[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = from_f<uint16_t>(x[2 * e]) | (uint32_t)from_f<uint16_t>(x[2 * e + 1]) << 16;
+  *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+}  // namespace
+
+// One thread: 8 dimensions d .. of a head's lower half and their partners d + 32.
+// back: head-first gradients -> projection gradients (the transposed rotation).
+// Null tensors are skipped. Arithmetic in fp32, one rounding to T.
+template <typename T, bool BACK>
+__global__ __launch_bounds__(kThreads) void k_rotary_heads(T* __restrict__ pq, T* __restrict__ pk, T* __restrict__ pv,
+                                                           T* __restrict__ hq, T* __restrict__ hk, T* __restrict__ hv,
+                                                           const T* __restrict__ cosine, const T* __restrict__ sine,
+                                                           int B, int N, int Hq, int Hkv) {
+  constexpr int kHalf = kD / 2, kOct = kHalf / 8;
+  const size_t x = (size_t)blockIdx.x * kThreads + threadIdx.x;
+  const int heads = Hq + 2 * Hkv;
+  if (x >= (size_t)B * N * heads * kOct) return;
+  const int d = 8 * (int)(x % kOct);
+  const int hh = (int)(x / kOct % heads);
+  const size_t row = x / kOct / heads;  // b N + n
+  const int n = (int)(row % N);
+  const size_t b = row / N;
+  const bool is_q = hh < Hq, is_v = hh >= Hq + Hkv;
+  T* const proj = is_q ? pq : is_v ? pv : pk;
+  T* const head = is_q ? hq : is_v ? hv : hk;
+  if (!proj || !head) return;
+  const int H = is_q ? Hq : Hkv, h = is_q ? hh : is_v ? hh - Hq - Hkv : hh - Hq;
+  T* const p = proj + (row * H + h) * kD + d;
+  T* const y = head + ((b * H + h) * N + n) * kD + d;
+  float lo[8], hi[8];
+  load8(lo, BACK ? y : p);
+  load8(hi, (BACK ? y : p) + kHalf);
+  if (!is_v) {
+    float cl[8], ch[8], sl[8], sh[8];
+    load8(cl, cosine + (size_t)n * kD + d);
+    load8(ch, cosine + (size_t)n * kD + d + kHalf);
+    load8(sl, sine + (size_t)n * kD + d);
+    load8(sh, sine + (size_t)n * kD + d + kHalf);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float a = lo[e], c = hi[e];
+      lo[e] = BACK ? a * cl[e] + c * sh[e] : a * cl[e] - c * sl[e];
+      hi[e] = BACK ? c * ch[e] - a * sl[e] : c * ch[e] + a * sh[e];
+    }
+  }
+  store8(BACK ? p : y, lo);
+  store8((BACK ? p : y) + kHalf, hi);
+}
+
 template <typename T>
 void launch_expand_factor(const T* factor, bool per_head, int Hq, int G, double eps, T* c0, T* lam, T* gam,
                           hipStream_t st) {
@@ -246,6 +326,22 @@ void launch_expand_pairs(const float* b, const float* c, int Hq, int D, float* l
 }
 void launch_expand_pairs_bwd(const float* dgam, int Hq, int D, float* dc, hipStream_t st) {
   hipLaunchKernelGGL(k_expand_pairs_bwd, dim3(Hq), dim3(kThreads), 0, st, dgam, D, dc);
+}
+
+void launch_rotary_heads(bool f32, bool back, void* const (&t)[6], const void* cosine, const void* sine, int B, int N,
+                         int Hq, int Hkv, hipStream_t st) {
+  const size_t threads = (size_t)B * N * (Hq + 2 * Hkv) * (kD / 16);
+  const dim3 grid((unsigned)((threads + kThreads - 1) / kThreads)), block(kThreads);
+  auto launch = [&](auto* kernel, auto zero) {
+    using T = decltype(zero);
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, static_cast<T*>(t[0]), static_cast<T*>(t[1]), static_cast<T*>(t[2]),
+                       static_cast<T*>(t[3]), static_cast<T*>(t[4]), static_cast<T*>(t[5]),
+                       static_cast<const T*>(cosine), static_cast<const T*>(sine), B, N, Hq, Hkv);
+  };
+  if (f32)
+    back ? launch(k_rotary_heads<float, true>, 0.f) : launch(k_rotary_heads<float, false>, 0.f);
+  else
+    back ? launch(k_rotary_heads<uint16_t, true>, uint16_t{}) : launch(k_rotary_heads<uint16_t, false>, uint16_t{});
 }
 
 void launch_check_labels(const void* labels, bool wide, bool per_head, int D, int Hq, int G, int32_t* table, int* flag,

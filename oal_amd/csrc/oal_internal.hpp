@@ -302,6 +302,9 @@ void launch_expand_factor_bwd(const T* factor, bool per_head, int Hq, int G, con
 void launch_expand_pairs(const float* b, const float* c, int Hq, int D, float* lam, float* gam, int32_t* labels,
                          hipStream_t st);
 void launch_expand_pairs_bwd(const float* dgam, int Hq, int D, float* dc, hipStream_t st);
+// t: q, k, v projections, then q, k, v head-first.
+void launch_rotary_heads(bool f32, bool back, void* const (&t)[6], const void* cosine, const void* sine, int B, int N,
+                         int Hq, int Hkv, hipStream_t st);
 void launch_check_labels(const void* labels, bool wide, bool per_head, int D, int Hq, int G, int32_t* table, int* flag,
                          hipStream_t st);
 int launch_check_outputs(bool wide, int out_kind, const void* num, const void* den, const void* out, size_t rows,

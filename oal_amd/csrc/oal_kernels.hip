@@ -1415,6 +1415,22 @@ int oal_expand_pairs_backward(const float* dgam, int q_heads, int head_dim, floa
   return launch_status("oal_expand_pairs_backward launch");
 }
 
+int oal_rotary_heads(void* proj_q, void* proj_k, void* proj_v, void* head_q, void* head_k, void* head_v,
+                     const void* cosine, const void* sine, int back, int batch, int q_heads, int kv_heads, int seq_len,
+                     int dtype, void* stream) {
+  Range range("oal_rotary_heads");
+  Geometry g;
+  if (check_geometry(batch, q_heads, kv_heads, seq_len, dtype, &g)) return 1;
+  if (!cosine || !sine) return fail("oal_rotary_heads: null pointer argument");
+  void* const t[6] = {proj_q, proj_k, proj_v, head_q, head_k, head_v};
+  for (const void* p : t)
+    if (p && !aligned16(p)) return fail("oal_rotary_heads: tensor pointers must be 16-byte aligned");
+  if (!aligned16(cosine) || !aligned16(sine)) return fail("oal_rotary_heads: tensor pointers must be 16-byte aligned");
+  oal::launch_rotary_heads(dtype == OAL_DTYPE_F32, back != 0, t, cosine, sine, batch, seq_len, q_heads, kv_heads,
+                           static_cast<hipStream_t>(stream));
+  return launch_status("oal_rotary_heads launch");
+}
+
 int oal_check_labels(const void* labels, int wide, int per_head, int head_dim, int q_heads, int groups, int32_t* table,
                      int* flag, void* stream) {
   Range range("oal_check_labels");

@@ -22,7 +22,9 @@ It mirrors the reference adapter chain around the operator:
 * activation checkpointing of each decoder layer (model_setup.py:621-665).
 
 The attention runs in liboal_amd.so (precision "bf16_tensorcore": bf16 operands,
-fp32 accumulation on the matrix cores); the projections, norms and MLP are torch.
+fp32 accumulation on the matrix cores); the rotary embedding with
+the head-first layout is one kernel of the same library; the projections, norms and
+MLP are torch.
 """
 
 from __future__ import annotations
@@ -35,6 +37,7 @@ import torch.nn.functional as F
 from torch import nn
 from torch.utils.checkpoint import checkpoint
 
+from . import _native
 from .hd_block_gemm_adapters import prepare_grouped_hd_block_gemm, run_prepared_grouped_hd_block_gemm
 
 
@@ -99,6 +102,44 @@ def apply_rotary(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch
     half = x.shape[-1] // 2
     rot = torch.cat((-x[..., half:], x[..., :half]), dim=-1)
     return x * cos + rot * sin
+
+
+class _RotaryHeads(torch.autograd.Function):
+    """The operator's q, k, v from the projections' [B, N, heads * 64] (one kernel each
+    way, oal_adapter.hip): head-first, q and k rotated."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, cos, sin, q_heads: int, kv_heads: int):
+        ctx.set_materialize_grads(False)
+        ctx.save_for_backward(cos, sin)
+        ctx.heads = (q_heads, kv_heads)
+        return _native.rotary_heads(tuple(t.detach().contiguous() for t in (q, k, v)), cos, sin, q_heads, kv_heads,
+                                    back=False)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, dq, dk, dv):
+        if dq is None and dk is None and dv is None:
+            return (None,) * 7
+        cos, sin = ctx.saved_tensors
+        grads = tuple(None if t is None else t.contiguous() for t in (dq, dk, dv))
+        return (*_native.rotary_heads(grads, cos, sin, *ctx.heads, back=True), None, None, None, None)
+
+
+def rotary_heads(q, k, v, cos, sin, q_heads: int, kv_heads: int, head_dim: int):
+    """Projections [B, N, heads * D] -> head-first q, k, v [B, heads, N, D], q and k
+    rotated. One kernel for the operator's own types and head dimension with
+    tables that need no gradient; otherwise :func:`apply_rotary`."""
+    b, n, _ = q.shape
+    if (
+        head_dim == _native.HEAD_DIM and q.device.type == "cuda" and torch.version.hip is not None
+        and q.dtype in (torch.float32, torch.bfloat16)
+        and all(t.dtype == q.dtype and t.device == q.device for t in (k, v, cos, sin))
+        and cos.shape == sin.shape == (n, head_dim) and not (cos.requires_grad or sin.requires_grad)
+    ):
+        return _RotaryHeads.apply(q, k, v, cos.contiguous(), sin.contiguous(), q_heads, kv_heads)
+    q, k, v = (t.view(b, n, h, head_dim).transpose(1, 2) for t, h in ((q, q_heads), (k, kv_heads), (v, kv_heads)))
+    return apply_rotary(q, cos, sin).contiguous(), apply_rotary(k, cos, sin).contiguous(), v.contiguous()
 
 
 def seeded_layer_groups(cfg: QwenOALConfig, gen: torch.Generator) -> torch.Tensor:
@@ -181,12 +222,8 @@ class OALAttention(nn.Module):
     def forward(self, x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
         b, n, _ = x.shape
         hq, hkv, d = self.cfg.num_heads, self.cfg.num_kv_heads, self.cfg.head_dim
-        q = self.q_proj(x).view(b, n, hq, d).transpose(1, 2)
-        k = self.k_proj(x).view(b, n, hkv, d).transpose(1, 2)
-        v = self.v_proj(x).view(b, n, hkv, d).transpose(1, 2)
-        q = apply_rotary(q, cos, sin).contiguous()
-        k = apply_rotary(k, cos, sin).contiguous()
-        o = self.head_attention(q, k, v.contiguous())
+        q, k, v = rotary_heads(self.q_proj(x), self.k_proj(x), self.v_proj(x), cos, sin, hq, hkv, d)
+        o = self.head_attention(q, k, v)
         return self.o_proj(o.transpose(1, 2).reshape(b, n, hq * d))
 
 

@@ -69,6 +69,36 @@ def test_pair_expansion_and_its_vjp(d):
     assert torch.equal(shared[1][2].cpu()[:d], b[0]) and torch.equal(shared[2][2].cpu(), want[0])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,n,hq,hkv", [(1, 1, 1, 1), (2, 7, 14, 2), (3, 65, 4, 4)])
+def test_rotary_heads(dtype, b, n, hq, hkv):
+    """Against apply_rotary in float64: two products and a sum in fp32 (3 x 6e-8), then
+    one rounding to bf16 (2^-9)."""
+    from oal_amd.qwen_oal import apply_rotary, rotary_heads, rotary_tables
+
+    dev, tol = _dev(), 2e-7 if dtype == torch.float32 else 2.0 ** -9
+    gen = torch.Generator().manual_seed(n)
+    leaves = [torch.randn((b, n, h * 64), generator=gen).to(dtype) for h in (hq, hkv, hkv)]
+    cos, sin = rotary_tables(n, 64, 1e6, dev, dtype)
+    mine = [t.to(dev).requires_grad_() for t in leaves]
+    got = rotary_heads(*mine, cos, sin, hq, hkv, 64)
+    ref = [t.double().requires_grad_() for t in leaves]
+    c64, s64 = cos.cpu().double(), sin.cpu().double()
+    heads = [t.view(b, n, h, 64).transpose(1, 2) for t, h in zip(ref, (hq, hkv, hkv))]
+    want = [apply_rotary(heads[0], c64, s64), apply_rotary(heads[1], c64, s64), heads[2]]
+    up = [torch.randn(t.shape, generator=gen).to(dtype) for t in want]
+    for used in ((0, 1, 2), (0,), (1, 2)):
+        da = torch.autograd.grad([got[i] for i in used], [mine[i] for i in used], [up[i].to(dev) for i in used],
+                                 retain_graph=True)
+        dr = torch.autograd.grad([want[i] for i in used], [ref[i] for i in used], [up[i].double() for i in used],
+                                 retain_graph=True)
+        for a, r in zip(da, dr):
+            assert a.is_contiguous() and float((a.cpu().double() - r).norm() / r.norm()) <= tol
+    for a, r in zip(got, want):
+        assert a.dtype == dtype and a.is_contiguous()
+        assert float((a.detach().cpu().double() - r.detach()).norm() / r.detach().norm()) <= tol
+
+
 def _prefix(row, groups):
     used = sorted(set(row))
     return 1 if any(x < 0 or x >= groups for x in row) else 0 if used == list(range(len(used))) else 2
