@@ -28,10 +28,13 @@
 // the end; a tile costs a lane 44 FMAs for kappa, in the backward 64 for the
 // slopes and 45 for the coefficient sums, times four entries: VALU issue bounds
 // it in bf16, matrix-core issue in fp32 (v_mfma_f32_16x16x4_f32: 32 cycles for a
-// sixteenth of the bf16 depth). The bf16 backward is direct_roles. In short
-// sequences what counts is the chain from the first load to the first tile, so
-// every wave works its group structure out for itself without a barrier; N = 64
-// takes 8 us forward and 25 us backward, against 48 and 155 through the state.
+// sixteenth of the bf16 depth). The bf16 backward is in direct_dq and
+// direct_dk_dv (roles). In short sequences what counts is the chain from the first
+// load to the first tile, so every wave works its group structure out for itself
+// without a barrier; N = 64 takes 16 us forward and 28 us backward with the
+// launches, against 48 and 155 through the state. At full load the waves' VALU and matrix-core cycles add up
+// to the time (they hardly overlap): a step of 64 rows of the bf16 dq is 293 VALU
+// and 50 matrix instructions a wave.
 //
 // The dimensions are sorted by group in LDS, a window of 16 positions for each
 // group's first 16 dimensions and at most three more in all. A group's sum is then
@@ -55,7 +58,7 @@ constexpr int kM = kDirectTile;  // tile edge
 constexpr int kWv = 4;           // waves per block
 constexpr int kMore = 3;         // blocks beyond each group's first: 64 dimensions hold at most three
 
-enum Mode { kFwd, kDq, kDkv };
+enum Mode { kFwd, kDq, kDkv, kDk, kDv };
 
 constexpr int kStep = kM * kWv;  // streamed rows that a block's waves share (bf16 backward)
 
@@ -194,11 +197,18 @@ if ((int)threadIdx.x < ex) {
   return t;
 }
 
-// LDS offsets of this lane's 16 elements (dimensions 16 (l % 4) ..) in a sorted tile.
+// Byte offsets of this lane's 16 elements (dimensions 16 (l % 4) ..) in the sorted
+// tile of 16 rows that starts at row row0 of an array: added to the array's own
+// (constant) LDS address they cost a write no instruction.
 template <bool F32, int GP>
-__device__ __forceinline__ void piece_offsets(int (&off)[16], const Head<F32, GP>& t, int l) {
+__device__ __forceinline__ void piece_offsets(int (&off)[16], const Head<F32, GP>& t, int row0, int l) {
 #pragma unroll
-  for (int e = 0; e < 16; ++e) off[e] = (l >> 2) * Lay<F32, GP>::LS + __shfl(t.pos, 16 * (l & 3) + e, 64);
+  for (int e = 0; e < 16; ++e)
+    off[e] = (int)sizeof(Elem<F32>) * ((row0 + (l >> 2)) * Lay<F32, GP>::LS + __shfl(t.pos, 16 * (l & 3) + e, 64));
+}
+template <typename E>
+__device__ __forceinline__ E& at_byte(E* p, int off) {
+  return *reinterpret_cast<E*>(reinterpret_cast<char*>(p) + off);
 }
 
 template <typename T>
@@ -206,8 +216,8 @@ __device__ __forceinline__ void put_sorted(uint16_t* tile, const Piece<T>& p, co
 #pragma unroll
   for (int x = 0; x < 8; ++x) {
     const uint32_t w = piece_word(p, x);
-    tile[off[2 * x]] = (uint16_t)w;
-    tile[off[2 * x + 1]] = (uint16_t)(w >> 16);
+    at_byte(tile, off[2 * x]) = (uint16_t)w;
+    at_byte(tile, off[2 * x + 1]) = (uint16_t)(w >> 16);
   }
 }
 template <typename T>
@@ -215,10 +225,10 @@ __device__ __forceinline__ void put_sorted(float* tile, const Piece<T>& p, const
 #pragma unroll
   for (int x = 0; x < 4; ++x) {
     const float4 f = piece4(p, x);
-    tile[off[4 * x]] = f.x;
-    tile[off[4 * x + 1]] = f.y;
-    tile[off[4 * x + 2]] = f.z;
-    tile[off[4 * x + 3]] = f.w;
+    at_byte(tile, off[4 * x]) = f.x;
+    at_byte(tile, off[4 * x + 1]) = f.y;
+    at_byte(tile, off[4 * x + 2]) = f.z;
+    at_byte(tile, off[4 * x + 3]) = f.w;
   }
 }
 template <int LN, typename T>
@@ -361,7 +371,8 @@ __device__ __forceinline__ f32x4 mma(const Row<true>& a, const Row<true>& b, f32
 }
 
 // A head's scaled coefficients in scalar registers (zero beyond G groups):
-// quad[g (g + 1) / 2 + h] = A_gh for h <= g.
+// quad[g (g + 1) / 2 + h] = 2 A_gh for h < g; the diagonal is A_gg for kappa
+// alone, 2 A_gg where the slopes are formed (kappa then follows from them).
 template <int GP>
 struct Coef {
   float c0, lin[GP], quad[GP * (GP + 1) / 2];
@@ -369,15 +380,16 @@ struct Coef {
 __device__ __forceinline__ float lane_value(float x, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
 }
-template <bool F32, int GP>
-__device__ __forceinline__ Coef<GP> head_coefficients(const Head<F32, GP>& t, float c0) {
+template <bool SLOPES, bool F32, int GP>
+__device__ __forceinline__ Coef<GP> head_coefficients(const Head<F32, GP>& t, float c0, int l) {
+  const float twice = 2.f * t.gam, held = !SLOPES && l % 9 == 0 ? t.gam : twice;  // lanes 8 g + g
   Coef<GP> c;
   c.c0 = c0;
 #pragma unroll
   for (int g = 0; g < GP; ++g) {
     c.lin[g] = lane_value(t.lam, g);
 #pragma unroll
-    for (int x = 0; x <= g; ++x) c.quad[g * (g + 1) / 2 + x] = lane_value(t.gam, 8 * g + x);
+    for (int x = 0; x <= g; ++x) c.quad[g * (g + 1) / 2 + x] = lane_value(held, 8 * g + x);
   }
   return c;
 }
@@ -392,19 +404,19 @@ __device__ __forceinline__ float kappa_of(const Coef<GP>& c, const f32x4 (&s)[GP
   float k = c.c0;
 #pragma unroll
   for (int g = 0; g < GP; ++g) {
-    float t = 0.f;
+    float t = c.lin[g];
 #pragma unroll
-    for (int h = 0; h < g; ++h) t = fmaf(quad_of(c, g, h), s[h][r], t);
-    k = fmaf(s[g][r], fmaf(2.f, t, fmaf(quad_of(c, g, g), s[g][r], c.lin[g])), k);
+    for (int h = 0; h <= g; ++h) t = fmaf(quad_of(c, g, h), s[h][r], t);
+    k = fmaf(s[g][r], t, k);
   }
   return k;
 }
-// sum_h A_gh s_h
+// d kappa / d s_g = a_g + sum_h 2 A_gh s_h
 template <int GP>
-__device__ __forceinline__ float half_slope(const Coef<GP>& c, const f32x4 (&s)[GP], int g, int r) {
-  float t = quad_of(c, g, 0) * s[0][r];
+__device__ __forceinline__ float slope(const Coef<GP>& c, const f32x4 (&s)[GP], int g, int r) {
+  float t = c.lin[g];
 #pragma unroll
-  for (int h = 1; h < GP; ++h) t = fmaf(quad_of(c, g, h), s[h][r], t);
+  for (int h = 0; h < GP; ++h) t = fmaf(quad_of(c, g, h), s[h][r], t);
   return t;
 }
 
@@ -438,7 +450,9 @@ __device__ __forceinline__ void normalization_vjp(Piece<Elem<F32>>& gp, float& g
   const size_t at = (size_t)bh * a.N + (ok ? row : a.N - 1), o = at * kD + 16 * (l & 3);
   float g[16], dot = 0.f;
   const float dd = a.den[at];
-  const float dp = a.floor > 0.f ? fmaxf(dd, a.floor) : dd;
+  const float dp = a.floor > 0.f ? fmaxf(dd, a.floor) : dd, inv = 1.f / dp;
+  // bf16: G is rounded to 8 bits, so the reciprocal's rounding does not count
+  auto over = [&](float x) { return F32 ? x / dp : x * inv; };
 #pragma unroll
   for (int e = 0; e < 16; ++e) g[e] = 0.f;
   if (a.dout) {
@@ -450,10 +464,10 @@ __device__ __forceinline__ void normalization_vjp(Piece<Elem<F32>>& gp, float& g
     for (int e = 0; e < 4; ++e) {
       const float4 y = piece4(x, e), n = piece4(nm, e);
       dot = fmaf(y.x, n.x, fmaf(y.y, n.y, fmaf(y.z, n.z, fmaf(y.w, n.w, dot))));
-      g[4 * e] = y.x / dp;
-      g[4 * e + 1] = y.y / dp;
-      g[4 * e + 2] = y.z / dp;
-      g[4 * e + 3] = y.w / dp;
+      g[4 * e] = over(y.x);
+      g[4 * e + 1] = over(y.y);
+      g[4 * e + 2] = over(y.z);
+      g[4 * e + 3] = over(y.w);
     }
   }
   if (a.dnum) {
@@ -509,6 +523,7 @@ __device__ __forceinline__ void zero_lds(A& x) {
 // put(w) is called for wave w between two barriers, by that wave alone.
 template <typename F>
 __device__ __forceinline__ void in_wave_order(int wave, F&& put) {
+#pragma unroll 1
   for (int w = 0; w < kWv; ++w) {
     if (w == wave) put(w == 0);
     __syncthreads();
@@ -518,15 +533,16 @@ __device__ __forceinline__ void in_wave_order(int wave, F&& put) {
 }  // namespace
 
 template <typename T, bool F32, int GP, int MODE>
-__global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a) {
-  static_assert(MODE == kFwd || F32, "the bf16 backward is direct_roles");
+__device__ __forceinline__ void tiles(const Args<T, F32>& a, Shared<F32, GP>& sh) {
+  constexpr bool kSums = MODE == kFwd || MODE == kDv;   // products with kappa alone
+  constexpr bool kKeys = MODE == kDkv || MODE == kDv;   // the fixed rows are keys
+  static_assert(kSums || F32, "the rest of the bf16 backward is in roles");
   using L = Lay<F32, GP>;
   using E = Elem<F32>;
-  __shared__ __attribute__((aligned(16))) Shared<F32, GP> sh;
   const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
   const int NT = gridDim.x, bh = blockIdx.y, N = a.N;
   // the tiles with the most pairs first: the last ones to start are short
-  const int ft = MODE == kDkv ? (int)blockIdx.x : NT - 1 - (int)blockIdx.x;
+  const int ft = kKeys ? (int)blockIdx.x : NT - 1 - (int)blockIdx.x;
   const int R = a.Hq / a.Hkv, b = bh / a.Hq, h = bh % a.Hq, u = b * a.Hkv + h / R;
   const size_t qbase = (size_t)bh * N * kD, kbase = (size_t)u * N * kD;
   const int row0 = ft * kM;
@@ -536,17 +552,17 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
   // zero the sorted tiles once: the padding positions stay zero
   zero_lds(sh.sorted);
   zero_lds(sh.fixed);
-  if constexpr (F32 && MODE != kFwd) {
+  if constexpr (!kSums) {
     for (int x = threadIdx.x; x < 16 * L::kWin; x += 64 * kWv) sh.dim[x] = 255;
   }
   int off[16];
-  piece_offsets(off, hd, l);
+  piece_offsets(off, hd, wave * kM, l);
   __syncthreads();
-  if constexpr (F32 && MODE != kFwd) {
+  if constexpr (!kSums) {
     // fp32 positions run 4 (p % 4) + p / 4 within a window
     if (wave == 0) sh.dim[(hd.pos & ~15) + ((hd.pos & 3) * 4 + ((hd.pos >> 2) & 3))] = (uint8_t)l;
   }
-  const Coef<GP> cf = head_coefficients(hd, c0);
+  const Coef<GP> cf = head_coefficients<!kSums>(hd, c0, l);
 
   E* const srt = &sh.sorted[wave][0][0];
   E* const nat = &sh.natural[wave][0][0];
@@ -556,7 +572,7 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
   float gzc = 0.f;  // dq: Gz of the lane's query column
   {
     Piece<T> p;
-    load_tile(p, MODE == kDkv ? a.k + kbase : a.q + qbase, row0, N, l);
+    load_tile(p, kKeys ? a.k + kbase : a.q + qbase, row0, N, l);
     if (wave == 0) put_sorted(&sh.fixed[0][0], p, off);
     if constexpr (MODE == kDq) {
       Piece<E> gp;
@@ -570,7 +586,7 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
       put_natural<L::LN>(nat, p, l);
     }
     __syncthreads();
-    if constexpr (MODE != kFwd) f2 = read_row<L::LN>(nat, l);
+    if constexpr (!kSums) f2 = read_row<L::LN>(nat, l);
   }
   Blk<F32> f1[GP];
   int wo[GP];
@@ -583,30 +599,30 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
   wave_order();
 
   f32x4 acc[MODE == kDkv ? 4 : 1] = {};  // dv columns (dkv)
-  f32x4 gacc[MODE == kFwd ? 4 : GP + kMore] = {};  // forward: num columns; else the groups' gradient blocks
+  f32x4 gacc[kSums ? 4 : GP + kMore] = {};  // num or dv columns; else the groups' gradient blocks
   float z = 0.f;
   float co[MODE == kDq ? coef_count(GP) : 1];
 #pragma unroll
   for (int x = 0; x < (MODE == kDq ? coef_count(GP) : 1); ++x) co[x] = 0.f;
   const bool want_grad = MODE == kDkv || (MODE == kDq && a.dq), want_co = MODE == kDq && a.part;
   const int fc = row0 + lr;  // the lane's fixed token
-  const T* const s1 = MODE == kDkv ? a.q + qbase : a.k + kbase;
+  const T* const s1 = kKeys ? a.q + qbase : a.k + kbase;
   auto load_second = [&](auto& p, int r0) {
-    if constexpr (MODE == kDkv)
+    if constexpr (kKeys)
       load_tile(p, const_cast<const E*>(a.Gv) + qbase, r0, N, l);
     else
       load_tile(p, a.v + kbase, r0, N, l);
   };
-  const int begin = (MODE == kDkv ? ft : 0) + wave;
-  const int end = MODE == kFwd || want_grad || want_co ? (MODE == kDkv ? NT : ft + 1) : 0;
+  const int begin = (kKeys ? ft : 0) + wave;
+  const int end = kSums || want_grad || want_co ? (kKeys ? NT : ft + 1) : 0;
   Piece<T> p1;
-  std::conditional_t<MODE == kDkv, Piece<E>, Piece<T>> p2;
+  std::conditional_t<kKeys, Piece<E>, Piece<T>> p2;
   if (begin < end) {
     load_tile(p1, s1, begin * kM, N, l);
     load_second(p2, begin * kM);
   }
   for (int st = begin; st < end; st += kWv) {
-    put_sorted(srt, p1, off);
+    put_sorted(&sh.sorted[0][0][0], p1, off);
     put_natural<L::LN>(nat, p2, l);
     wave_order();
     if (st + kWv < end) {  // the next tile's rows, in flight during this one
@@ -628,27 +644,34 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
           for (int r = 0; r < 4; ++r) s[g][r] += sh.more.group[x] == g ? e[r] : 0.f;
       }
     }
-    bool ok[4];
+    // tiles off the diagonal and inside the sequence: every pair counts
+    const bool edge = kKeys ? st <= ft || (st + 1) * kM > N : st >= ft;
+    auto mask = [&](f32x4& x) {
+      if (!edge) return;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int sc = st * kM + 4 * lg + r;
+        x[r] = (kKeys ? fc <= sc && sc < N && fc < N : sc <= fc && sc < N) ? x[r] : 0.f;
+      }
+    };
     f32x4 ds = {};
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int sc = st * kM + 4 * lg + r;
-      ok[r] = MODE == kDkv ? fc <= sc && sc < N && fc < N : sc <= fc && sc < N;
       if constexpr (MODE == kDkv) ds[r] = a.Gz[(size_t)bh * N + (sc < N ? sc : N - 1)];
       if constexpr (MODE == kDq) ds[r] = gzc;
     }
-    if constexpr (MODE != kFwd) {
+    if constexpr (!kSums) {
       ds = mma(read_row<L::LN>(nat, l), f2, ds);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ds[r] = ok[r] ? ds[r] : 0.f;
+      mask(ds);
     }
-    if constexpr (MODE == kFwd) {
+    if constexpr (kSums) {
       f32x4 kap;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        kap[r] = ok[r] ? kappa_of<GP>(cf, s, r) : 0.f;
-        z += kap[r];
-      }
+      for (int r = 0; r < 4; ++r) kap[r] = kappa_of<GP>(cf, s, r);
+      mask(kap);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) z += kap[r];
       const Blk<F32> ka = as_operand<F32>(kap);
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb) gacc[cb] = mma(ka, rows_operand(nat, L::LN, 16 * cb, lr, l), gacc[cb]);
@@ -669,18 +692,18 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
         }
       }
     }
-    if constexpr (MODE != kFwd) {
+    if constexpr (!kSums) {
       if (want_grad) {
-        f32x4 kap = {cf.c0, cf.c0, cf.c0, cf.c0};
+        f32x4 kap = {2.f * cf.c0, 2.f * cf.c0, 2.f * cf.c0, 2.f * cf.c0};  // twice kappa
         f32x4 xm[kMore] = {};  // the tiles of the groups that hold the further blocks
 #pragma unroll
         for (int g = 0; g < GP; ++g) {
           f32x4 x;
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float t = half_slope<GP>(cf, s, g, r);
+            const float t = slope<GP>(cf, s, g, r);
             if constexpr (MODE == kDkv) kap[r] = fmaf(s[g][r], cf.lin[g] + t, kap[r]);
-            x[r] = ds[r] * fmaf(2.f, t, cf.lin[g]);
+            x[r] = ds[r] * t;
           }
           const Blk<F32> xa = as_operand<F32>(x);
           gacc[g] = mma(xa, rows_operand(srt, L::LS, hd.at[g], L::in_block(lr), l), gacc[g]);
@@ -698,8 +721,8 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
                                gacc[GP + m]);
         }
         if constexpr (MODE == kDkv) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) kap[r] = ok[r] ? kap[r] : 0.f;
+          kap *= 0.5f;
+          mask(kap);
           const Blk<F32> ka = as_operand<F32>(kap);
 #pragma unroll
           for (int cb = 0; cb < 4; ++cb) acc[cb] = mma(ka, rows_operand(nat, L::LN, 16 * cb, lr, l), acc[cb]);
@@ -732,7 +755,7 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float* const row = t0 + (4 * lg + r) * kD;
-      if constexpr (MODE == kFwd) {
+      if constexpr (kSums) {
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb) row[16 * cb + lr] = gacc[cb][r] + (fresh ? 0.f : row[16 * cb + lr]);
       } else {
@@ -779,6 +802,13 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
     *reinterpret_cast<float4*>(a.dkh + o) = x;
     *reinterpret_cast<float4*>(a.dvh + o) = *reinterpret_cast<const float4*>(t1 + er * kD + ec);
   }
+  if constexpr (MODE == kDv) *reinterpret_cast<float4*>(a.dvh + qbase + (size_t)tok * kD + ec) = x;
+}
+
+template <typename T, bool F32, int GP, int MODE>
+__global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a) {
+  __shared__ __attribute__((aligned(16))) Shared<F32, GP> sh;
+  tiles<T, F32, GP, MODE>(a, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -792,25 +822,27 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
 // t_g and the 45 coefficient products formed per pair. For the coefficient sums ds
 // s_h goes in as two bf16 halves (as one, their error was 1.07 to 1.14 times as
 // large as that of fp32 sums over the pairs up to N = 256). dk likewise, with the
-// streamed q and one half; dv needs kappa, formed as in the forward.
+// streamed q and one half; dv needs kappa, formed as in the forward (tiles).
 //
 // All (GP + 1) x 4 column blocks of P are 144 registers, too many for one wave,
 // and P_h needs s_h alone: the four waves share each staged step of 64 streamed
-// rows and wave w takes the groups w GP / 4 .. and column block w of P_GP. For
-// kappa (dkv) each wave takes its own 16 rows of the step. Two tiles of a step
-// make one 32-deep product (k slots 8 g + 0 .. 3 the first tile's rows 4 g .., + 4
+// rows and wave w takes the groups w GP / 4 .. and column block w of P_GP. Two
+// tiles of a step make one 32-deep product (k slots 8 g + 0 .. 3 the first tile's rows 4 g .., + 4
 // .. 7 the second's).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ bf16x8 both(s16x4 a, s16x4 b) {
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 // x in bf16, and with two halves also what that leaves: x to 2^-17.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void split4(s16x4 (&h)[1], const float (&x)[4]) { h[0] = pack4(x); }
 __device__ __forceinline__ void split4(s16x4 (&h)[2], const float (&x)[4]) {
-  h[0] = pack4(x);
+  const u32x2 w = {pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
   float y[4];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) y[r] = x[r] - bf16_to_f((uint16_t)h[0][r]);
+  for (int r = 0; r < 4; ++r)
+    y[r] = x[r] - __uint_as_float(r & 1 ? w[r >> 1] & 0xffff0000u : w[r >> 1] << 16);
+  h[0] = __builtin_bit_cast(s16x4, w);
   h[1] = pack4(y);
 }
 
@@ -823,43 +855,41 @@ struct SharedRoles {
       uint16_t nat1[kStep][L::LN], nat2[kStep][L::LN];  // k and v, or q and G
     };
     struct {
-      float t0[kM][kD], t1[kM][kD];  // results
-      float y[GP + 1][kD];           // coefficient sums per dimension
+      float t0[kM][kD];     // results
+      float y[GP + 1][kD];  // coefficient sums per dimension
     };
   };
   uint16_t fixed[kM][L::LS];
-  uint16_t fnat[kM][L::LN];  // dq: q; dkv: unused
-  float gz[kStep];           // dkv: Gz of the step's rows
+  uint16_t fnat[kM][L::LN];  // dq: q
+  float gz[kStep];           // dk: Gz of the step's rows
   int grp[kD];               // dq: group of a dimension
   More more;
   float dc0[kWv];
 };
 
 template <typename T, int GP, int MODE>
-__global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false> a) {
+__device__ __forceinline__ void roles(const Args<T, false>& a, SharedRoles<GP>& sh) {
   using L = Lay<false, GP>;
   constexpr int kOwn = GP / kWv;  // groups per wave
-  __shared__ __attribute__((aligned(16))) SharedRoles<GP> sh;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, lr = l & 15, lg = l >> 4;
   const int NT = gridDim.x, bh = blockIdx.y, N = a.N;
-  const int ft = MODE == kDkv ? (int)blockIdx.x : NT - 1 - (int)blockIdx.x;
+  const int ft = MODE == kDk ? (int)blockIdx.x : NT - 1 - (int)blockIdx.x;
   const int R = a.Hq / a.Hkv, b = bh / a.Hq, h = bh % a.Hq, u = b * a.Hkv + h / R;
   const size_t qbase = (size_t)bh * N * kD, kbase = (size_t)u * N * kD;
   const int row0 = ft * kM;
 
-  const float c0 = MODE == kDkv ? a.c0[h] : 0.f;
   const Head<false, GP> hd = read_head<false, GP>(a.labels, a.lam, a.gam, a.G, h, a.scale, l, sh.more);
   zero_lds(sh.sorted);
   zero_lds(sh.fixed);
   if (MODE == kDq && wave == 0) sh.grp[l] = hd.lab;
   int off[16];
-  piece_offsets(off, hd, l);
+  piece_offsets(off, hd, wave * kM, l);
   __syncthreads();
   Row<false> f2;
   float gzc = 0.f;
   {
     Piece<T> p;
-    load_tile(p, MODE == kDkv ? a.k + kbase : a.q + qbase, row0, N, l);
+    load_tile(p, MODE == kDk ? a.k + kbase : a.q + qbase, row0, N, l);
     if (wave == 0) put_sorted(&sh.fixed[0][0], p, off);
     if constexpr (MODE == kDq) {
       if (wave == 0) put_natural<L::LN>(&sh.fnat[0][0], p, l);
@@ -875,9 +905,9 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
     __syncthreads();
     f2 = read_row<L::LN>(&sh.nat2[0][0], l);
   }
-  // for kappa, every group; for P, the wave's own
-  Blk<false> f1[MODE == kDkv ? GP : 1], fo[kOwn];
-  int wo[MODE == kDkv ? GP : 1], wown[kOwn];
+  // the wave's own groups
+  Blk<false> fo[kOwn];
+  int wown[kOwn];
 #pragma unroll
   for (int x = 0; x < kOwn; ++x) {
     int at = hd.at[x], n = hd.count[x];
@@ -889,31 +919,20 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
     fo[x] = fixed_window(&sh.fixed[lr][0], at, n, l);
     wown[x] = window_offset<false, GP>(at, l);
   }
-  if constexpr (MODE == kDkv) {
-#pragma unroll
-    for (int g = 0; g < GP; ++g) {
-      f1[g] = fixed_window(&sh.fixed[lr][0], hd.at[g], hd.count[g], l);
-      wo[g] = window_offset<false, GP>(hd.at[g], l);
-    }
-  }
   const bool any_more = hd.any_more;
-  Coef<GP> cf;
-  if constexpr (MODE == kDkv) cf = head_coefficients(hd, c0);
-
   f32x4 P[kOwn][4] = {}, Pl = {};
-  f32x4 dv[MODE == kDkv ? 4 : 1] = {};
   float c0sum = 0.f;
   const int fc = row0 + lr;
-  const bool want = MODE == kDkv || a.dq || a.part;
-  const int begin = MODE == kDkv ? ft / 4 : 0, end = want ? (MODE == kDkv ? (NT + 3) / 4 : ft / 4 + 1) : 0;
-  const T* const s1 = MODE == kDkv ? a.q + qbase : a.k + kbase;
+  const bool want = MODE == kDk || a.dq || a.part;
+  const int begin = MODE == kDk ? ft / 4 : 0, end = want ? (MODE == kDk ? (NT + 3) / 4 : ft / 4 + 1) : 0;
+  const T* const s1 = MODE == kDk ? a.q + qbase : a.k + kbase;
   Piece<T> p1;
-  std::conditional_t<MODE == kDkv, Piece<uint16_t>, Piece<T>> p2;
+  std::conditional_t<MODE == kDk, Piece<uint16_t>, Piece<T>> p2;
   float pz = 0.f;
   auto fetch = [&](int step) {
     const int r0 = step * kStep + wave * kM;
     load_tile(p1, s1, r0, N, l);
-    if constexpr (MODE == kDkv) {
+    if constexpr (MODE == kDk) {
       load_tile(p2, const_cast<const uint16_t*>(a.Gv) + qbase, r0, N, l);
       const int row = r0 + lr;
       pz = a.Gz[(size_t)bh * N + (row < N ? row : N - 1)];
@@ -924,10 +943,10 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
   if (begin < end) fetch(begin);
   for (int step = begin; step < end; ++step) {
     lds_sync();  // the previous step's reads (and the prologue's)
-    put_sorted(&sh.sorted[wave * kM][0], p1, off);
+    put_sorted(&sh.sorted[0][0], p1, off);
     put_natural<L::LN>(&sh.nat1[wave * kM][0], p1, l);
     put_natural<L::LN>(&sh.nat2[wave * kM][0], p2, l);
-    if constexpr (MODE == kDkv) {
+    if constexpr (MODE == kDk) {
       if (lg == 0) sh.gz[wave * kM + lr] = pz;
     }
     lds_sync();
@@ -936,7 +955,7 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
 #pragma unroll 1
     for (int pr = 0; pr < 2; ++pr) {
       const int ta = t0 + 2 * pr;
-      if (MODE == kDkv ? ta + 1 < ft || ta >= NT : ta > ft) continue;
+      if (MODE == kDk ? ta + 1 < ft || ta >= NT : ta > ft) continue;
       // dq: both halves of ds s_h, since the coefficient sums are fp32 sums of fp32 values
       constexpr int kHalves = MODE == kDq ? 2 : 1;
       s16x4 xh[2][kOwn][kHalves], xl[2][kHalves];
@@ -944,7 +963,7 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
       for (int e = 0; e < 2; ++e) {
         const int r0 = (2 * pr + e) * kM, tok = (ta + e) * kM + 4 * lg;
         f32x4 ds;
-        if constexpr (MODE == kDkv) {
+        if constexpr (MODE == kDk) {
           ds = *reinterpret_cast<const f32x4*>(&sh.gz[r0 + 4 * lg]);
         } else {
           ds = f32x4{gzc, gzc, gzc, gzc};
@@ -967,11 +986,13 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
               for (int r = 0; r < 4; ++r) s[x][r] += mg == wave * kOwn + x ? v[r] : 0.f;
           }
         }
-        float y[4];
+        float y[4] = {ds[0], ds[1], ds[2], ds[3]};
+        if (MODE == kDk ? ta + e <= ft || (ta + e + 1) * kM > N : ta + e >= ft) {  // else every pair counts
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const bool ok = MODE == kDkv ? fc <= tok + r && tok + r < N && fc < N : tok + r <= fc && tok + r < N;
-          y[r] = ok ? ds[r] : 0.f;
+          for (int r = 0; r < 4; ++r) {
+            const bool ok = MODE == kDk ? fc <= tok + r && tok + r < N && fc < N : tok + r <= fc && tok + r < N;
+            y[r] = ok ? y[r] : 0.f;
+          }
         }
         if (MODE == kDq && ((ta + e) & 3) == wave) c0sum += (y[0] + y[1]) + (y[2] + y[3]);
         split4(xl[e], y);
@@ -998,34 +1019,6 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
 #pragma unroll
       for (int f = 0; f < kHalves; ++f) Pl = mfma16(both(xl[0][f], xl[1][f]), kl, Pl);
     }
-    if constexpr (MODE == kDkv) {
-      const int t = t0 + wave;
-      if (t >= ft && t < NT) {
-        const int r0 = wave * kM, tok = t * kM + 4 * lg;
-        f32x4 s[GP];
-#pragma unroll
-        for (int g = 0; g < GP; ++g)
-          s[g] = mma(read_at<false>(&sh.sorted[r0][0], wo[g]), f1[g], f32x4{});
-        if (any_more) {
-#pragma unroll
-          for (int m = 0; m < kMore; ++m) {
-            const f32x4 v = mma(read_window<false>(&sh.sorted[r0 + lr][0], sh.more.at[m], l),
-                                fixed_window(&sh.fixed[lr][0], sh.more.at[m], sh.more.count[m], l), f32x4{});
-#pragma unroll
-            for (int g = 0; g < GP; ++g)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) s[g][r] += sh.more.group[m] == g ? v[r] : 0.f;
-          }
-        }
-        float kap[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) kap[r] = fc <= tok + r && tok + r < N && fc < N ? kappa_of<GP>(cf, s, r) : 0.f;
-        const s16x4 ka = pack4(kap);
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-          dv[cb] = mfma16k16(ka, rows_operand(&sh.nat2[r0][0], L::LN, 16 * cb, 0, l).v, dv[cb]);
-      }
-    }
   }
 
   // the waves' parts in wave order, through LDS
@@ -1044,7 +1037,6 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
 #pragma unroll
         for (int x = 0; x < kOwn; ++x) v = fmaf(c[x], P[x][cb][r], v);
         sh.t0[4 * lg + r][d] = fmaf(cl, Pl[r], v);
-        if constexpr (MODE == kDkv) sh.t1[4 * lg + r][d] = dv[cb][r] + (fresh ? 0.f : sh.t1[4 * lg + r][d]);
       }
     }
   });
@@ -1077,7 +1069,19 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
       if (t < (GP + 1) * GP) {
         const int hh = t / GP, g = t % GP;
         float y = 0.f;
-        for (int d = 0; d < kD; ++d) y += sh.grp[d] == g ? sh.y[hh][d] : 0.f;
+#pragma unroll 1
+        for (int d0 = 0; d0 < kD; d0 += 16) {
+          float v[16];
+          int o[16];
+#pragma unroll
+          for (int d = 0; d < 16; ++d) {
+            v[d] = sh.y[hh][d0 + d];
+            o[d] = sh.grp[d0 + d];
+            asm volatile("" : "+v"(v[d]));  // read whether or not it counts, not behind a branch
+          }
+#pragma unroll
+          for (int d = 0; d < 16; ++d) y += o[d] == g ? v[d] : 0.f;
+        }
         dst[1 + t] = y;
       }
       if (t == 0) dst[0] = (sh.dc0[0] + sh.dc0[1]) + (sh.dc0[2] + sh.dc0[3]);
@@ -1091,8 +1095,28 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_roles(const Args<T, false>
     if (a.dq) store4(a.dq + o, x);
   } else {
     *reinterpret_cast<float4*>(a.dkh + o) = x;
-    *reinterpret_cast<float4*>(a.dvh + o) = *reinterpret_cast<const float4*>(&sh.t1[er][ec]);
   }
+}
+
+template <typename T, int GP>
+__global__ __launch_bounds__(64 * kWv, 3) void direct_dq(const Args<T, false> a) {
+  __shared__ __attribute__((aligned(16))) SharedRoles<GP> sh;
+  roles<T, GP, kDq>(a, sh);
+}
+
+// dk in the blocks of z = 0, dv in those of z = 1: side by side their chains
+// overlap, and each needs fewer registers than one kernel of both (201 and two
+// waves per SIMD).
+template <typename T, int GP>
+__global__ __launch_bounds__(64 * kWv, 3) void direct_dk_dv(const Args<T, false> a) {
+  __shared__ __attribute__((aligned(16))) union {
+    SharedRoles<GP> k;
+    Shared<false, GP> v;
+  } sh;
+  if (blockIdx.z == 0)
+    roles<T, GP, kDk>(a, sh.k);
+  else
+    tiles<T, false, GP, kDv>(a, sh.v);
 }
 
 // The last launch of a backward: blocks [0, sums) add the unit's R heads of dk
@@ -1209,8 +1233,10 @@ void backward_of(const LaunchGeom& g, const Args<T, F32>& a, const Work<F32>& w,
     if (kv)
       timed("direct_dkv", st, [&] { hipLaunchKernelGGL((direct_tiles<T, true, GP, kDkv>), grid, block, 0, st, a); });
   } else {
-    timed("direct_dq", st, [&] { hipLaunchKernelGGL((direct_roles<T, GP, kDq>), grid, block, 0, st, a); });
-    if (kv) timed("direct_dkv", st, [&] { hipLaunchKernelGGL((direct_roles<T, GP, kDkv>), grid, block, 0, st, a); });
+    timed("direct_dq", st, [&] { hipLaunchKernelGGL((direct_dq<T, GP>), grid, block, 0, st, a); });
+    if (kv)
+      timed("direct_dkv", st,
+            [&] { hipLaunchKernelGGL((direct_dk_dv<T, GP>), dim3(grid.x, grid.y, 2), block, 0, st, a); });
   }
   const size_t per_head = (size_t)g.N * kD, total4 = (size_t)g.B * g.Hkv * per_head / 4;
   const int sums = kv ? (int)((total4 + 255) / 256) : 0, heads = dc0 ? g.Hq : 0;

@@ -16,19 +16,21 @@ constexpr int kDirectTile = 16;  // tokens per tile edge
 // shorter one. A function of the geometry alone, so that the size queries and
 // both directions agree. A direct call costs its launches and the longest row,
 // its 16 x 16 tiles and its blocks of 16 rows; the state route its longer chain
-// of launches and its rows. Measured, bf16, 14/2 heads and 8 groups, direct
-// against state: B=1 N=128 49 / 216, N=512 87 / 237, N=1024 190 / 255, N=1536
-// 334 / 266; B=2 N=800 210 / 276, N=1000 297 / 269; B=8 N=512 413 / 319; B=64
-// N=128 393 / 458. fp32: B=1 N=256 90 / 438, N=1024 400 / 581, N=1536 744 / 674;
-// B=4 N=512 502 / 800, N=1024 1343 / 1241; B=64 N=256 2440 / 3818. Up to 4
-// groups: bf16 B=4 N=512 170 / 257, fp32 B=4 N=1024 777 / 1159.
+// of launches (in bf16 with 30 us for what the host takes longer over them) and
+// its rows. Measured, bf16, 14/2 heads and 8 groups, direct against state: B=1
+// N=128 46 / 216, N=512 90 / 238, N=1024 177 / 257, N=1300 233 / 266, N=1600 299 /
+// 277; B=2 N=800 196 / 274, N=1000 272 / 270, N=1200 335 / 315; B=8 N=512 394 /
+// 315; B=64 N=128 404 / 437, N=256 1011 / 929. fp32: B=1 N=256 93 / 438, N=1024
+// 426 / 586, N=1536 766 / 663; B=4 N=512 502 / 800, N=1024 1394 / 1202; B=64 N=256
+// 2589 / 3814. Up to 4 groups: bf16 B=1 N=1600 228 / 280, B=4 N=1024 408 / 321;
+// fp32 B=1 N=2048 629 / 769, B=4 N=1024 755 / 1171.
 inline bool direct_route(bool f32, int groups, int B, int Hq, int N) {
   if (groups > 8 || (long)B * Hq > 65535) return false;
   const double nt = (N + kDirectTile - 1) / kDirectTile, blocks = (double)B * Hq * nt, tiles = blocks * (nt + 1) / 2,
                rows = (double)B * Hq * N;
   const bool few = groups <= 4;
   if (f32) return 60 + 0.03 * N + (few ? 0.0042 : 0.0082) * tiles + (few ? 0.06 : 0.085) * blocks < 420 + 0.0145 * rows;
-  return 30 + 0.03 * N + (few ? 0.0029 : 0.0042) * tiles + 0.031 * blocks < 200 + 0.0028 * rows;
+  return 35 + 0.02 * N + (few ? 0.0018 : 0.0027) * tiles + (few ? 0.05 : 0.055) * blocks < 230 + 0.0028 * rows;
 }
 
 // Workspace of a direct backward.
