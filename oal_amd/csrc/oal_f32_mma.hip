@@ -311,6 +311,8 @@ __global__ __launch_bounds__(256) void k3_seg_carry(float* __restrict__ segt, fl
 // ---------------------------------------------------------------------------
 constexpr int kStRow = kD + 4;
 constexpr int kMT = kS / 32;  // 69
+constexpr int kSlices = kF32Slices, kSliceTiles = kMT / kSlices;
+static_assert(kSlices == 3 && kSlices * kSliceTiles == kMT, "three equal slices of the tiles");
 
 // NT threads stage one tile: thread t moves 2048 / NT values (float4s) and,
 // for t < 32, the ones column of row t. With wqh (a query head's feature
@@ -414,7 +416,7 @@ __device__ __forceinline__ void readout_base(const float (&x)[kD], const float* 
 // then takes tile M + 1 + PD. Two help the dv readout (one block per chunk and
 // unit, few waves per CU); the query readout, with seven times the blocks,
 // keeps one and its fourth wave per SIMD.
-template <int M, int MODE, bool ADD, int PD>
+template <int M, int END, int MODE, bool ADD, int PD>
 __device__ __forceinline__ void readout_tiles(const float (&x)[kD], float* st0, float* st1,
                                               const float* __restrict__ S, const float* __restrict__ Sz, size_t cb,
                                               const float* wqh, int m, int s, int row, TileRegs<256> (&tr)[PD],
@@ -423,24 +425,38 @@ __device__ __forceinline__ void readout_tiles(const float (&x)[kD], float* st0, 
   [&]<int... J>(std::integer_sequence<int, J...>) {
     (readout_base<16 * M + J, MODE>(x, st, m, s, row, acc, zacc), ...);
   }(std::make_integer_sequence<int, 16>{});
-  if constexpr (M + 1 < kMT) {
+  if constexpr (M + 1 < END) {
     store_tile<256, ADD, MODE == 0>((M & 1) ? st0 : st1, tr[(M + 1) % PD]);
-    if constexpr (M + 1 + PD < kMT)
+    if constexpr (M + 1 + PD < END)
       load_tile<256, ADD, MODE == 0>(S, Sz, cb, M + 1 + PD, wqh, natl, tr[(M + 1) % PD], sc);
     lds_sync();
     __builtin_amdgcn_sched_barrier(0);
-    readout_tiles<M + 1, MODE, ADD, PD>(x, st0, st1, S, Sz, cb, wqh, m, s, row, tr, acc, zacc, natl, sc);
+    readout_tiles<M + 1, END, MODE, ADD, PD>(x, st0, st1, S, Sz, cb, wqh, m, s, row, tr, acc, zacc, natl, sc);
   }
 }
+// The tiles [M0, END) from the first load on.
+template <int M0, int END, int MODE, bool ADD, int PD>
+__device__ __forceinline__ void readout_range(const float (&x)[kD], float* st0, float* st1,
+                                              const float* __restrict__ S, const float* __restrict__ Sz, size_t cb,
+                                              const float* wqh, int m, int s, int row, f32x16& acc, float& zacc,
+                                              const int16_t* natl, const SegCarry& sc) {
+  TileRegs<256> tr[PD];
+  load_tile<256, ADD, MODE == 0>(S, Sz, cb, M0, wqh, natl, tr[M0 % PD], sc);
+  store_tile<256, ADD, MODE == 0>((M0 & 1) ? st1 : st0, tr[M0 % PD]);
+#pragma unroll
+  for (int i = 1; i <= PD; ++i) load_tile<256, ADD, MODE == 0>(S, Sz, cb, M0 + i, wqh, natl, tr[(M0 + i) % PD], sc);
+  __syncthreads();
+  readout_tiles<M0, END, MODE, ADD, PD>(x, st0, st1, S, Sz, cb, wqh, m, s, row, tr, acc, zacc, natl, sc);
+}
 
-template <typename T, int MODE, bool CARRY = false>
+template <typename T, int MODE, bool CARRY = false, bool SLICED = false>
 __global__ __launch_bounds__(256, 2) void k3_readout(const T* __restrict__ x_in, const float* __restrict__ wq,
                                                      const float* __restrict__ S, const float* __restrict__ Sz, int Hq,
                                                      int Hkv, int N, int NB, float floor, float* __restrict__ num,
                                                      float* __restrict__ den, T* __restrict__ out,
                                                      const float* __restrict__ dvl, T* __restrict__ dv,
                                                      const float* __restrict__ cS, const float* __restrict__ cSz,
-                                                     int SL, int nseg) {
+                                                     int SL, int nseg, float* __restrict__ part, int U) {
   __shared__ __attribute__((aligned(16))) float st0[32 * kStRow], st1[32 * kStRow];
   __shared__ float zd[kC];
   __shared__ int16_t natl[kS];
@@ -468,15 +484,26 @@ __global__ __launch_bounds__(256, 2) void k3_readout(const T* __restrict__ x_in,
   for (int i = tid; i < kS; i += 256) natl[i] = kSlot3.nat[i];
   __syncthreads();
   constexpr int PD = MODE == 1 ? 2 : 1;
-  TileRegs<256> tr[PD];
-  load_tile<256, CARRY, MODE == 0>(S, Sz, cb, 0, wqh, natl, tr[0], sc);
-  store_tile<256, CARRY, MODE == 0>(st0, tr[0]);
-#pragma unroll
-  for (int i = 1; i <= PD; ++i) load_tile<256, CARRY, MODE == 0>(S, Sz, cb, i, wqh, natl, tr[i % PD], sc);
-  __syncthreads();
   f32x16 acc = f32x16{};
   float zacc = 0.f;
-  readout_tiles<0, MODE, CARRY, PD>(x, st0, st1, S, Sz, cb, wqh, m, s, row, tr, acc, zacc, natl, sc);
+  if constexpr (SLICED) {
+    auto run = [&](auto first) {
+      constexpr int kM0 = decltype(first)::value * kSliceTiles;
+      readout_range<kM0, kM0 + kSliceTiles, MODE, CARRY, PD>(x, st0, st1, S, Sz, cb, wqh, m, s, row, acc, zacc, natl, sc);
+    };
+    if (blockIdx.y == 0) run(std::integral_constant<int, 0>{});
+    if (blockIdx.y == 1) run(std::integral_constant<int, 1>{});
+    if (blockIdx.y == 2) run(std::integral_constant<int, 2>{});
+    if (ok) {
+      float* prow = part + ((size_t)blockIdx.y * U * N + (size_t)u * N + tok) * kD + 32 * m + 4 * s;
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+        *reinterpret_cast<float4*>(prow + 8 * a) =
+            make_float4(acc[4 * a], acc[4 * a + 1], acc[4 * a + 2], acc[4 * a + 3]);
+    }
+    return;
+  }
+  readout_range<0, kMT, MODE, CARRY, PD>(x, st0, st1, S, Sz, cb, wqh, m, s, row, acc, zacc, natl, sc);
 
   if constexpr (MODE == 0) {
     const size_t dbase = (size_t)(b * Hq + h) * N;
@@ -554,30 +581,42 @@ __device__ __forceinline__ void fold_tile_f32(const float (&x)[kD], float (&dx)[
   fold::fold_tile<M>(D, x, dx, w16);
 }
 
-template <int M, bool ADD, bool W>
+template <int M, int END, bool ADD, bool W>
 __device__ __forceinline__ void fold_tiles(const float (&x)[kD], float (&dx)[kD], const float (&yv)[32], float yz,
                                            float* st0, float* st1, const float* __restrict__ S,
                                            const float* __restrict__ Sz, size_t cb, const float* wqh, int s, int row,
                                            TileRegs<128>& tr, const int16_t* natl, const SegCarry& sc) {
   pin64(dx);
   fold_tile_f32<M>(x, dx, yv, yz, (M & 1) ? st1 : st0, s, row);
-  if constexpr (M + 1 < kMT) {
+  if constexpr (M + 1 < END) {
     store_tile<128, ADD, W>((M & 1) ? st0 : st1, tr);
-    if constexpr (M + 2 < kMT) load_tile<128, ADD, W>(S, Sz, cb, M + 2, wqh, natl, tr, sc);
+    if constexpr (M + 2 < END) load_tile<128, ADD, W>(S, Sz, cb, M + 2, wqh, natl, tr, sc);
     lds_sync();
     __builtin_amdgcn_sched_barrier(0);
-    fold_tiles<M + 1, ADD, W>(x, dx, yv, yz, st0, st1, S, Sz, cb, wqh, s, row, tr, natl, sc);
+    fold_tiles<M + 1, END, ADD, W>(x, dx, yv, yz, st0, st1, S, Sz, cb, wqh, s, row, tr, natl, sc);
   }
 }
+template <int M0, int END, bool ADD, bool W>
+__device__ __forceinline__ void fold_range(const float (&x)[kD], float (&dx)[kD], const float (&yv)[32], float yz,
+                                           float* st0, float* st1, const float* __restrict__ S,
+                                           const float* __restrict__ Sz, size_t cb, const float* wqh, int s, int row,
+                                           const int16_t* natl, const SegCarry& sc) {
+  TileRegs<128> tr;
+  load_tile<128, ADD, W>(S, Sz, cb, M0, wqh, natl, tr, sc);
+  store_tile<128, ADD, W>((M0 & 1) ? st1 : st0, tr);
+  load_tile<128, ADD, W>(S, Sz, cb, M0 + 1, wqh, natl, tr, sc);
+  __syncthreads();
+  fold_tiles<M0, END, ADD, W>(x, dx, yv, yz, st0, st1, S, Sz, cb, wqh, s, row, tr, natl, sc);
+}
 
-template <typename T, int MODE, bool CARRY = false>
+template <typename T, int MODE, bool CARRY = false, bool SLICED = false>
 __global__ __launch_bounds__(128, 2) void k3_fold(const T* __restrict__ x_in, const float* __restrict__ y_in,
                                                   const T* __restrict__ v_in, const float* __restrict__ yz_in,
                                                   const float* __restrict__ wq, const float* __restrict__ S,
                                                   const float* __restrict__ Sz, const float* __restrict__ local,
                                                   int Hq, int Hkv, int N, int NB, T* __restrict__ dx_out,
                                                   const float* __restrict__ cS, const float* __restrict__ cSz, int SL,
-                                                  int nseg) {
+                                                  int nseg, float* __restrict__ part, int U) {
   __shared__ __attribute__((aligned(16))) float st0[32 * kStRow], st1[32 * kStRow];
   __shared__ int16_t natl[kS];
   int hh = 0, ch, u;
@@ -628,13 +667,24 @@ __global__ __launch_bounds__(128, 2) void k3_fold(const T* __restrict__ x_in, co
   const SegCarry sc = seg_carry(cS, cSz, u, ch, SL, nseg);
   for (int i = tid; i < kS; i += 128) natl[i] = kSlot3.nat[i];
   __syncthreads();
-  TileRegs<128> tr;
-  load_tile<128, CARRY, MODE == 0>(S, Sz, cb, 0, wqh, natl, tr, sc);
-  store_tile<128, CARRY, MODE == 0>(st0, tr);
-  load_tile<128, CARRY, MODE == 0>(S, Sz, cb, 1, wqh, natl, tr, sc);
-  __syncthreads();
-  fold_tiles<0, CARRY, MODE == 0>(x, dx, yv, yz, st0, st1, S, Sz, cb, wqh, s, row, tr, natl, sc);
   float full[32];
+  if constexpr (SLICED) {
+    auto run = [&](auto first) {
+      constexpr int kM0 = decltype(first)::value * kSliceTiles;
+      fold_range<kM0, kM0 + kSliceTiles, CARRY, MODE == 0>(x, dx, yv, yz, st0, st1, S, Sz, cb, wqh, s, row, natl, sc);
+    };
+    if (blockIdx.y == 0) run(std::integral_constant<int, 0>{});
+    if (blockIdx.y == 1) run(std::integral_constant<int, 1>{});
+    if (blockIdx.y == 2) run(std::integral_constant<int, 2>{});
+    fold::combine_rotation_groups(dx, s, full);
+    if (ok) {
+      float4* prow = reinterpret_cast<float4*>(part + ((size_t)blockIdx.y * U * N + (size_t)u * N + tok) * kD + 32 * s);
+#pragma unroll
+      for (int a = 0; a < 8; ++a) prow[a] = make_float4(full[4 * a], full[4 * a + 1], full[4 * a + 2], full[4 * a + 3]);
+    }
+    return;
+  }
+  fold_range<0, kMT, CARRY, MODE == 0>(x, dx, yv, yz, st0, st1, S, Sz, cb, wqh, s, row, natl, sc);
   fold::combine_rotation_groups(dx, s, full);
   if (ok) {
     // local part: dq's own head (MODE 0), or the unit's heads in order (MODE 1)
@@ -652,6 +702,36 @@ __global__ __launch_bounds__(128, 2) void k3_fold(const T* __restrict__ x_in, co
     }
     fold::store32(dx_out + rowoff + 32 * s, full);
   }
+}
+
+// The sliced key side's last step: dk and dv (blockIdx.y 0 and 1) = the unit's
+// heads' local parts in head order + the slices in order. Four values a thread.
+template <typename T>
+__global__ __launch_bounds__(256) void k3_kv_sum(const float* __restrict__ dkl, const float* __restrict__ dvl,
+                                                 const float* __restrict__ part, int U, int R, int N,
+                                                 T* __restrict__ dk, T* __restrict__ dv) {
+  const size_t per_head = (size_t)N * kD, total = (size_t)U * per_head;
+  const size_t e = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
+  T* dst = blockIdx.y ? dv : dk;
+  if (!dst || e >= total) return;
+  const float* local = (blockIdx.y ? dvl : dkl) + (e / per_head) * R * per_head + e % per_head;
+  const float* p = part + (size_t)blockIdx.y * kSlices * total + e;
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto add = [&](const float* src) {
+    const float4 x = *reinterpret_cast<const float4*>(src);
+    a.x += x.x;
+    a.y += x.y;
+    a.z += x.z;
+    a.w += x.w;
+  };
+#pragma unroll
+  for (int i = 0; i < kSlices; ++i) add(p + i * total);
+#pragma unroll 4
+  for (int r = 0; r < R; ++r) add(local + (size_t)r * per_head);
+  dst[e] = from_f<T>(a.x);
+  dst[e + 1] = from_f<T>(a.y);
+  dst[e + 2] = from_f<T>(a.z);
+  dst[e + 3] = from_f<T>(a.w);
 }
 
 // ---------------------------------------------------------------------------
@@ -1145,8 +1225,42 @@ void launch_f32_readout_fwd(const LaunchGeom& g, const T* q, const float* wq, co
                             float floor, float* num, float* den, T* out, hipStream_t st, const Timer& timed) {
   timed("k3_readout", st, [&] {
     hipLaunchKernelGGL((k3_readout<T, 0>), dim3(g.R * g.NB * g.U), dim3(256), 0, st, q, wq, carry, carry_z, g.Hq,
-                       g.Hkv, g.N, g.NB, floor, num, den, out, nullptr, nullptr, nullptr, nullptr, 1, 1);
+                       g.Hkv, g.N, g.NB, floor, num, den, out, nullptr, nullptr, nullptr, nullptr, 1, 1, nullptr, g.U);
   });
+}
+
+// dk and dv from the state and the local parts. With a.kv_part (f32_sliced) the
+// two kernels run over three slices of the state's tiles side by side and
+// k3_kv_sum adds them up.
+template <typename T>
+void launch_f32_key_side(const LaunchGeom& g, const F32BwdArgs<T>& a, const float* cS, const float* cSz,
+                         hipStream_t st, const Timer& timed) {
+  const bool sliced = a.kv_part != nullptr;
+  const dim3 grid(g.NB * g.U, sliced ? kSlices : 1);
+  float* const vpart = sliced ? a.kv_part + (size_t)kSlices * g.U * g.N * kD : nullptr;
+  if (a.dk) {
+    timed("k3_fold_k", st, [&] {
+      auto* kern = sliced ? (cS ? k3_fold<T, 1, true, true> : k3_fold<T, 1, false, true>)
+                          : (cS ? k3_fold<T, 1, true> : k3_fold<T, 1, false>);
+      hipLaunchKernelGGL(kern, grid, dim3(128), 0, st, a.k, nullptr, a.v, nullptr, nullptr, a.dT, a.dTz, a.dkl, g.Hq,
+                         g.Hkv, g.N, g.NB, a.dk, cS, cSz, a.plan.SL, a.plan.S, a.kv_part, g.U);
+    });
+  }
+  if (a.dv) {
+    timed("k3_readout_v", st, [&] {
+      auto* kern = sliced ? (cS ? k3_readout<T, 1, true, true> : k3_readout<T, 1, false, true>)
+                          : (cS ? k3_readout<T, 1, true> : k3_readout<T, 1, false>);
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a.k, nullptr, a.dT, a.dTz, g.Hq, g.Hkv, g.N, g.NB, 0.f, nullptr,
+                         nullptr, nullptr, a.dvl, a.dv, cS, cSz, a.plan.SL, a.plan.S, vpart, g.U);
+    });
+  }
+  if (sliced && (a.dk || a.dv)) {
+    timed("k3_kv_sum", st, [&] {
+      const size_t quads = (size_t)g.U * g.N * kD / 4;
+      hipLaunchKernelGGL(k3_kv_sum<T>, dim3((unsigned)((quads + 255) / 256), 2), dim3(256), 0, st, a.dkl, a.dvl,
+                         a.kv_part, g.U, g.R, g.N, a.dk, a.dv);
+    });
+  }
 }
 
 // One stream (the allocation-free entry point, the profiling mode, a call
@@ -1184,23 +1298,10 @@ void launch_f32_backward_serial(const LaunchGeom& g, const F32BwdArgs<T>& a, hip
   if (a.dq) {
     timed("k3_fold_q", st, [&] {
       hipLaunchKernelGGL((k3_fold<T, 0>), dim3(g.R * g.NB * g.U), dim3(128), 0, st, a.q, a.G, nullptr, a.Gz, a.wq,
-                         a.P, a.Pz, a.dql, g.Hq, g.Hkv, g.N, g.NB, a.dq, nullptr, nullptr, 1, 1);
+                         a.P, a.Pz, a.dql, g.Hq, g.Hkv, g.N, g.NB, a.dq, nullptr, nullptr, 1, 1, nullptr, g.U);
     });
   }
-  if (a.dk) {
-    timed("k3_fold_k", st, [&] {
-      auto* kern = cS ? k3_fold<T, 1, true> : k3_fold<T, 1, false>;
-      hipLaunchKernelGGL(kern, dim3(g.NB * g.U), dim3(128), 0, st, a.k, nullptr, a.v, nullptr, nullptr,
-                         a.dT, a.dTz, a.dkl, g.Hq, g.Hkv, g.N, g.NB, a.dk, cS, cSz, a.plan.SL, a.plan.S);
-    });
-  }
-  if (a.dv) {
-    timed("k3_readout_v", st, [&] {
-      auto* kern = cS ? k3_readout<T, 1, true> : k3_readout<T, 1, false>;
-      hipLaunchKernelGGL(kern, dim3(g.NB * g.U), dim3(256), 0, st, a.k, nullptr, a.dT, a.dTz, g.Hq,
-                         g.Hkv, g.N, g.NB, 0.f, nullptr, nullptr, nullptr, a.dvl, a.dv, cS, cSz, a.plan.SL, a.plan.S);
-    });
-  }
+  launch_f32_key_side(g, a, cS, cSz, st, timed);
   if (a.coefl) {
     timed("k3_coef_reduce", st, [&] {
       hipLaunchKernelGGL(k3_coef_reduce, dim3(73, g.Hq), dim3(256), 0, st, a.coefl, g.B, g.Hq, g.NB, a.coefs);
@@ -1221,6 +1322,22 @@ void launch_f32_backward(const LaunchGeom& g, const F32BwdArgs<T>& a, hipStream_
     return;
   }
   stream_wait(aux, st);
+  // The scan is launched first: it heads the longer chain, and the host takes
+  // some 10 us over each fork and event. It also forms the state coefficient
+  // partials (its per-item products).
+  if (a.dk || a.dv || a.dwq_part) {
+    timed("k3_state_bwd", st, [&] {
+      hipLaunchKernelGGL(k3_state_bwd<T>, dim3(kFP / 64, g.U, a.plan.S), dim3(256), 0, st, a.q, a.G, a.Gz, a.wq, a.P, a.Pz,
+                         g.Hq, g.Hkv, g.N, g.NB, a.plan.SL, a.dT, a.dTz, a.segt, a.segtz, a.dwq_part);
+    });
+    if (a.plan.S > 1 && (a.dk || a.dv)) {
+      timed("k3_seg_carry", st, [&] {
+        const size_t n = (size_t)g.U * kFP * (kD + 1);
+        hipLaunchKernelGGL(k3_seg_carry, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.segt, a.segtz, g.U,
+                           a.plan.S);
+      });
+    }
+  }
   // the two orientations in separate launches: the dq part fits two blocks per
   // CU, the dk / dv / coefficient part one
   timed("k3_local_kv", aux, [&] {
@@ -1237,42 +1354,15 @@ void launch_f32_backward(const LaunchGeom& g, const F32BwdArgs<T>& a, hipStream_
   if (a.dq) {
     timed("k3_fold_q", aux, [&] {
       hipLaunchKernelGGL((k3_fold<T, 0>), dim3(g.R * g.NB * g.U), dim3(128), 0, aux, a.q, a.G, nullptr, a.Gz, a.wq,
-                         a.P, a.Pz, a.dql, g.Hq, g.Hkv, g.N, g.NB, a.dq, nullptr, nullptr, 1, 1);
+                         a.P, a.Pz, a.dql, g.Hq, g.Hkv, g.N, g.NB, a.dq, nullptr, nullptr, 1, 1, nullptr, g.U);
     });
-  }
-  // the scan also forms the state coefficient partials (its per-item products)
-  if (a.dk || a.dv || a.dwq_part) {
-    timed("k3_state_bwd", st, [&] {
-      hipLaunchKernelGGL(k3_state_bwd<T>, dim3(kFP / 64, g.U, a.plan.S), dim3(256), 0, st, a.q, a.G, a.Gz, a.wq, a.P, a.Pz,
-                         g.Hq, g.Hkv, g.N, g.NB, a.plan.SL, a.dT, a.dTz, a.segt, a.segtz, a.dwq_part);
-    });
-    if (a.plan.S > 1 && (a.dk || a.dv)) {
-      timed("k3_seg_carry", st, [&] {
-        const size_t n = (size_t)g.U * kFP * (kD + 1);
-        hipLaunchKernelGGL(k3_seg_carry, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a.segt, a.segtz, g.U,
-                           a.plan.S);
-      });
-    }
   }
   // dT holds each segment's own suffix; the dk and dv kernels add the segment
   // carries (the later segments' totals) as they stage the state
   const float* cS = a.plan.S > 1 ? a.segt : nullptr;
   const float* cSz = a.plan.S > 1 ? a.segtz : nullptr;
   if (forked) wait_event(st, ev_kv);
-  if (a.dk) {
-    timed("k3_fold_k", st, [&] {
-      auto* kern = cS ? k3_fold<T, 1, true> : k3_fold<T, 1, false>;
-      hipLaunchKernelGGL(kern, dim3(g.NB * g.U), dim3(128), 0, st, a.k, nullptr, a.v, nullptr, nullptr,
-                         a.dT, a.dTz, a.dkl, g.Hq, g.Hkv, g.N, g.NB, a.dk, cS, cSz, a.plan.SL, a.plan.S);
-    });
-  }
-  if (a.dv) {
-    timed("k3_readout_v", st, [&] {
-      auto* kern = cS ? k3_readout<T, 1, true> : k3_readout<T, 1, false>;
-      hipLaunchKernelGGL(kern, dim3(g.NB * g.U), dim3(256), 0, st, a.k, nullptr, a.dT, a.dTz, g.Hq,
-                         g.Hkv, g.N, g.NB, 0.f, nullptr, nullptr, nullptr, a.dvl, a.dv, cS, cSz, a.plan.SL, a.plan.S);
-    });
-  }
+  launch_f32_key_side(g, a, cS, cSz, st, timed);
   if (a.coefl) {
     timed("k3_coef_reduce", st, [&] {
       hipLaunchKernelGGL(k3_coef_reduce, dim3(73, g.Hq), dim3(256), 0, st, a.coefl, g.B, g.Hq, g.NB, a.coefs);

@@ -228,6 +228,20 @@ inline F32ScanPlan f32_bwd_plan(int U, int NB, int R) {
   return best;
 }
 
+// Whether the key side of the fp32 backward runs in slices. Its two kernels have
+// one block per (chunk, unit), of two and four waves, that walks the 69 tiles of
+// the state one after the other: a chain, and few blocks on short sequences. In
+// slices three blocks walk 23 tiles each and k3_kv_sum adds the parts up. The
+// whole backward on MI355X, in us, unsliced and sliced, by U * NB:
+// 48: 466, 431; 64: 512, 490; 128: 910, 806; 160: 1081, 1047; 192: 1206, 1191;
+// 256: 1528, 1566 (two units of seven heads; 8 of one head at 256: 513, 536).
+// Beyond half a block per CU the parts' traffic and the third pass cost what the
+// slices give, so the line lies under the last size with a clear gain. Three
+// shorter sums are no less exact: rel-L2 error of dk 2.6e-7 (2.7e-7 in one
+// chain), of dv 5.0e-7 (1.0e-6).
+constexpr int kF32Slices = 3;
+inline bool f32_sliced(int U, int NB) { return U * NB <= 160; }
+
 template <typename T>
 struct F32BwdArgs {
   const T *q, *k, *v;
@@ -243,6 +257,7 @@ struct F32BwdArgs {
   float *dql, *dkl, *dvl;  // local parts, [B][Hq][N][64] per query head
   float* coefl;       // local coefficient partials [B][Hq][NB][73] (nullptr: not requested)
   float* coefs;       // their per-head sums [Hq][73]
+  float* kv_part;     // f32_sliced: dk then dv parts, [2][kF32Slices][U][N][64] (else nullptr)
   T *dq, *dk, *dv;
 };
 template <typename T>

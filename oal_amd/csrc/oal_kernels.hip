@@ -699,6 +699,7 @@ struct WorkView {
   float* coefs;  // [Hq][73]
   float* segt;   // backward scan segment totals [U][S][kFP][64] (S > 1)
   float* segtz;  // [U][S][kFP]
+  float* kv_part;  // sliced key side [2][kF32Slices][U][N][64]
   size_t bytes;
 };
 
@@ -730,6 +731,9 @@ WorkView work_view(const Geometry& g, void* base, bool mma) {
   const int S = mma ? oal::f32_bwd_plan(g.U, g.NB, g.R).S : 1;
   w.segt = S > 1 ? take(sizeof(float) * (size_t)g.U * S * oal::kFP * oal::kD) : nullptr;
   w.segtz = S > 1 ? take(sizeof(float) * (size_t)g.U * S * oal::kFP) : nullptr;
+  w.kv_part = mma && oal::f32_sliced(g.U, g.NB)
+                  ? take(sizeof(float) * 2 * oal::kF32Slices * (size_t)g.U * g.N * oal::kD)
+                  : nullptr;
   w.bytes = off;
   return w;
 }
@@ -972,7 +976,7 @@ int backward_impl(const Geometry& g, const void* q, const void* k, const void* v
     oal::F32BwdArgs<T> a{qt, kt, vt, w.G, w.Gz, sv.wq, sv.carry, sv.carry_z, labels, c0, lam, gam, groups, scale,
                          w.dT, w.dTz, oal::f32_bwd_plan(g.U, g.NB, g.R), w.segt, w.segtz,
                          need_coef ? w.dwq_part : nullptr, w.dql, w.dkl, w.dvl,
-                         need_coef ? w.coefl : nullptr, w.coefs, static_cast<T*>(dq), static_cast<T*>(dk),
+                         need_coef ? w.coefl : nullptr, w.coefs, w.kv_part, static_cast<T*>(dq), static_cast<T*>(dk),
                          static_cast<T*>(dv)};
     oal::launch_f32_backward<T>(lg, a, st, aux, make_timer());
     if (need_coef) {
