@@ -731,9 +731,11 @@ WorkView work_view(const Geometry& g, void* base, bool mma) {
   const int S = mma ? oal::f32_bwd_plan(g.U, g.NB, g.R).S : 1;
   w.segt = S > 1 ? take(sizeof(float) * (size_t)g.U * S * oal::kFP * oal::kD) : nullptr;
   w.segtz = S > 1 ? take(sizeof(float) * (size_t)g.U * S * oal::kFP) : nullptr;
-  w.kv_part = mma && oal::f32_sliced(g.U, g.NB)
-                  ? take(sizeof(float) * 2 * oal::kF32Slices * (size_t)g.U * g.N * oal::kD)
-                  : nullptr;
+  // not where the slices' parts alone would put the workspace beyond the
+  // allocation-free entry point's scratch
+  const size_t part_bytes = sizeof(float) * 2 * oal::kF32Slices * (size_t)g.U * g.N * oal::kD;
+  const bool over = off <= OAL_NOALLOC_SCRATCH_BYTES && off + align_up(part_bytes) > OAL_NOALLOC_SCRATCH_BYTES;
+  w.kv_part = mma && oal::f32_sliced(g.U, g.NB) && !over ? take(part_bytes) : nullptr;
   w.bytes = off;
   return w;
 }
