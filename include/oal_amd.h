@@ -8,8 +8,8 @@
  * the caller's HIP stream and nothing is synchronized (oal_backward, and
  * oal_forward on the fp32 route, may run part of their work on a second stream
  * of the library's own, forked from and joined back to the caller's stream by
- * events, so the caller sees one stream). The library allocates no device
- * memory.
+ * events, so the caller sees one stream; short sequences stay on the caller's).
+ * The library allocates no device memory.
  *
  * Operator (reference oal_attention/grouped_reference.py:102-211):
  *   s_g(i,j)   = scale * sum_{d: labels[h][d] == g} q[i][d] * k[j][d]
@@ -50,7 +50,9 @@ extern "C" {
  * OAL_PRECISION_BF16  bf16 operands, fp32 accumulation on the gfx950 matrix cores
  *                     (MFMA) for any group count up to 64 and up to 8 query heads
  *                     per KV head (more run the fp32 kernels). Up to 8 groups the
- *                     intra-chunk term is formed from group sums; more groups --
+ *                     intra-chunk term is formed from group sums and, in both
+ *                     precisions, short sequences are evaluated over token pairs
+ *                     alone (no running state); more groups --
  *                     per-pair coefficients, labels d -> d with 64 groups -- form
  *                     the intra-chunk local score in feature form,
  *                     phi_Q . phi_K^T on the matrix cores. */
@@ -82,7 +84,8 @@ int oal_feature_stride(void);
 int oal_chunk_size(void);
 
 /* Bytes of the forward's saved state (per-chunk exclusive prefix states and
- * feature coefficients), needed by oal_backward. */
+ * feature coefficients; 256 bytes that nothing reads where the call is evaluated
+ * over token pairs), needed by oal_backward. */
 size_t oal_forward_saved_bytes(int batch, int q_heads, int kv_heads, int seq_len, int groups, int dtype,
                                int precision);
 
@@ -117,8 +120,9 @@ int oal_forward(const void* q, const void* k, const void* v,
  * gather, grouped_reference.py:89-93, routes pair (r, c), r >= c, to
  * [g(r)][g(c)] only; gradients reaching a factor L with gam = L L^T, or a
  * per-pair coefficient, are the same under both.) Invalid combinations are
- * refused before anything is enqueued. On the matrix-core paths (bf16, and fp32
- * with up to 8 groups) most of the intra-chunk VJP and of the query-side fold
+ * refused before anything is enqueued. A call that is evaluated over token pairs
+ * runs on the caller's stream alone. On the other matrix-core paths (bf16, and
+ * fp32 with up to 8 groups) most of the intra-chunk VJP and of the query-side fold
  * run on a second stream, on the bf16 group-sum path at up to 128 chunks per
  * unit with the denominator kernels (one per device, default
  * priority, created with its fork/join events on the first call; not created
@@ -179,8 +183,8 @@ int oal_selftest(int* device_errors, void* stream);
  * Same operator and layouts as oal_forward with every tensor float64: q, k, v
  * (padded to 64 features), c0 [Hq], lam [Hq][groups], gam [Hq][groups][groups]
  * (symmetric), out and num [B][Hq][N][64], den [B][Hq][N]; out = num / den, no
- * floor. Evaluated over token pairs in tiles (O(N^2) per head), for
- * validation in double precision rather than speed. No saved state: the
+ * floor. Evaluated over token pairs in tiles (O(N^2) per head), on the fp64
+ * matrix cores from group sums for up to 8 groups. No saved state: the
  * backward recomputes from q, k, v.
  */
 int oal_forward_f64(const double* q, const double* k, const double* v,
