@@ -29,8 +29,8 @@
 // labels, tiles of 32 queries x 32 keys, a block's 128 threads being 32 tokens x
 // 4 quarters, each quarter owning 16 of the 64 dimensions. Kernel time of one
 // forward and backward at B=1, Hq=14, Hkv=2, N=256 and 8 groups: 43.4 ms from
-// per-dimension sums (32.8 in k64_dkv's 16 blocks), 0.20 ms from group sums
-// (k64g_fwd 44, k64g_dq 76, k64g_dkv 75 us).
+// per-dimension sums (32.8 in k64_dkv's 16 blocks), 0.17 ms from group sums
+// (k64g_fwd 30, k64g_dq 67, k64g_dkv 53 us; at N=1024 160, 400 and 361 us).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -482,15 +482,21 @@ __global__ __launch_bounds__(256) void k64_coef_grad(const double* __restrict__ 
 // over the tile's rows: k-step r, row l % 16 of the result. So a kernel that
 // sums over keys forms the tiles transposed ([key][query]) and one that sums
 // over queries forms them straight, and no tile passes through LDS.
-// A block's four waves share one row of tiles, taken in turn (tile index mod 4),
+// A block's waves share one row of tiles, taken in turn (tile index mod waves),
 // and add their sums in wave order at the end: a fixed order whatever the
-// device does. 14 heads of 256 tokens are 224 blocks of four waves.
+// device does. 14 heads of 256 tokens are 224 blocks. Eight waves, two on a SIMD,
+// hide part of one another's latency and halve the longest row's chain; k64g_dq with eight
+// spills 128 registers and is slower (78 against 72 us). The blocks are
+// numbered with every head's longest rows first, so that the last to run are short:
+// N = 1024, 14 heads, k64g_fwd 227 to 160 us, k64g_dq 571 to 400, k64g_dkv 514 to 361
+// (head by head before).
 // ---------------------------------------------------------------------------
 namespace {
 
 constexpr int kG64 = 8;          // groups of these kernels
 constexpr int kM = 16;           // tile edge
-constexpr int kWv = 4;           // waves per block
+constexpr int kWv = 8;           // waves per block
+constexpr int kWvDq = 4;         // of k64g_dq: its coefficient sums take more than half of the registers
 constexpr int kPairs64 = kG64 * (kG64 + 1) / 2;
 constexpr int kCo = 1 + kG64 + kPairs64;  // coefficient sums: 1, s_g, s_g s_h (g >= h)
 
@@ -507,16 +513,22 @@ struct HeadTab {
   int first[kG64 + 1];                    // group g holds positions [first[g], first[g + 1])
 };
 
+// Positions by ballot: one load of the labels per block. Counted label by label they
+// were a chain of 64 dependent reads, twice, before the first tile.
 __device__ void stage_head(HeadTab& tab, const int32_t* __restrict__ labels, const double* __restrict__ c0,
                            const double* __restrict__ lam, const double* __restrict__ gam, int G, int h) {
   const int t = threadIdx.x;
-  if (t < kD) {
+  if (t < kD) {  // the first wave: one lane per dimension
     const int own = labels[h * kD + t], g = own < 0 ? 0 : (own >= G ? G - 1 : own);
-    int pos = 0;
-    for (int d = 0; d < kD; ++d) {
-      const int x = labels[h * kD + d], o = x < 0 ? 0 : (x >= G ? G - 1 : x);
-      pos += o < g || (o == g && d < t);
+    int before = 0, pos = 0;  // dimensions of lower groups; this lane's position
+#pragma unroll
+    for (int e = 0; e < kG64; ++e) {
+      const uint64_t members = __ballot(g == e);
+      if (t == 0) tab.first[e] = before;
+      if (g == e) pos = before + __popcll(members & ((1ull << t) - 1));
+      before += __popcll(members);
     }
+    if (t == 0) tab.first[kG64] = before;
     tab.perm[pos] = t;
     tab.grp[pos] = g;
   }
@@ -526,12 +538,6 @@ __device__ void stage_head(HeadTab& tab, const int32_t* __restrict__ labels, con
   }
   if (t < kG64) tab.lam[t] = t < G ? lam[(size_t)h * G + t] : 0.0;
   if (t == 0) tab.c0 = c0 ? c0[h] : 0.0;
-  __syncthreads();
-  if (t <= kG64) {
-    int n = 0;
-    for (int d = 0; d < kD; ++d) n += tab.grp[d] < t;
-    tab.first[t] = n;
-  }
   __syncthreads();
 }
 
@@ -557,6 +563,15 @@ __device__ __forceinline__ void load_rows(double (&x)[16], const double* __restr
 // loop it is 144 coefficient and 256 mask registers, which spill.
 __device__ __forceinline__ void reread() { asm volatile("" ::: "memory"); }
 
+// The W-position steps that group g's range touches, one bit each. In a scalar
+// register: the 128 + 32 tests of a tile are a bit test and a scalar branch each,
+// and not a lane mask formed, saved and restored around every product.
+template <int W>
+__device__ __forceinline__ uint32_t touched(const HeadTab& tab, int g) {
+  const int lo = __builtin_amdgcn_readfirstlane(tab.first[g]), hi = __builtin_amdgcn_readfirstlane(tab.first[g + 1]);
+  return lo < hi ? (1u << (hi + W - 1) / W) - (1u << lo / W) : 0u;
+}
+
 // s[g] = scale * sum over the group's positions of a[row] b[col].
 __device__ __forceinline__ void group_sums(d4 (&s)[kG64], const double (&a)[16], const double (&b)[16], double scale,
                                            const HeadTab& tab, int lane) {
@@ -566,11 +581,11 @@ __device__ __forceinline__ void group_sums(d4 (&s)[kG64], const double (&a)[16],
   for (int k = 0; k < 16; ++k) lab[k] = tab.grp[4 * k + (lane >> 4)];
 #pragma unroll
   for (int g = 0; g < kG64; ++g) {
-    const int lo = tab.first[g], hi = tab.first[g + 1];
+    const uint32_t steps = touched<4>(tab, g);
     d4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < 16; ++k)
-      if (lo < 4 * k + 4 && hi > 4 * k) acc = mma64(lab[k] == g ? a[k] : 0.0, b[k], acc);
+      if (steps >> k & 1) acc = mma64(lab[k] == g ? a[k] : 0.0, b[k], acc);
     s[g] = acc * scale;
   }
 }
@@ -621,11 +636,11 @@ __device__ __forceinline__ void gradient_products(d4 (&acc)[4], const d4 (&s)[kG
   }
 #pragma unroll
   for (int g = 0; g < kG64; ++g) {
-    const int lo = tab.first[g], hi = tab.first[g + 1];
+    const uint32_t blocks = touched<16>(tab, g);
     const d4 x = ds * (tab.lam[g] + 2.0 * quadratic_row(s, tab, g));
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb)
-      if (lo < 16 * cb + 16 && hi > 16 * cb) {
+      if (blocks >> cb & 1) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[cb] = mma64(x[r], lab[cb] == g ? y[cb][r] : 0.0, acc[cb]);
       }
@@ -644,7 +659,8 @@ __device__ __forceinline__ void value_products(d4 (&acc)[4], const d4& t, const 
   }
 }
 
-// The block's four accumulator sets summed in wave order through LDS; wave 0 holds the result.
+// The block's W accumulator sets summed in wave order through LDS; wave 0 holds the result.
+template <int W>
 __device__ __forceinline__ void add_waves(d4 (&acc)[4], double* red, int wave, int lane) {
   __syncthreads();
   if (wave) {
@@ -655,7 +671,7 @@ __device__ __forceinline__ void add_waves(d4 (&acc)[4], double* red, int wave, i
   }
   __syncthreads();
   if (!wave) {
-    for (int w = 0; w < kWv - 1; ++w)
+    for (int w = 0; w < W - 1; ++w)
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb)
 #pragma unroll
@@ -663,7 +679,7 @@ __device__ __forceinline__ void add_waves(d4 (&acc)[4], double* red, int wave, i
   }
 }
 
-constexpr int kRed = (kWv - 1) * 16 * 64;  // doubles of add_waves' scratch
+constexpr int red_size(int waves) { return (waves - 1) * 16 * 64; }  // doubles of add_waves' scratch
 
 }  // namespace
 
@@ -675,9 +691,10 @@ __global__ __launch_bounds__(64 * kWv) void k64g_fwd(const double* __restrict__ 
                                                      double scale, double* __restrict__ out,
                                                      double* __restrict__ num, double* __restrict__ den) {
   __shared__ HeadTab tab;
-  __shared__ double red[kRed];
+  __shared__ double red[red_size(kWv)];
   __shared__ double zred[kWv][kM];
-  const int it = blockIdx.x, bh = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int NT = (N + kM - 1) / kM, BH = gridDim.x / NT;
+  const int it = NT - 1 - blockIdx.x / BH, bh = blockIdx.x % BH, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
   stage_head(tab, labels, c0, lam, gam, G, h);
   const int tq = it * kM + (lane & 15);
@@ -703,7 +720,7 @@ __global__ __launch_bounds__(64 * kWv) void k64g_fwd(const double* __restrict__ 
   }
   z = column_sum(z);
   if (lane < kM) zred[wave][lane] = z;
-  add_waves(acc, red, wave, lane);
+  add_waves<kWv>(acc, red, wave, lane);
   if (wave) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -723,16 +740,17 @@ __global__ __launch_bounds__(64 * kWv) void k64g_fwd(const double* __restrict__ 
 
 // dq of one query tile (dq may be null) and, with part given, the tile's
 // coefficient sums part[bh][it][kCo] = sum of ds {1, s_g, s_g s_h (g >= h)}.
-__global__ __launch_bounds__(64 * kWv) void k64g_dq(const double* __restrict__ q, const double* __restrict__ k,
+__global__ __launch_bounds__(64 * kWvDq) void k64g_dq(const double* __restrict__ q, const double* __restrict__ k,
                                                     const double* __restrict__ v, const int32_t* __restrict__ labels,
                                                     const double* __restrict__ lam, const double* __restrict__ gam,
                                                     int G, int Hq, int Hkv, int N, double scale,
                                                     const double* __restrict__ Gv, const double* __restrict__ Gz,
                                                     double* __restrict__ dq, double* __restrict__ part) {
   __shared__ HeadTab tab;
-  __shared__ double red[kRed];
-  __shared__ double cred[kWv][kCo];
-  const int it = blockIdx.x, bh = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ double red[red_size(kWvDq)];
+  __shared__ double cred[kWvDq][kCo];
+  const int NT = (N + kM - 1) / kM, BH = gridDim.x / NT;
+  const int it = NT - 1 - blockIdx.x / BH, bh = blockIdx.x % BH, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
   stage_head(tab, labels, nullptr, lam, gam, G, h);
   const int tq = it * kM + (lane & 15);
@@ -746,7 +764,7 @@ __global__ __launch_bounds__(64 * kWv) void k64g_dq(const double* __restrict__ q
   double co[kCo];
 #pragma unroll
   for (int c = 0; c < kCo; ++c) co[c] = 0.0;
-  for (int jt = wave; jt <= it; jt += kWv) {
+  for (int jt = wave; jt <= it; jt += kWvDq) {
     double kr[16], vr[16];
     load_sorted(kr, ku, jt * kM, N, tab, lane);
     load_rows(vr, vu, jt * kM, N, lane);
@@ -784,11 +802,11 @@ __global__ __launch_bounds__(64 * kWv) void k64g_dq(const double* __restrict__ q
       if (lane == 0) cred[wave][c] = x;
     }
   }
-  add_waves(acc, red, wave, lane);
+  add_waves<kWvDq>(acc, red, wave, lane);
   if (part && threadIdx.x < kCo) {
     double x = 0.0;
-    for (int w = 0; w < kWv; ++w) x += cred[w][threadIdx.x];
-    part[((size_t)bh * gridDim.x + it) * kCo + threadIdx.x] = x;
+    for (int w = 0; w < kWvDq; ++w) x += cred[w][threadIdx.x];
+    part[((size_t)bh * NT + it) * kCo + threadIdx.x] = x;
   }
   if (wave || !dq) return;
 #pragma unroll
@@ -811,10 +829,10 @@ __global__ __launch_bounds__(64 * kWv) void k64g_dkv(const double* __restrict__ 
                                                      const double* __restrict__ Gz, double* __restrict__ dkh,
                                                      double* __restrict__ dvh) {
   __shared__ HeadTab tab;
-  __shared__ double red[kRed];
-  const int jt = blockIdx.x, bh = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  __shared__ double red[red_size(kWv)];
+  const int NT = (N + kM - 1) / kM, BH = gridDim.x / NT;
+  const int jt = blockIdx.x / BH, bh = blockIdx.x % BH, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
-  const int NT = gridDim.x;
   stage_head(tab, labels, c0, lam, gam, G, h);
   const int tk = jt * kM + (lane & 15);
   const double* qh = q + (size_t)bh * N * kD;
@@ -847,8 +865,8 @@ __global__ __launch_bounds__(64 * kWv) void k64g_dkv(const double* __restrict__ 
     if (dvh) value_products(av, kap, gh, it * kM, N, lane);
     if (dkh) gradient_products(ak, s, ds, qh, it * kM, N, tab, lane);
   }
-  add_waves(ak, red, wave, lane);
-  add_waves(av, red, wave, lane);
+  add_waves<kWv>(ak, red, wave, lane);
+  add_waves<kWv>(av, red, wave, lane);
   if (wave) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -924,7 +942,7 @@ void launch_f64_forward(const F64Geom& g, const double* q, const double* k, cons
                         double* num, double* den, hipStream_t st, const Timer& timed) {
   if (G <= kG64) {
     timed("k64g_fwd", st, [&] {
-      hipLaunchKernelGGL(k64g_fwd, dim3((g.N + kM - 1) / kM, g.B * g.Hq), dim3(64 * kWv), 0, st, q, k, v, labels, c0,
+      hipLaunchKernelGGL(k64g_fwd, dim3((unsigned)((g.N + kM - 1) / kM) * g.B * g.Hq), dim3(64 * kWv), 0, st, q, k, v, labels, c0,
                          lam, gam, G, g.Hq, g.Hkv, g.N, scale, out, num, den);
     });
     return;
@@ -959,10 +977,10 @@ void launch_f64_backward(const F64Geom& g, const double* q, const double* k, con
     double* dkh = take(rows * kD);
     double* dvh = take(rows * kD);
     double* part = take((size_t)g.B * g.Hq * NM * kCo);
-    const dim3 grid(NM, g.B * g.Hq), block(64 * kWv);
+    const dim3 grid((unsigned)NM * g.B * g.Hq);
     if (dq || dc0) {
       timed("k64g_dq", st, [&] {
-        hipLaunchKernelGGL(k64g_dq, grid, block, 0, st, q, k, v, labels, lam, gam, G, g.Hq, g.Hkv, g.N, scale, Gv, Gz,
+        hipLaunchKernelGGL(k64g_dq, grid, dim3(64 * kWvDq), 0, st, q, k, v, labels, lam, gam, G, g.Hq, g.Hkv, g.N, scale, Gv, Gz,
                            dq, dc0 ? part : nullptr);
       });
     }
@@ -971,7 +989,7 @@ void launch_f64_backward(const F64Geom& g, const double* q, const double* k, con
       double* dk1 = R == 1 ? dk : dk ? dkh : nullptr;
       double* dv1 = R == 1 ? dv : dv ? dvh : nullptr;
       timed("k64g_dkv", st, [&] {
-        hipLaunchKernelGGL(k64g_dkv, grid, block, 0, st, q, k, v, labels, c0, lam, gam, G, g.Hq, g.Hkv, g.N, scale,
+        hipLaunchKernelGGL(k64g_dkv, grid, dim3(64 * kWv), 0, st, q, k, v, labels, c0, lam, gam, G, g.Hq, g.Hkv, g.N, scale,
                            Gv, Gz, dk1, dv1);
       });
       if (R > 1) {

@@ -242,6 +242,14 @@ def test_group_sum_tiles_at_their_edges(n, hq, hkv, sizes):
         assert err <= 1e-11, (name, err)
 
 
+@pytest.mark.parametrize("n", [127, 128, 130, 144, 273])
+def test_group_sum_tiles_around_the_eight_wave_turn(n):
+    """The forward and key-side blocks take their tiles in a turn of eight waves:
+    eight tiles (128 tokens) with and without a remainder, a ninth, and a third
+    turn. The edge test's sums and bound; at N = 273 its 64 N terms are 2e-12."""
+    test_group_sum_tiles_at_their_edges(n, 4, 2, (3, 5, 1, 20, 16, 2, 9, 8))
+
+
 def test_partial_requests_and_reruns_are_bitwise_identical():
     from oal_amd import _native
     from oal_amd.hd_block_gemm_autograd import pad_labels
