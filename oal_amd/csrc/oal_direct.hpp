@@ -24,6 +24,10 @@ constexpr int kDirectTile = 16;  // tokens per tile edge
 // 426 / 586, N=1536 766 / 663; B=4 N=512 502 / 800, N=1024 1394 / 1202; B=64 N=256
 // 2589 / 3814. Up to 4 groups: bf16 B=1 N=1600 228 / 280, B=4 N=1024 408 / 321;
 // fp32 B=1 N=2048 629 / 769, B=4 N=1024 755 / 1171.
+// All measured with the blocks numbered head by head. Longest rows of all heads
+// first, a forward and backward take up to a quarter less (bf16 B=1 N=1024 160 to
+// 130, B=2 N=1000 256 to 219, B=16 N=256 246 to 202; fp32 B=1 N=1024 382 to 274; no
+// size slower), so the line is on the safe side for the direct route.
 inline bool direct_route(bool f32, int groups, int B, int Hq, int N) {
   if (groups > 8 || (long)B * Hq > 65535) return false;
   const double nt = (N + kDirectTile - 1) / kDirectTile, blocks = (double)B * Hq * nt, tiles = blocks * (nt + 1) / 2,
