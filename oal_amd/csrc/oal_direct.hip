@@ -46,6 +46,7 @@
 
 #include "oal_direct.hpp"
 #include "oal_internal.hpp"
+#include "oal_layout.hpp"
 #include "oal_mfma_common.hpp"
 
 namespace oal {
@@ -56,7 +57,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kM = kDirectTile;  // tile edge
 constexpr int kWv = 4;           // waves per block
-constexpr int kMore = 3;         // blocks beyond each group's first: 64 dimensions hold at most three
 
 enum Mode { kFwd, kDq, kDkv, kDk, kDv };
 
@@ -124,7 +124,7 @@ __device__ __forceinline__ void load_tile(Piece<T>& p, const T* __restrict__ bas
 template <bool F32, int GP>
 struct Lay {
   static constexpr int kWin = GP + kMore;
-  static constexpr int kPos = F32 ? 16 * kWin : kD + 3 * (GP - 1) + 16;  // the last window may start at the end
+  static constexpr int kPos = WindowWalk<F32, GP>::kPositions;
   static constexpr int LS = F32 ? kPos + 4 : (kPos + 7) / 8 * 8 + 4;
   static constexpr int LN = kD + (F32 ? 4 : 8);
   static __device__ __forceinline__ constexpr int in_block(int p) { return F32 ? 4 * (p & 3) + (p >> 2) : p; }
@@ -134,6 +134,11 @@ struct Lay {
 // have any, and in scalar registers they displace the coefficients.
 struct More {
   int group[kMore], at[kMore], count[kMore];  // group -1: none
+  __device__ __forceinline__ void put(int slot, const Window& w) {
+    group[slot] = w.group;
+    at[slot] = w.at;
+    count[slot] = w.count;
+  }
 };
 
 template <bool F32, int GP>
@@ -172,28 +177,22 @@ __device__ __forceinline__ Head<F32, GP> read_head(const int32_t* __restrict__ l
   t.lab = own < 0 ? 0 : (own >= G ? G - 1 : own);
   t.gam = x < G && y < G ? scale * scale * gv : 0.f;
   t.lam = l < G ? scale * lv : 0.f;
-  int more = 0, start = 0;
+  WindowWalk<F32, GP> walk;
   t.pos = 0;
-  if (threadIdx.x < kMore) mw.group[threadIdx.x] = -1;
+  if (threadIdx.x < kMore) mw.put(threadIdx.x, Window{});
 #pragma unroll
   for (int g = 0; g < GP; ++g) {
     const uint64_t in = __ballot(t.lab == g);
-    const int n = __popcll(in), ex = n > 16 ? (n + 15) / 16 - 1 : 0;
-    const int next = F32 ? 16 * (GP + more) : start + 16;
-    t.at[g] = F32 ? 16 * g : start;
+    const int n = __popcll(in);
+    t.at[g] = walk.first(g);
     t.count[g] = min(16, n);
     const int i = __builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in, 0));
-    const int w = i < 16 ? t.at[g] : next + (i & ~15) - 16;
+    const int w = i < 16 ? t.at[g] : walk.next() + (i & ~15) - 16;
     t.pos = t.lab == g ? w + L::in_block(i & 15) : t.pos;
-if ((int)threadIdx.x < ex) {
-      mw.group[more + threadIdx.x] = g;
-      mw.at[more + threadIdx.x] = next + 16 * (int)threadIdx.x;
-      mw.count[more + threadIdx.x] = min(16, n - 16 * ((int)threadIdx.x + 1));
-    }
-    more += ex;
-    start += (n + 3) & ~3;
+    if ((int)threadIdx.x < walk.extra(n)) mw.put(walk.more + threadIdx.x, walk.further(threadIdx.x, g, n));
+    walk.pass(n);
   }
-  t.any_more = more > 0;
+  t.any_more = walk.more > 0;
   return t;
 }
 

@@ -1,0 +1,87 @@
+"""Rules of oal_amd/csrc/oal_layout.hpp over their whole range, in a host program:
+what the kernels read by them stays inside its arrays."""
+
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oal_amd", "csrc")
+
+
+def _run(tmp_path, source):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    src, exe = tmp_path / "rule.cpp", tmp_path / "rule"
+    src.write_text(source)
+    subprocess.run([cxx, "-std=c++20", "-O1", "-Wall", "-Werror", "-I" + CSRC, str(src), "-o", str(exe)], check=True)
+    done = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stdout
+
+
+def test_every_window_slot_is_inside_the_sorted_row(tmp_path):
+    """The token-pair kernels read all kMore slots of further windows as LDS
+    positions, present or not: as a block leaves them in memory that held
+    anything, each is an aligned window inside the row, and the windows hold all
+    64 dimensions. Every size of up to three groups, and random sizes of all."""
+    _run(tmp_path, r"""
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <new>
+#include <random>
+#include <vector>
+#include "oal_layout.hpp"
+using namespace oal;
+
+template <bool F32, int GP>
+void check(const std::vector<int>& sizes) {
+  using Walk = WindowWalk<F32, GP>;
+  alignas(Window) unsigned char memory[sizeof(Window) * kMore];
+  std::memset(memory, 0x7f, sizeof memory);
+  Window* const table = reinterpret_cast<Window*>(memory);
+  int held = 0;
+  for (int x = 0; x < kMore; ++x) new (table + x) Window;  // as read_head does
+  Walk walk;
+  for (int g = 0; g < GP; ++g) {
+    const int n = g < (int)sizes.size() ? sizes[g] : 0;
+    if (walk.first(g) % 4 || walk.first(g) < 0 || walk.first(g) + 16 > Walk::kPositions) std::exit(1);
+    held += n < 16 ? n : 16;
+    if (walk.more + walk.extra(n) > kMore) std::exit(2);
+    for (int i = 0; i < walk.extra(n); ++i) table[walk.more + i] = walk.further(i, g, n);
+    walk.pass(n);
+  }
+  for (int x = 0; x < kMore; ++x) {
+    const Window& w = table[x];
+    const bool ok = w.at >= 0 && w.at % 4 == 0 && w.at + 16 <= Walk::kPositions && w.group >= -1 && w.group < GP &&
+                    (w.group < 0 ? w.count == 0 : w.count > 0 && w.count <= 16);
+    if (!ok) {
+      std::printf("F32=%d GP=%d: window %d %d %d\n", F32, GP, w.group, w.at, w.count);
+      std::exit(3);
+    }
+    held += w.count;
+  }
+  if (held != 64) std::exit(4);
+}
+void all(const std::vector<int>& sizes) {
+  if (sizes.size() <= 4) {
+    check<false, 4>(sizes);
+    check<true, 4>(sizes);
+  }
+  check<false, 8>(sizes);
+  check<true, 8>(sizes);
+}
+int main() {
+  for (int a = 0; a <= 64; ++a)
+    for (int b = 0; a + b <= 64; ++b) all({a, b, 64 - a - b});
+  std::mt19937 rng(1);
+  for (int i = 0; i < 200000; ++i) {
+    std::vector<int> sizes(1 + rng() % 8);
+    const int few = 1 + rng() % sizes.size();
+    for (int d = 0; d < 64; ++d) ++sizes[rng() % few * sizes.size() / few];
+    all(sizes);
+  }
+}
+""")
