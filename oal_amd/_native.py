@@ -621,9 +621,11 @@ class Verdict:
     set bits in; :meth:`read` synchronizes that stream. One per call: the words
     live until the kernels that may write them are done."""
 
+    _pending = False
+
     def __init__(self, device: torch.device):
-        self._pending = False
-        self._words = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+        # on the host whatever the caller's default device is
+        self._words = torch.zeros(2, dtype=torch.int32, device="cpu", pin_memory=True)
         self._stream = torch.cuda.current_stream(device)
         self._device = device
 

@@ -173,3 +173,23 @@ def test_errors_come_in_the_reference_order():
         oal_attention(q, k, v, good + 2, factor)
     with pytest.raises(RuntimeError, match="result must be finite"):
         oal_attention(q * float("inf"), k, v, good, factor)
+
+
+def test_calls_under_a_default_device():
+    """torch.device("cuda") as the caller's default moves neither the checks' host words nor any table."""
+    from oal_amd import oal_attention
+    from oal_amd.hd_block_gemm_adapters import prepare_grouped_hd_block_gemm, run_prepared_grouped_hd_block_gemm
+
+    dev = _dev()
+    q, k, v = (torch.randn(1, 2, 70, 64, device=dev) for _ in range(3))
+    factor = torch.eye(3, device=dev)[tuple(torch.tril_indices(3, 3))].expand(2, -1).contiguous()
+    labels = (torch.arange(64, device=dev) % 2).to(torch.int32)
+
+    def both():
+        prepared = prepare_grouped_hd_block_gemm(q, k, v, labels, factor, kernel_eps=1e-6, precision="bf16_tensorcore")
+        return oal_attention(q, k, v, labels, factor), run_prepared_grouped_hd_block_gemm(prepared, q, k, v, factor)[0]
+
+    want = both()
+    with torch.device("cuda"):
+        got = both()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
