@@ -37,6 +37,7 @@
 
 #include "oal_common.hpp"
 #include "oal_internal.hpp"
+#include "oal_layout.hpp"
 
 namespace oal {
 
@@ -693,8 +694,9 @@ __global__ __launch_bounds__(64 * kWv) void k64g_fwd(const double* __restrict__ 
   __shared__ HeadTab tab;
   __shared__ double red[red_size(kWv)];
   __shared__ double zred[kWv][kM];
-  const int NT = (N + kM - 1) / kM, BH = gridDim.x / NT;
-  const int it = NT - 1 - blockIdx.x / BH, bh = blockIdx.x % BH, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int NT = (N + kM - 1) / kM, it = NT - 1 - (int)tile_of(blockIdx.y, blockIdx.z, gridDim.y);
+  if (it < 0) return;
+  const int bh = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
   stage_head(tab, labels, c0, lam, gam, G, h);
   const int tq = it * kM + (lane & 15);
@@ -749,8 +751,9 @@ __global__ __launch_bounds__(64 * kWvDq) void k64g_dq(const double* __restrict__
   __shared__ HeadTab tab;
   __shared__ double red[red_size(kWvDq)];
   __shared__ double cred[kWvDq][kCo];
-  const int NT = (N + kM - 1) / kM, BH = gridDim.x / NT;
-  const int it = NT - 1 - blockIdx.x / BH, bh = blockIdx.x % BH, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int NT = (N + kM - 1) / kM, it = NT - 1 - (int)tile_of(blockIdx.y, blockIdx.z, gridDim.y);
+  if (it < 0) return;
+  const int bh = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
   stage_head(tab, labels, nullptr, lam, gam, G, h);
   const int tq = it * kM + (lane & 15);
@@ -830,8 +833,9 @@ __global__ __launch_bounds__(64 * kWv) void k64g_dkv(const double* __restrict__ 
                                                      double* __restrict__ dvh) {
   __shared__ HeadTab tab;
   __shared__ double red[red_size(kWv)];
-  const int NT = (N + kM - 1) / kM, BH = gridDim.x / NT;
-  const int jt = blockIdx.x / BH, bh = blockIdx.x % BH, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int NT = (N + kM - 1) / kM, jt = (int)tile_of(blockIdx.y, blockIdx.z, gridDim.y);
+  if (jt >= NT) return;
+  const int bh = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int b = bh / Hq, h = bh % Hq, u = b * Hkv + h / (Hq / Hkv);
   stage_head(tab, labels, c0, lam, gam, G, h);
   const int tk = jt * kM + (lane & 15);
@@ -942,8 +946,9 @@ void launch_f64_forward(const F64Geom& g, const double* q, const double* k, cons
                         double* num, double* den, hipStream_t st, const Timer& timed) {
   if (G <= kG64) {
     timed("k64g_fwd", st, [&] {
-      hipLaunchKernelGGL(k64g_fwd, dim3((unsigned)((g.N + kM - 1) / kM) * g.B * g.Hq), dim3(64 * kWv), 0, st, q, k, v, labels, c0,
-                         lam, gam, G, g.Hq, g.Hkv, g.N, scale, out, num, den);
+      const TileGrid t = tile_grid(g.B * g.Hq, (g.N + kM - 1) / kM);
+      hipLaunchKernelGGL(k64g_fwd, dim3(t.x, t.y, t.z), dim3(64 * kWv), 0, st, q, k, v, labels, c0, lam, gam, G, g.Hq,
+                         g.Hkv, g.N, scale, out, num, den);
     });
     return;
   }
@@ -977,7 +982,8 @@ void launch_f64_backward(const F64Geom& g, const double* q, const double* k, con
     double* dkh = take(rows * kD);
     double* dvh = take(rows * kD);
     double* part = take((size_t)g.B * g.Hq * NM * kCo);
-    const dim3 grid((unsigned)NM * g.B * g.Hq);
+    const TileGrid t = tile_grid(g.B * g.Hq, NM);
+    const dim3 grid(t.x, t.y, t.z);
     if (dq || dc0) {
       timed("k64g_dq", st, [&] {
         hipLaunchKernelGGL(k64g_dq, grid, dim3(64 * kWvDq), 0, st, q, k, v, labels, lam, gam, G, g.Hq, g.Hkv, g.N, scale, Gv, Gz,

@@ -35,4 +35,18 @@ struct WindowWalk {
   }
 };
 
+// Grid of kernels with one block for each of `heads` (at most 65535) and each of
+// `tiles`, the heads side by side: heads in x, tiles over y and, past its limit,
+// z. (In x alone, tiles * heads blocks of 512 threads pass the 2^32 threads that a
+// launch may have in one dimension.) Blocks with tile >= tiles have no work.
+struct TileGrid {
+  unsigned x, y, z;
+};
+constexpr unsigned kGridLimit = 65535;
+constexpr TileGrid tile_grid(unsigned heads, unsigned tiles) {
+  const unsigned z = (tiles + kGridLimit - 1) / kGridLimit;
+  return {heads, (tiles + z - 1) / z, z};
+}
+constexpr unsigned tile_of(unsigned block_y, unsigned block_z, unsigned grid_y) { return block_z * grid_y + block_y; }
+
 }  // namespace oal

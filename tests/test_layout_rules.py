@@ -85,3 +85,25 @@ int main() {
   }
 }
 """)
+
+
+def test_the_float64_group_kernels_grid_stays_inside_the_launch_limits(tmp_path):
+    """Every (batch, head) and sequence length that the float64 entry points take
+    (65535 heads, 65535 32-token tiles): each tile has one block, y and z stay under
+    65536, and no dimension reaches 2^32 threads of 512-thread blocks."""
+    _run(tmp_path, r"""
+#include <initializer_list>
+#include "oal_layout.hpp"
+using namespace oal;
+int main() {
+  for (unsigned heads : {1u, 14u, 4096u, 65535u})
+    for (unsigned tiles = 1; tiles <= 131070; tiles = tiles < 3000 ? tiles + 1 : tiles + 7) {
+      const TileGrid g = tile_grid(heads, tiles);
+      if (g.x * 512ull >= 1ull << 32 || g.x != heads || g.y > 65535 || g.z > 65535) return 1;
+      const unsigned last = tile_of(g.y - 1, g.z - 1, g.y);
+      if (last < tiles - 1 || tile_of(0, g.z - 1, g.y) >= tiles || tile_of(0, 1, g.y) != g.y) return 2;
+    }
+  const TileGrid g = tile_grid(65535, 131070);
+  return g.y * g.z < 131070;
+}
+""")
