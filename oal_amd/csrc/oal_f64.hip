@@ -930,13 +930,15 @@ __global__ __launch_bounds__(256) void k64g_coef_grad(const double* __restrict__
 // ---------------------------------------------------------------------------
 // Host launches.
 // ---------------------------------------------------------------------------
-size_t f64_workspace_bytes(int B, int Hq, int N, int G) {
+size_t f64_workspace_bytes(const F64Geom& g, int G) {
+  const int B = g.B, Hq = g.Hq, N = g.N;
   const size_t rows = (size_t)B * Hq * N;
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
   const size_t grads = al(sizeof(double) * rows * kD) + al(sizeof(double) * rows);
-  // group sums: dk and dv per query head, coefficient sums per 16-token tile
+  // group sums: dk and dv per query head where a unit has several, coefficient sums per 16-token tile
   if (G <= kG64)
-    return grads + 2 * al(sizeof(double) * rows * kD) + al(sizeof(double) * B * Hq * ((N + kM - 1) / kM) * kCo);
+    return grads + (Hq == g.Hkv ? 0 : 2 * al(sizeof(double) * rows * kD)) +
+           al(sizeof(double) * B * Hq * ((N + kM - 1) / kM) * kCo);
   const size_t NT = (size_t)(N + kT - 1) / kT;
   return grads + al(sizeof(double) * B * Hq * NT * kFP);
 }
@@ -979,8 +981,8 @@ void launch_f64_backward(const F64Geom& g, const double* q, const double* k, con
   });
   if (G <= kG64) {
     const int NM = (g.N + kM - 1) / kM, R = g.Hq / g.Hkv;
-    double* dkh = take(rows * kD);
-    double* dvh = take(rows * kD);
+    double* dkh = R > 1 ? take(rows * kD) : nullptr;
+    double* dvh = R > 1 ? take(rows * kD) : nullptr;
     double* part = take((size_t)g.B * g.Hq * NM * kCo);
     const TileGrid t = tile_grid(g.B * g.Hq, NM);
     const dim3 grid(t.x, t.y, t.z);

@@ -325,11 +325,11 @@ void launch_check_labels(const void* labels, bool wide, bool per_head, int D, in
 int launch_check_outputs(bool wide, int out_kind, const void* num, const void* den, const void* out, size_t rows,
                          int width, int num_stride, int out_stride, int* flag, hipStream_t st);
 
-// FP64 route (oal_f64.hip): pairwise evaluation over 32-token tiles.
+// FP64 route (oal_f64.hip): evaluation over token pairs, in tiles of 16 tokens up to 8 groups, of 32 beyond.
 struct F64Geom {
   int B, Hq, Hkv, N;
 };
-size_t f64_workspace_bytes(int B, int Hq, int N, int G);
+size_t f64_workspace_bytes(const F64Geom& g, int G);
 void launch_f64_forward(const F64Geom& g, const double* q, const double* k, const double* v, const int32_t* labels,
                         const double* c0, const double* lam, const double* gam, int G, double scale, double* out,
                         double* num, double* den, hipStream_t st, const Timer& timed);

@@ -1346,7 +1346,7 @@ int oal_forward_f64(const double* q, const double* k, const double* v, const int
 size_t oal_backward_f64_workspace_bytes(int batch, int q_heads, int kv_heads, int seq_len, int groups) {
   oal::F64Geom g;
   if (check_f64(groups, batch, q_heads, kv_heads, seq_len, &g)) return 0;
-  return oal::f64_workspace_bytes(g.B, g.Hq, g.N, groups);
+  return oal::f64_workspace_bytes(g, groups);
 }
 
 int oal_backward_f64(const double* q, const double* k, const double* v, const int32_t* labels, const double* c0,

@@ -174,3 +174,17 @@ def test_sliced_key_side_stays_inside_the_allocation_free_scratch():
     if not os.path.exists(_native.library_path()):
         pytest.skip("liboal_amd.so not built")
     assert _native.load_library().oal_backward_workspace_bytes(1, 26, 2, 5000, 8, 0, 0) <= 256 << 20
+
+
+@pytest.mark.parametrize("b,heads,n", [(1, 8, 1000), (3, 5, 77), (1, 1, 1)])
+def test_float64_workspace_holds_head_gradients_only_where_heads_are_summed(b, heads, n):
+    """One query head per KV head writes dk and dv to the results themselves."""
+    if not os.path.exists(_native.library_path()):
+        pytest.skip("liboal_amd.so not built")
+    size = _native.load_library().oal_backward_f64_workspace_bytes
+    per_tensor = 8 * 64 * b * heads * n
+    own = size(b, heads, heads, n, 8)
+    # G and Gz, and 45 sums per 16-token tile, each rounded up to 256 bytes
+    assert own <= per_tensor + 8 * b * heads * n + 8 * 45 * b * heads * ((n + 15) // 16) + 3 * 256
+    if heads > 1:
+        assert size(b, heads, 1, n, 8) == own + 2 * ((per_tensor + 255) // 256 * 256)
