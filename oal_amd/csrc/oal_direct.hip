@@ -820,9 +820,13 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
 // are applied once at its end. A tile's VALU work is then ds s_h alone, 36
 // multiplies and their packs a lane against about 560 instructions with the slopes
 // t_g and the 45 coefficient products formed per pair. For the coefficient sums ds
-// s_h goes in as two bf16 halves (as one, their error was 1.07 to 1.14 times as
-// large as that of fp32 sums over the pairs up to N = 256). dk likewise, with the
-// streamed q and one half; dv needs kappa, formed as in the forward (tiles).
+// s_h goes in as several bf16 parts (as one, their error was 1.07 to 1.14 times as
+// large as that of fp32 sums over the pairs up to N = 256). Three up to kC
+// tokens, where the state route sums fp32 pair values: with an upstream of den
+// alone G is zero and ds exact, and two parts gave lam's gradient 2.5e-6 where
+// those sums give 1e-7. Two beyond, where that route's state holds bf16 features
+// (1e-3). dk likewise, with the streamed q and one part; dv needs kappa, formed as
+// in the forward (tiles).
 //
 // All (GP + 1) x 4 column blocks of P are 144 registers, too many for one wave,
 // and P_h needs s_h alone: the four waves share each staged step of 64 streamed
@@ -833,17 +837,20 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
 __device__ __forceinline__ bf16x8 both(s16x4 a, s16x4 b) {
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
-// x in bf16, and with two halves also what that leaves: x to 2^-17.
+// x as a sum of bf16 parts, each what the ones before leave: x to 2^-9, 2^-17 or
+// (24 bits) 2^-25 with one, two or three.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split4(s16x4 (&h)[1], const float (&x)[4]) { h[0] = pack4(x); }
-__device__ __forceinline__ void split4(s16x4 (&h)[2], const float (&x)[4]) {
-  const u32x2 w = {pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
-  float y[4];
+template <int PARTS>
+__device__ __forceinline__ void split4(s16x4 (&h)[PARTS], const float (&x)[4]) {
+  float y[4] = {x[0], x[1], x[2], x[3]};
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
-    y[r] = x[r] - __uint_as_float(r & 1 ? w[r >> 1] & 0xffff0000u : w[r >> 1] << 16);
-  h[0] = __builtin_bit_cast(s16x4, w);
-  h[1] = pack4(y);
+  for (int p = 0; p < PARTS; ++p) {
+    const u32x2 w = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      y[r] -= __uint_as_float(r & 1 ? w[r >> 1] & 0xffff0000u : w[r >> 1] << 16);
+    h[p] = __builtin_bit_cast(s16x4, w);
+  }
 }
 
 template <int GP>
@@ -867,7 +874,7 @@ struct SharedRoles {
   float dc0[kWv];
 };
 
-template <typename T, int GP, int MODE>
+template <typename T, int GP, int MODE, int PARTS>
 __device__ __forceinline__ void roles(const Args<T, false>& a, SharedRoles<GP>& sh) {
   using L = Lay<false, GP>;
   constexpr int kOwn = GP / kWv;  // groups per wave
@@ -957,9 +964,7 @@ __device__ __forceinline__ void roles(const Args<T, false>& a, SharedRoles<GP>& 
     for (int pr = 0; pr < 2; ++pr) {
       const int ta = t0 + 2 * pr;
       if (MODE == kDk ? ta + 1 < ft || ta >= NT : ta > ft) continue;
-      // dq: both halves of ds s_h, since the coefficient sums are fp32 sums of fp32 values
-      constexpr int kHalves = MODE == kDq ? 2 : 1;
-      s16x4 xh[2][kOwn][kHalves], xl[2][kHalves];
+      s16x4 xh[2][kOwn][PARTS], xl[2][PARTS];  // of ds s_h and ds
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const int r0 = (2 * pr + e) * kM, tok = (ta + e) * kM + 4 * lg;
@@ -1014,11 +1019,11 @@ __device__ __forceinline__ void roles(const Args<T, false>& a, SharedRoles<GP>& 
 #pragma unroll
         for (int x = 0; x < kOwn; ++x)
 #pragma unroll
-          for (int f = 0; f < kHalves; ++f) P[x][cb] = mfma16(both(xh[0][x][f], xh[1][x][f]), k8, P[x][cb]);
+          for (int f = 0; f < PARTS; ++f) P[x][cb] = mfma16(both(xh[0][x][f], xh[1][x][f]), k8, P[x][cb]);
       }
       const bf16x8 kl = operand(16 * wave);
 #pragma unroll
-      for (int f = 0; f < kHalves; ++f) Pl = mfma16(both(xl[0][f], xl[1][f]), kl, Pl);
+      for (int f = 0; f < PARTS; ++f) Pl = mfma16(both(xl[0][f], xl[1][f]), kl, Pl);
     }
   }
 
@@ -1099,10 +1104,10 @@ __device__ __forceinline__ void roles(const Args<T, false>& a, SharedRoles<GP>& 
   }
 }
 
-template <typename T, int GP>
+template <typename T, int GP, int PARTS>
 __global__ __launch_bounds__(64 * kWv, 3) void direct_dq(const Args<T, false> a) {
   __shared__ __attribute__((aligned(16))) SharedRoles<GP> sh;
-  roles<T, GP, kDq>(a, sh);
+  roles<T, GP, kDq, PARTS>(a, sh);
 }
 
 // dk in the blocks of z = 0, dv in those of z = 1: side by side their chains
@@ -1115,7 +1120,7 @@ __global__ __launch_bounds__(64 * kWv, 3) void direct_dk_dv(const Args<T, false>
     Shared<false, GP> v;
   } sh;
   if (blockIdx.z == 0)
-    roles<T, GP, kDk>(a, sh.k);
+    roles<T, GP, kDk, 1>(a, sh.k);
   else
     tiles<T, false, GP, kDv>(a, sh.v);
 }
@@ -1234,7 +1239,12 @@ void backward_of(const LaunchGeom& g, const Args<T, F32>& a, const Work<F32>& w,
     if (kv)
       timed("direct_dkv", st, [&] { hipLaunchKernelGGL((direct_tiles<T, true, GP, kDkv>), grid, block, 0, st, a); });
   } else {
-    timed("direct_dq", st, [&] { hipLaunchKernelGGL((direct_dq<T, GP>), grid, block, 0, st, a); });
+    timed("direct_dq", st, [&] {
+      if (g.N <= kC)
+        hipLaunchKernelGGL((direct_dq<T, GP, 3>), grid, block, 0, st, a);
+      else
+        hipLaunchKernelGGL((direct_dq<T, GP, 2>), grid, block, 0, st, a);
+    });
     if (kv)
       timed("direct_dkv", st,
             [&] { hipLaunchKernelGGL((direct_dk_dv<T, GP>), dim3(grid.x, grid.y, 2), block, 0, st, a); });

@@ -41,7 +41,7 @@ def _rel(a, b):
     return float((a - b).norm() / b.norm())
 
 
-def _run(b, hq, hkv, n, sizes, precision, dtype, seed, floor=0.0, only=None):
+def _run(b, hq, hkv, n, sizes, precision, dtype, seed, floor=0.0, only=None, upstream=(True, True, True)):
     from oal_amd import _native
 
     dev, g = _dev(), len(sizes)
@@ -59,9 +59,10 @@ def _run(b, hq, hkv, n, sizes, precision, dtype, seed, floor=0.0, only=None):
     out, num, den, saved = _native.forward(*args, scale=scale, floor=floor, precision=precision)
     dout = torch.randn(out.shape, generator=gen).to(dtype)
     dnum, dden = torch.randn(num.shape, generator=gen), torch.randn(den.shape, generator=gen)
+    dout, dnum, dden = (t if given else None for t, given in zip((dout, dnum, dden), upstream))
     need = {**dict(need_q=True, need_k=True, need_v=True, need_coef=True), **(only or {})}
-    grads = _native.backward(*args, num, den, saved, dout.to(dev), dnum.to(dev), dden.to(dev), scale=scale, floor=floor,
-                             precision=precision, **need)
+    grads = _native.backward(*args, num, den, saved, *(t if t is None else t.to(dev) for t in (dout, dnum, dden)),
+                             scale=scale, floor=floor, precision=precision, **need)
     return (q, k, v, labels, c0, lam, gam, scale), (out, num, den), grads, (dout, dnum, dden)
 
 
@@ -126,3 +127,23 @@ def test_requests_do_not_change_results(precision):
         for i in range(6):
             assert (some[i] is not None) == (i in index)
             assert some[i] is None or torch.equal(some[i], full[i])
+
+
+@pytest.mark.parametrize("n", [1, 16, 33, 64])
+@pytest.mark.parametrize("sizes", ["one", "uneven"])
+def test_one_chunk_sums_coefficients_in_fp32(n, sizes):
+    """Up to 64 tokens in bf16 mode the coefficient sums are those of fp32 pair values.
+    With an upstream gradient of den alone every term is exact in its bf16
+    operands but for fp32 roundings: a group sum of 64 products, its product with
+    ds, the three parts' sum and the sums over pairs, a few 2^-24 each on terms
+    whose signs are random. 5e-7 is eight of them (1.3e-7 measured); two parts
+    give 2e-6 to 3e-6 for lam and 7e-7 to 2e-6 for gam."""
+    case, got, grads, up = _run(2, 4, 2, n, SIZES[sizes], "bf16", torch.bfloat16, seed=n, upstream=(False, False, True))
+    q, k, v, labels, c0, lam, gam, scale = case
+    wq = go.feature_coefficients(labels, c0.double(), lam.double(), gam.double(), scale=scale, head_dim=64)
+    _, num, den = go.chunked_forward(q.double(), k.double(), v.double(), wq, chunk=64)
+    dwq = go.chunked_backward(q.double(), k.double(), v.double(), wq, num, den, torch.zeros_like(num),
+                              torch.zeros_like(num), up[2].double())[3]
+    _, dlam, dgam = go.coefficient_gradients_from_wq(dwq, labels, lam.shape[1], scale=scale, head_dim=64)
+    assert _rel(grads[4], dlam) <= 5e-7
+    assert _rel(grads[5], go.symmetrize_gamma_gradient(dgam)) <= 5e-7
