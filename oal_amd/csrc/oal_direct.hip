@@ -330,6 +330,22 @@ __device__ __forceinline__ Blk<F32> as_operand(const f32x4& x) {
   return b;
 }
 
+// x as a sum of bf16 parts, each what the ones before leave: x to 2^-9, 2^-17 or
+// (24 bits) 2^-25 with one, two or three.
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+template <int PARTS>
+__device__ __forceinline__ void split4(s16x4 (&h)[PARTS], const float (&x)[4]) {
+  float y[4] = {x[0], x[1], x[2], x[3]};
+#pragma unroll
+  for (int p = 0; p < PARTS; ++p) {
+    const u32x2 w = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      y[r] -= __uint_as_float(r & 1 ? w[r >> 1] & 0xffff0000u : w[r >> 1] << 16);
+    h[p] = __builtin_bit_cast(s16x4, w);
+  }
+}
+
 // The whole 64-wide row as operand (ds = G . v): bf16 two 32-wide k-steps, fp32
 // sixteen, step s of lane group g being position 16 g + s.
 template <bool F32>
@@ -672,9 +688,30 @@ __device__ __forceinline__ void tiles(const Args<T, F32>& a, Shared<F32, GP>& sh
       mask(kap);
 #pragma unroll
       for (int r = 0; r < 4; ++r) z += kap[r];
-      const Blk<F32> ka = as_operand<F32>(kap);
+      if constexpr (F32) {
+        const Blk<F32> ka = as_operand<F32>(kap);
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) gacc[cb] = mma(ka, rows_operand(nat, L::LN, 16 * cb, lr, l), gacc[cb]);
+        for (int cb = 0; cb < 4; ++cb) gacc[cb] = mma(ka, rows_operand(nat, L::LN, 16 * cb, lr, l), gacc[cb]);
+      } else {
+        // kappa in two parts. One rounds it to 2^-9, on evenly scaled inputs more than the
+        // state route loses in its features' many independent roundings: at N=800, 8 groups
+        // num's error was 1.7e-3 and dv's, of an upstream of num, 2.9e-3, against the
+        // state's 1.5e-3 and 2.7e-3; in two parts 2.6e-6 and 2.3e-3 (dv's own type and
+        // G's). They cost up to 4 % of a forward (B=2, N=1000 36.8 to 38.1 us) and up to 2 %
+        // of a forward and backward (205 to 209).
+        const float y[4] = {kap[0], kap[1], kap[2], kap[3]};
+        Blk<F32> ka[2];
+        s16x4 parts[2];
+        split4(parts, y);
+        ka[0].v = parts[0];
+        ka[1].v = parts[1];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+          const Blk<F32> vb = rows_operand(nat, L::LN, 16 * cb, lr, l);
+          gacc[cb] = mma(ka[0], vb, gacc[cb]);
+          gacc[cb] = mma(ka[1], vb, gacc[cb]);
+        }
+      }
     }
     if (want_co) {
       if constexpr (MODE == kDq) {
@@ -837,22 +874,6 @@ __global__ __launch_bounds__(64 * kWv, 2) void direct_tiles(const Args<T, F32> a
 __device__ __forceinline__ bf16x8 both(s16x4 a, s16x4 b) {
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
-// x as a sum of bf16 parts, each what the ones before leave: x to 2^-9, 2^-17 or
-// (24 bits) 2^-25 with one, two or three.
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-template <int PARTS>
-__device__ __forceinline__ void split4(s16x4 (&h)[PARTS], const float (&x)[4]) {
-  float y[4] = {x[0], x[1], x[2], x[3]};
-#pragma unroll
-  for (int p = 0; p < PARTS; ++p) {
-    const u32x2 w = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      y[r] -= __uint_as_float(r & 1 ? w[r >> 1] & 0xffff0000u : w[r >> 1] << 16);
-    h[p] = __builtin_bit_cast(s16x4, w);
-  }
-}
-
 template <int GP>
 struct SharedRoles {
   using L = Lay<false, GP>;

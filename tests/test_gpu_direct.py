@@ -41,12 +41,14 @@ def _rel(a, b):
     return float((a - b).norm() / b.norm())
 
 
-def _run(b, hq, hkv, n, sizes, precision, dtype, seed, floor=0.0, only=None, upstream=(True, True, True)):
+def _run(b, hq, hkv, n, sizes, precision, dtype, seed, floor=0.0, only=None, upstream=(True, True, True),
+         exact=False):
     from oal_amd import _native
 
     dev, g = _dev(), len(sizes)
     gen = torch.Generator().manual_seed(seed)
-    q, k, v = (torch.randn((b, h, n, 64), generator=gen).to(dtype) for h in (hq, hkv, hkv))
+    rounded = (lambda t: t.bfloat16().to(t.dtype)) if exact else (lambda t: t)  # exact: operands that bf16 holds
+    q, k, v = (rounded(torch.randn((b, h, n, 64), generator=gen)).to(dtype) for h in (hq, hkv, hkv))
     lab = torch.repeat_interleave(torch.arange(g), torch.tensor(sizes)).to(torch.int32)
     labels = torch.stack([lab[torch.randperm(64, generator=gen)] for _ in range(hq)])
     low = torch.tril(torch.randn((hq, g + 1, g + 1), generator=gen) * 0.15) + torch.diag_embed(
@@ -58,7 +60,7 @@ def _run(b, hq, hkv, n, sizes, precision, dtype, seed, floor=0.0, only=None, ups
     args = [t.to(dev) for t in (q, k, v, labels, c0, lam, gam)]
     out, num, den, saved = _native.forward(*args, scale=scale, floor=floor, precision=precision)
     dout = torch.randn(out.shape, generator=gen).to(dtype)
-    dnum, dden = torch.randn(num.shape, generator=gen), torch.randn(den.shape, generator=gen)
+    dnum, dden = rounded(torch.randn(num.shape, generator=gen)), torch.randn(den.shape, generator=gen)
     dout, dnum, dden = (t if given else None for t, given in zip((dout, dnum, dden), upstream))
     need = {**dict(need_q=True, need_k=True, need_v=True, need_coef=True), **(only or {})}
     grads = _native.backward(*args, num, den, saved, *(t if t is None else t.to(dev) for t in (dout, dnum, dden)),
@@ -147,3 +149,20 @@ def test_one_chunk_sums_coefficients_in_fp32(n, sizes):
     _, dlam, dgam = go.coefficient_gradients_from_wq(dwq, labels, lam.shape[1], scale=scale, head_dim=64)
     assert _rel(grads[4], dlam) <= 5e-7
     assert _rel(grads[5], go.symmetrize_gamma_gradient(dgam)) <= 5e-7
+
+
+@pytest.mark.parametrize("n", [16, 130, 800])
+@pytest.mark.parametrize("sizes", ["uneven", "tail"])
+def test_pair_weights_keep_their_bits(n, sizes):
+    """kappa goes into num and dv in two bf16 parts. With operands that bf16 holds
+    and an upstream gradient of num alone nothing else is rounded to bf16: 2^-17 =
+    7.6e-6 of each term at most (2.6e-6 measured; in one part 1.7e-3)."""
+    case, got, grads, up = _run(1, 4, 2, n, SIZES[sizes], "bf16", torch.float32, seed=n, upstream=(False, True, False),
+                                exact=True)
+    q, k, v, labels, c0, lam, gam, scale = case
+    wq = go.feature_coefficients(labels, c0.double(), lam.double(), gam.double(), scale=scale, head_dim=64)
+    _, num, den = go.chunked_forward(q.double(), k.double(), v.double(), wq, chunk=64)
+    dv = go.chunked_backward(q.double(), k.double(), v.double(), wq, num, den, torch.zeros_like(num), up[1].double(),
+                             torch.zeros_like(den))[2]
+    assert _rel(got[1], num) <= 7.6e-6
+    assert _rel(grads[2], dv) <= 7.6e-6
