@@ -196,13 +196,28 @@ def grouped_oal_f64(q, k, v, labels, c0, lam, gam, *, scale: float):
 def logical_to_grouped(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, head_dim: int):
     """Logical (a [Hq], b [Hq, D], c [Hq, D(D+1)/2]) -> one group per dimension.
 
-    labels = d, lam = b, Gam[r][c] = Gam[c][r] = c_p(r, c) (D padded to 64).
+    labels = d, lam = b, Gam[r][c] = Gam[c][r] = c_p(r, c) (D padded to 64). One
+    kernel on the device where no gradient is asked for, as the Function below
+    calls it; torch operations, which autograd sees, otherwise.
     """
     if head_dim > HEAD_DIM:
         raise ValueError(f"the HIP kernels support head and value dimensions up to {HEAD_DIM}")
-    hq, pairs = a.shape[0], head_dim * (head_dim + 1) // 2
-    b, c = (t.to(device=a.device, dtype=torch.float32).expand(hq, n).contiguous() for t, n in ((b, head_dim), (c, pairs)))
-    lam, gam, labels = _native.expand_pairs(b, c)
+    hq, dev = a.shape[0], a.device
+    recorded = torch.is_grad_enabled() and (b.requires_grad or c.requires_grad)
+    if dev.type == "cuda" and c.device == dev and not recorded:
+        pairs = head_dim * (head_dim + 1) // 2
+        lam, gam, labels = _native.expand_pairs(
+            b.to(device=dev, dtype=torch.float32).expand(hq, head_dim).contiguous(),
+            c.to(torch.float32).expand(hq, pairs).contiguous())
+        return a.to(torch.float32).contiguous(), lam, gam, labels
+    rows, cols = torch.tril_indices(head_dim, head_dim, device=dev)
+    gam = torch.zeros((hq, HEAD_DIM, HEAD_DIM), dtype=torch.float32, device=dev)
+    cf = c.to(torch.float32)
+    gam[:, rows, cols] = cf
+    gam[:, cols, rows] = cf
+    lam = torch.zeros((hq, HEAD_DIM), dtype=torch.float32, device=dev)
+    lam[:, :head_dim] = b.to(torch.float32)
+    labels = torch.arange(HEAD_DIM, dtype=torch.int32, device=dev).unsqueeze(0).expand(hq, -1).contiguous()
     return a.to(torch.float32).contiguous(), lam, gam, labels
 
 

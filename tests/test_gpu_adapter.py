@@ -65,6 +65,12 @@ def test_pair_expansion_and_its_vjp(d):
     dgam = torch.randn((hq, 64, 64), generator=gen)
     dc = torch.where(rows == cols, dgam[:, rows, cols], dgam[:, rows, cols] + dgam[:, cols, rows])
     assert torch.equal(_native.expand_pairs_backward(dgam.to(dev), d).cpu(), dc)
+    # gradients that autograd is to record: the same values, and the same VJP
+    bg, cg = b.to(dev).requires_grad_(), c.to(dev).requires_grad_()
+    _, lam_g, gam_g, _ = logical_to_grouped(a.to(dev), bg, cg, d)
+    assert torch.equal(gam_g, gam) and torch.equal(lam_g, lam)
+    db, dcg = torch.autograd.grad((lam_g.sum(), (gam_g * dgam.to(dev)).sum()), (bg, cg))
+    assert torch.equal(dcg.cpu(), dc) and torch.equal(db.cpu(), torch.ones_like(b))
     shared = logical_to_grouped(a.to(dev), b[0].to(dev), c[:1].to(dev), d)
     assert torch.equal(shared[1][2].cpu()[:d], b[0]) and torch.equal(shared[2][2].cpu(), want[0])
 

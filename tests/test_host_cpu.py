@@ -188,3 +188,17 @@ def test_float64_workspace_holds_head_gradients_only_where_heads_are_summed(b, h
     assert own <= per_tensor + 8 * b * heads * n + 8 * 45 * b * heads * ((n + 15) // 16) + 3 * 256
     if heads > 1:
         assert size(b, heads, 1, n, 8) == own + 2 * ((per_tensor + 255) // 256 * 256)
+
+
+def test_logical_coefficients_expand_on_the_host_with_their_gradients():
+    """Pure layout: every device, and autograd reaches b and c (an off-diagonal pair has two entries)."""
+    from oal_amd.hd_block_gemm_autograd import logical_to_grouped
+
+    gen = torch.Generator().manual_seed(0)
+    a, b, c = (torch.randn(s, generator=gen, requires_grad=True) for s in ((2,), (2, 5), (2, 15)))
+    c0, lam, gam, labels = logical_to_grouped(a, b, c, 5)
+    rows, cols = torch.tril_indices(5, 5)
+    assert torch.equal(gam[:, rows, cols], c) and torch.equal(gam[:, cols, rows], c) and torch.equal(lam[:, :5], b)
+    assert not gam[:, 5:].any() and not gam[:, :, 5:].any() and not lam[:, 5:].any()
+    db, dc = torch.autograd.grad((lam.sum(), gam.sum()), (b, c))
+    assert torch.equal(db, torch.ones_like(b)) and torch.equal(dc, (1.0 + (rows != cols)).expand(2, -1))
