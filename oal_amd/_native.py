@@ -155,6 +155,26 @@ def _scope(device: torch.device, name: str | None = None):
     return stack
 
 
+_TRACERS = tuple(getattr(torch._C._TorchDispatchModeKey, name) for name in ("FAKE", "PROXY", "FUNCTIONAL"))
+
+
+def ordinary(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may stand in for a few torch operations on these tensors:
+    plain ROCm tensors in an eager call. Whatever has to see the operations -- a
+    compiler or tracer, fake tensors, a tensor subclass, functorch's transforms,
+    forward-mode derivatives -- gets them."""
+    return (
+        torch.version.hip is not None
+        and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device.type == "cuda" for t in tensors)
+        and not torch.compiler.is_compiling()
+        and not torch._C._is_tracing()
+        and not torch._C._are_functorch_transforms_active()
+        and torch.autograd.forward_ad._current_level < 0
+        and (not torch._C._len_torch_dispatch_stack()
+             or all(torch._C._get_dispatch_mode(key) is None for key in _TRACERS))
+    )
+
+
 def _aligned(t: torch.Tensor | None) -> torch.Tensor | None:
     """t, or a fresh copy when its data pointer is not 16-byte aligned (the
     kernels move rows with 16-byte accesses; a view with an odd storage offset

@@ -171,10 +171,26 @@ def _canonicalize_dim_groups(
     return dim_groups.to(torch.int32).contiguous()
 
 
-class _FactorExpansion(torch.autograd.Function):
-    """factor [P] or [Hq, P] -> (c0, lam, gam) on the device, one launch each way.
+def _expand_factor_in_torch(factor: torch.Tensor, query_heads: int, gmax: int, kernel_eps: float):
+    """The expansion of [P] or [Hq, P] or [1, P] as torch operations, in the factor's dtype."""
+    fac = factor.unsqueeze(0) if factor.ndim == 1 else factor
+    if fac.shape[0] == 1:
+        fac = fac.expand(query_heads, -1)
+    side, dtype, device = gmax + 1, factor.dtype, factor.device
+    rows, cols = torch.tril_indices(side, side, device=device)
+    flat = torch.zeros((query_heads, side * side), dtype=dtype, device=device)
+    flat = flat.scatter(1, (rows * side + cols).unsqueeze(0).expand(query_heads, -1), fac)
+    lower = flat.reshape(query_heads, side, side)
+    matrix = (lower.unsqueeze(2) * lower.unsqueeze(1)).sum(dim=-1)
+    constant = matrix[:, 0, 0] + float(kernel_eps)
+    linear = 2.0 * matrix[:, 0, 1:]
+    quadratic = matrix[:, 1:, 1:].contiguous()
+    return constant, linear, quadratic
 
-    Not twice differentiable, as the operator that its results go to is not."""
+
+class _FactorExpansion(torch.autograd.Function):
+    """factor [P] or [Hq, P] -> (c0, lam, gam) on the device, one launch each way;
+    a backward that is itself recorded goes through the torch operations."""
 
     @staticmethod
     def forward(ctx, factor, query_heads: int, gmax: int, kernel_eps: float):
@@ -184,12 +200,17 @@ class _FactorExpansion(torch.autograd.Function):
         return _native.expand_factor(factor.detach(), query_heads, gmax, kernel_eps)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, dc0, dlam, dgam):
-        if dc0 is None and dlam is None and dgam is None:
+        given = [(i, g) for i, g in enumerate((dc0, dlam, dgam)) if g is not None]
+        if not given:
             return None, None, None, None
         (factor,) = ctx.saved_tensors
-        return _native.expand_factor_backward(factor, *ctx.sizes, dc0, dlam, dgam), None, None, None
+        if torch.is_grad_enabled():
+            outs = _expand_factor_in_torch(factor, *ctx.sizes, 0.0)
+            (dfactor,) = torch.autograd.grad([outs[i] for i, _ in given], factor, [g for _, g in given], create_graph=True)
+        else:
+            dfactor = _native.expand_factor_backward(factor, *ctx.sizes, dc0, dlam, dgam)
+        return dfactor, None, None, None
 
 
 def _expand_factor_coefficients(
@@ -203,23 +224,10 @@ def _expand_factor_coefficients(
     On the device it is one kernel (oal_adapter.hip) for the group counts that
     the operator takes.
     """
-    if _on_device(factor) and gmax <= 64 and working_dtype in (torch.float32, torch.float64):
+    if _native.ordinary(factor) and gmax <= 64 and working_dtype in (torch.float32, torch.float64):
         fac = factor[0] if factor.ndim == 2 and factor.shape[0] == 1 else factor
         return _FactorExpansion.apply(fac.to(dtype=working_dtype).contiguous(), query_heads, gmax, float(kernel_eps))
-    fac = factor.unsqueeze(0) if factor.ndim == 1 else factor
-    fac = fac.to(dtype=working_dtype)
-    if fac.shape[0] == 1:
-        fac = fac.expand(query_heads, -1)
-    side = gmax + 1
-    rows, cols = torch.tril_indices(side, side, device=factor.device)
-    flat = torch.zeros((query_heads, side * side), dtype=working_dtype, device=factor.device)
-    flat = flat.scatter(1, (rows * side + cols).unsqueeze(0).expand(query_heads, -1), fac)
-    lower = flat.reshape(query_heads, side, side)
-    matrix = (lower.unsqueeze(2) * lower.unsqueeze(1)).sum(dim=-1)
-    constant = matrix[:, 0, 0] + torch.as_tensor(kernel_eps, dtype=working_dtype, device=factor.device)
-    linear = 2.0 * matrix[:, 0, 1:]
-    quadratic = matrix[:, 1:, 1:].contiguous()
-    return constant, linear, quadratic
+    return _expand_factor_in_torch(factor.to(dtype=working_dtype), query_heads, gmax, kernel_eps)
 
 
 def _validate_public_options(*, causal, execution, output_dtype, return_unnormalized):

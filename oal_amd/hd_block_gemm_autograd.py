@@ -204,7 +204,7 @@ def logical_to_grouped(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, head_d
         raise ValueError(f"the HIP kernels support head and value dimensions up to {HEAD_DIM}")
     hq, dev = a.shape[0], a.device
     recorded = torch.is_grad_enabled() and (b.requires_grad or c.requires_grad)
-    if dev.type == "cuda" and c.device == dev and not recorded:
+    if _native.ordinary(a, b, c) and c.device == dev and not recorded:
         pairs = head_dim * (head_dim + 1) // 2
         lam, gam, labels = _native.expand_pairs(
             b.to(device=dev, dtype=torch.float32).expand(hq, head_dim).contiguous(),

@@ -199,3 +199,55 @@ def test_calls_under_a_default_device():
     with torch.device("cuda"):
         got = both()
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def _expansion(groups=8, heads=2):
+    from oal_amd import grouped_quadratic as gq
+
+    gen = torch.Generator().manual_seed(groups)
+    factor = torch.randn((heads, (groups + 1) * (groups + 2) // 2), generator=gen).to(_dev())
+
+    def expand(t):
+        return gq._expand_factor_coefficients(t, query_heads=heads, gmax=groups, kernel_eps=1e-3, working_dtype=torch.float32)
+
+    return factor, expand
+
+
+def test_expansion_under_tracers():
+    """A traced expansion is the operations, not this call's result: it follows other inputs."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    factor, expand = _expansion()
+    other = factor.flip(0) + 1
+    want = expand(other)
+    graphs = [make_fx(expand, tracing_mode=mode)(factor) for mode in ("real", "fake")]
+    graphs += [torch.compile(expand, backend="eager", fullgraph=True), torch.jit.trace(expand, factor, check_trace=False)]
+    for graph in graphs:
+        for a, r in zip(graph(other), want):
+            # sums of at most 9 products in float32, where the kernel's are in float64
+            assert float((a - r).norm() / r.norm()) <= 9 * 2.0 ** -24
+
+
+def test_expansion_under_transforms():
+    """vmap, forward mode, functorch's grad and a second derivative: M = L L^T is
+    quadratic, so its derivative along L itself is twice its value, and the gradient
+    of its gradient's sum is a constant."""
+    factor, expand = _expansion()
+    c0, lam, gam = expand(factor)
+    batched = torch.func.vmap(expand)(torch.stack([factor, 2 * factor]))
+    assert torch.allclose(batched[2][0], gam, rtol=1e-5, atol=1e-5)
+    assert torch.allclose(batched[2][1], 4 * gam, rtol=1e-5, atol=1e-5)
+    _, tangent = torch.func.jvp(expand, (factor,), (factor,))
+    assert torch.allclose(tangent[2], 2 * gam, rtol=1e-5, atol=1e-5)
+    with torch.autograd.forward_ad.dual_level():
+        dual = expand(torch.autograd.forward_ad.make_dual(factor, factor))
+        assert torch.allclose(torch.autograd.forward_ad.unpack_dual(dual[1]).tangent, 2 * lam, rtol=1e-5, atol=1e-5)
+    leaf = factor.clone().requires_grad_()
+    up = [torch.randn_like(t) for t in (c0, lam, gam)]
+    first = torch.autograd.grad(expand(leaf), leaf, up)[0]
+    again = torch.autograd.grad(expand(leaf), leaf, up, create_graph=True)[0]
+    assert torch.allclose(again, first, rtol=1e-5, atol=1e-5)
+    value = torch.func.grad(lambda t: sum((o * u).sum() for o, u in zip(expand(t), up)))(factor)
+    assert torch.allclose(value, first, rtol=1e-5, atol=1e-5)
+    # the gradient is linear in the factor and its Jacobian symmetric: applied to the factor it is the gradient
+    assert torch.allclose(torch.autograd.grad(again, leaf, factor)[0], first, rtol=1e-5, atol=1e-5)

@@ -89,3 +89,25 @@ def test_make_fx_traces_the_forward():
         gm = make_fx(fwd, tracing_mode="fake")(*_fake_inputs(dv=48))
     targets = [str(n.target) for n in gm.graph.nodes if n.op == "call_function"]
     assert "oal_amd.forward.default" in targets
+
+
+def test_make_fx_traces_the_factor_expansion():
+    """Code above the operators expands a factor or per-pair coefficients in the
+    traced function: the graph holds that expansion, on fake tensors as on real ones."""
+    from oal_amd.grouped_quadratic import _expand_factor_coefficients
+    from oal_amd.hd_block_gemm_autograd import logical_to_grouped
+
+    _lib_or_skip()
+
+    def fwd(q, k, v, labels, factor, a, b, c):
+        coef = _expand_factor_coefficients(factor, query_heads=14, gmax=8, kernel_eps=1e-6, working_dtype=torch.float32)
+        kw = dict(scale=0.125, floor=0.0, precision="bf16")
+        c0, lam, gam, each = logical_to_grouped(a, b, c, 64)
+        return ops.grouped_oal_op(q, k, v, labels, *coef, **kw)[0], ops.grouped_oal_op(q, k, v, each, c0, lam, gam, **kw)[0]
+
+    with FakeTensorMode():
+        q, k, v, labels, *_ = _fake_inputs()
+        small = [torch.empty(s, device="cuda") for s in ((14, 45), (14,), (14, 64), (14, 2080))]
+        gm = make_fx(fwd, tracing_mode="fake")(q, k, v, labels, *small)
+    inputs = [n for n in gm.graph.nodes if n.op == "placeholder"]
+    assert all(n.users for n in inputs)  # none baked in
