@@ -155,24 +155,24 @@ def _scope(device: torch.device, name: str | None = None):
     return stack
 
 
-_TRACERS = tuple(getattr(torch._C._TorchDispatchModeKey, name) for name in ("FAKE", "PROXY", "FUNCTIONAL"))
+_C = torch._C
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+_TRACERS = tuple(getattr(_C._TorchDispatchModeKey, name) for name in ("FAKE", "PROXY", "FUNCTIONAL"))
 
 
 def ordinary(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may stand in for a few torch operations on these tensors:
     plain ROCm tensors in an eager call. Whatever has to see the operations -- a
     compiler or tracer, fake tensors, a tensor subclass, functorch's transforms,
-    forward-mode derivatives -- gets them."""
-    return (
-        torch.version.hip is not None
-        and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device.type == "cuda" for t in tensors)
-        and not torch.compiler.is_compiling()
-        and not torch._C._is_tracing()
-        and not torch._C._are_functorch_transforms_active()
-        and torch.autograd.forward_ad._current_level < 0
-        and (not torch._C._len_torch_dispatch_stack()
-             or all(torch._C._get_dispatch_mode(key) is None for key in _TRACERS))
-    )
+    forward-mode derivatives -- gets them. (Under 1 us: it is asked in every call.)"""
+    for t in tensors:
+        if type(t) not in _PLAIN_TYPES or not t.is_cuda:
+            return False
+    if (torch.compiler.is_compiling() or _C._is_tracing() or _C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    tracing = _C._len_torch_dispatch_stack() and any(_C._get_dispatch_mode(key) is not None for key in _TRACERS)
+    return torch.version.hip is not None and not tracing
 
 
 def _aligned(t: torch.Tensor | None) -> torch.Tensor | None:
