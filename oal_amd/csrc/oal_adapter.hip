@@ -75,50 +75,55 @@ __global__ __launch_bounds__(kThreads) void k_expand_factor(const T* __restrict_
   }
 }
 
-// dL_im = sum_{j >= m} (dM_ij + dM_ji) L_jm; a shared factor's gradient is the
-// sum over the heads in order, in one block. Any of dc0, dlam, dgam may be null.
+// dL_im = sum_{j >= m} S_ij L_jm with S = dM + dM^T, a shared factor's S being the
+// sum over the heads: its L is the same for all of them, so the product is formed
+// once. With per_head a block takes a head's whole factor; a shared factor has a
+// block for each row i, whose threads share the heads of the row's entries out and
+// add them up in a fixed order. Expansion and VJP of 64 heads of 64 groups, with the
+// host: 52 us; 3725 with all heads' products in one block, 437 as torch operations (256
+// heads of 22 groups 53, 1356, 356). Any of dc0, dlam, dgam may be null. Sums in fp64.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void k_expand_factor_bwd(const T* __restrict__ factor, bool per_head, int Hq,
                                                                 int G, const T* __restrict__ dc0,
                                                                 const T* __restrict__ dlam,
                                                                 const T* __restrict__ dgam, T* __restrict__ dfactor) {
   __shared__ T L[kPackMax];
-  __shared__ T S[kSideMax * kSideMax];
+  __shared__ double S[kSideMax * kSideMax];
+  static_assert(kSideMax * kSideMax >= kThreads, "the heads' parts of one row fit");
   const int side = G + 1, P = side * (side + 1) / 2;
-  const int first = per_head ? blockIdx.x : 0, last = per_head ? blockIdx.x + 1 : Hq;
-  for (int x = threadIdx.x; x < P; x += kThreads) L[x] = factor[(per_head ? (size_t)first * P : 0) + x];
-  constexpr int kOwn = (kPackMax + kThreads - 1) / kThreads;  // entries per thread, at most
-  double sum[kOwn] = {};
-  for (int h = first; h < last; ++h) {
-    __syncthreads();
-    for (int x = threadIdx.x; x < side * side; x += kThreads) {
-      const int i = x / side, j = x % side;
-      T s = 0;
-      if (x == 0)
-        s = dc0 ? 2 * dc0[h] : T(0);
+  const int first = per_head ? blockIdx.x : 0, heads = per_head ? 1 : Hq;
+  const int row0 = per_head ? 0 : blockIdx.x, rows = per_head ? side : 1;
+  for (int x = threadIdx.x; x < P; x += kThreads) L[x] = factor[(size_t)first * P + x];
+  const int n = rows * side, parts = max(1, min(heads, kThreads / n));
+  for (int y = threadIdx.x; y < n * parts; y += kThreads) {
+    const int i = row0 + y % n / side, j = y % side;
+    double s = 0;
+#pragma unroll 4
+    for (int e = y / n; e < heads; e += parts) {
+      const size_t h = first + e;
+      if (i == 0 && j == 0)
+        s += dc0 ? 2 * (double)dc0[h] : 0.0;
       else if (i == 0 || j == 0)
-        s = dlam ? 2 * dlam[(size_t)h * G + i + j - 1] : T(0);
+        s += dlam ? 2 * (double)dlam[h * G + i + j - 1] : 0.0;
       else if (dgam)
-        s = dgam[((size_t)h * G + i - 1) * G + j - 1] + dgam[((size_t)h * G + j - 1) * G + i - 1];
-      S[x] = s;
+        s += (double)dgam[(h * G + i - 1) * G + j - 1] + dgam[(h * G + j - 1) * G + i - 1];
     }
-    __syncthreads();
-#pragma unroll
-    for (int n = 0; n < kOwn; ++n) {
-      const int x = threadIdx.x + n * kThreads;
-      if (x >= P) break;
-      int i = 0;
-      while (packed(i + 1, 0) <= x) ++i;
-      const int m = x - packed(i, 0);
-      double acc = 0;
-      for (int j = m; j < side; ++j) acc += (double)S[i * side + j] * L[packed(j, m)];
-      sum[n] += acc;
-    }
+    S[y] = s;
   }
-#pragma unroll
-  for (int n = 0; n < kOwn; ++n) {
-    const int x = threadIdx.x + n * kThreads;
-    if (x < P) dfactor[(size_t)first * (per_head ? P : 0) + x] = (T)sum[n];
+  __syncthreads();
+  if (parts > 1) {
+    if (threadIdx.x < n)
+      for (int p = 1; p < parts; ++p) S[threadIdx.x] += S[p * n + threadIdx.x];
+    __syncthreads();
+  }
+  const int begin = packed(row0, 0), count = packed(row0 + rows, 0) - begin;
+  for (int x = threadIdx.x; x < count; x += kThreads) {
+    int i = row0;
+    while (packed(i + 1, 0) <= begin + x) ++i;
+    const int m = begin + x - packed(i, 0);
+    double acc = 0;
+    for (int j = m; j < side; ++j) acc += S[(i - row0) * side + j] * L[packed(j, m)];
+    dfactor[(size_t)first * P + begin + x] = (T)acc;
   }
 }
 
@@ -310,8 +315,8 @@ void launch_expand_factor(const T* factor, bool per_head, int Hq, int G, double 
 template <typename T>
 void launch_expand_factor_bwd(const T* factor, bool per_head, int Hq, int G, const T* dc0, const T* dlam,
                               const T* dgam, T* dfactor, hipStream_t st) {
-  hipLaunchKernelGGL(k_expand_factor_bwd<T>, dim3(per_head ? Hq : 1), dim3(kThreads), 0, st, factor, per_head, Hq, G,
-                     dc0, dlam, dgam, dfactor);
+  hipLaunchKernelGGL(k_expand_factor_bwd<T>, dim3(per_head ? Hq : G + 1), dim3(kThreads), 0, st, factor, per_head, Hq,
+                     G, dc0, dlam, dgam, dfactor);
 }
 template void launch_expand_factor<float>(const float*, bool, int, int, double, float*, float*, float*, hipStream_t);
 template void launch_expand_factor<double>(const double*, bool, int, int, double, double*, double*, double*, hipStream_t);

@@ -45,6 +45,30 @@ def test_factor_expansion_and_its_vjp(dtype, tol, groups, shared):
         assert float((da[0].cpu().double() - dr[0]).norm() / dr[0].norm()) <= tol, used
 
 
+@pytest.mark.parametrize("groups", [1, 8, 22, 64])
+@pytest.mark.parametrize("heads", [1, 2, 5, 130])
+def test_shared_factor_gradient_over_heads(groups, heads):
+    """One factor for all heads: the threads of a row share its heads out (256 / (groups
+    + 1) parts at most: more than the heads, and with and without a remainder of
+    them). Sums in fp64 of fp32 gradients, rounded once: 2^-24, and each product's
+    operands are exact."""
+    from oal_amd import _native
+
+    dev, side = _dev(), groups + 1
+    gen = torch.Generator().manual_seed(groups + heads)
+    packed = torch.randn(side * (side + 1) // 2, generator=gen)
+    up = [torch.randn(s, generator=gen) for s in ((heads,), (heads, groups), (heads, groups, groups))]
+    got = _native.expand_factor_backward(packed.to(dev), heads, groups, *(t.to(dev) for t in up))
+    rows, cols = torch.tril_indices(side, side)
+    low = torch.zeros(side, side, dtype=torch.float64)
+    low[rows, cols] = packed.double()
+    dm = torch.zeros(heads, side, side, dtype=torch.float64)
+    dm[:, 0, 0], dm[:, 0, 1:], dm[:, 1:, 1:] = up[0].double(), 2 * up[1].double(), up[2].double()
+    want = ((dm + dm.transpose(1, 2)).sum(0) @ low)[rows, cols]
+    # rounded to float32 once: half a unit in the last place
+    assert float((got.cpu().double() - want).norm() / want.norm()) <= 2.0 ** -24
+
+
 @pytest.mark.parametrize("d", [1, 5, 48, 64])
 def test_pair_expansion_and_its_vjp(d):
     """Copies and sums of two values: the same bits as the indexed assignment."""
