@@ -33,6 +33,13 @@ inline bool direct_route(bool f32, int groups, int B, int Hq, int N) {
   const double nt = (N + kDirectTile - 1) / kDirectTile, blocks = (double)B * Hq * nt, tiles = blocks * (nt + 1) / 2,
                rows = (double)B * Hq * N;
   const bool few = groups <= 4;
+  // One or two heads: the time is the longest row's chain, 61 ns a token and direction
+  // (50 up to 4 groups) against the state's 21, which the terms below do not hold. One
+  // head, 8 groups: N=3000 197 / 232, N=3600 237 / 245, N=3900 253 / 249, N=4390 285 /
+  // 262; without gradients of the coefficients N=4416 273 / 248; two heads of one
+  // unit N=3392 239 / 234. Up to 4 groups: N=4400 231 / 261, N=5000 270 / 277, without
+  // coefficients N=5088 266 / 260.
+  if (!f32 && N > (few ? 4500 : 3200)) return false;
   if (f32) return 60 + 0.03 * N + (few ? 0.0042 : 0.0082) * tiles + (few ? 0.06 : 0.085) * blocks < 420 + 0.0145 * rows;
   return 35 + 0.02 * N + (few ? 0.0018 : 0.0027) * tiles + (few ? 0.05 : 0.055) * blocks < 230 + 0.0028 * rows;
 }

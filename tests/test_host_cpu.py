@@ -202,3 +202,18 @@ def test_logical_coefficients_expand_on_the_host_with_their_gradients():
     assert not gam[:, 5:].any() and not gam[:, :, 5:].any() and not lam[:, 5:].any()
     db, dc = torch.autograd.grad((lam.sum(), gam.sum()), (b, c))
     assert torch.equal(db, torch.ones_like(b)) and torch.equal(dc, (1.0 + (rows != cols)).expand(2, -1))
+
+
+def test_long_rows_of_few_heads_take_the_state_route_in_bf16():
+    """Beyond these lengths one head's longest row takes longer over its pairs than the state route does."""
+    if not os.path.exists(_native.library_path()):
+        pytest.skip("liboal_amd.so not built")
+    size = _native.load_library().oal_forward_saved_bytes
+    bf16, fp32 = (1, 1), (0, 0)  # type and precision codes
+
+    def direct(heads, n, groups, codes):
+        return size(1, heads, 1, n, groups, *codes) <= 256
+
+    assert direct(1, 3200, 8, bf16) and not direct(1, 3300, 8, bf16) and not direct(2, 3300, 8, bf16)
+    assert direct(1, 4500, 4, bf16) and not direct(1, 4600, 4, bf16)
+    assert direct(1, 4100, 8, fp32) and direct(1, 5500, 4, fp32)
