@@ -1,7 +1,8 @@
 """Run-to-run determinism: two identical fwd+bwd calls give bitwise-identical
 outputs and gradients, on the fp32 route (oal_attention's "triton"/"auto" and
 "reference" executions) and on the bf16 matrix-core route, for 8 groups (the
-group-sum intra-chunk kernels), 12 groups and 64 groups (per-pair
+direct route's token pairs, and at 1700 tokens the state with the group-sum
+intra-chunk kernels), 12 groups and 64 groups (per-pair
 coefficients; the fp32 route's scalar kernels, the bf16 route's feature-form
 local kernels and their per-head dk partials). Every reduction in the library
 has a fixed order (partial buffers summed in order, no atomics; the fp32
@@ -11,6 +12,7 @@ import pytest
 import torch
 
 from oracle import grouped_oracle as go
+from routes import takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -49,6 +51,7 @@ def _inputs(gcount, n, seed):
 
 @pytest.mark.parametrize("precision,dtype,n,gcount", [
     ("fp32", torch.float32, 777, 8), ("fp32", torch.bfloat16, 320, 8), ("bf16", torch.bfloat16, 1000, 8),
+    ("fp32", torch.float32, 1700, 8), ("fp32", torch.bfloat16, 1700, 8), ("bf16", torch.bfloat16, 1700, 8),
     ("fp32", torch.float32, 450, 12), ("bf16", torch.bfloat16, 450, 12),
     ("fp32", torch.float32, 300, 64), ("bf16", torch.bfloat16, 520, 64),
 ])
@@ -56,6 +59,7 @@ def test_two_runs_are_bitwise_identical(precision, dtype, n, gcount):
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     dev = _dev()
+    assert takes_state(1, 14, 2, n, gcount, precision, dtype) == (gcount > 8 or n >= 1700)
     inp = _inputs(gcount, n, seed=17)
     print(f"determinism: precision={precision} dtype={dtype} N={n} groups={gcount}", flush=True)
 

@@ -1,4 +1,5 @@
-"""Edge shapes of the bf16 matrix-core path against the fp32 oracle (GPU).
+"""Edge shapes of bf16 mode against the fp32 oracle (GPU), short ones over token
+pairs, and the same head layouts past the direct route's line, through the state.
 
 * sequence lengths at chunk boundaries: N = 1 (one token, one chunk, one scan
   segment), 63, 64, 65 (a one-token last chunk);
@@ -17,6 +18,7 @@ import pytest
 import torch
 
 from oracle import grouped_oracle as go
+from routes import past_the_line, takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -99,10 +101,17 @@ def test_sequence_lengths_at_chunk_boundaries(n):
 
 @pytest.mark.parametrize("hq,hkv", [(2, 2), (6, 2), (4, 1), (10, 2), (12, 2), (16, 2), (18, 2)])
 def test_heads_per_kv_head(hq, hkv):
+    """1 to 9 query heads per KV head over token pairs, in fp32 arithmetic for 9."""
+    assert not takes_state(1, hq, hkv, 130, 4, "bf16")
+    _run(1, hq, hkv, 130, _labels(hq, 4), seed=hq)
+
+
+@pytest.mark.parametrize("hq,hkv", [(2, 2), (6, 2), (4, 1), (10, 2), (12, 2), (16, 2), (18, 2)])
+def test_heads_per_kv_head_through_the_state(hq, hkv):
     """1 to 9 query heads per KV head: the shared-copy readout for 1 to 7 (one
     readout wave per head plus the copy wave), per-head readout blocks for 8, the
     fp32 kernels for 9."""
-    _run(1, hq, hkv, 130, _labels(hq, 4), seed=hq)
+    _run(1, hq, hkv, past_the_line(1, hq, hkv, 8, "bf16"), _labels(hq, 8), seed=hq)
 
 
 def test_single_group_and_empty_groups():
@@ -151,11 +160,19 @@ def test_partial_gradient_requests(grads):
 
 @pytest.mark.parametrize("b,hq,hkv,n", [(3, 6, 3, 1000), (1, 7, 1, 777), (5, 4, 2, 200), (1, 2, 1, 4165)])
 def test_irregular_shapes(b, hq, hkv, n):
+    """Unit counts B * Hkv = 9, 1, 10, N not a multiple of any tile, 2 to 7 query heads
+    per KV head, over token pairs. N = 4165, through the state, is 66 chunks: the
+    denominator prefix scans take a full 64-chunk tile, then a tile of two."""
+    assert takes_state(b, hq, hkv, n, 6, "bf16") == (n > 4096)
+    _run(b, hq, hkv, n, _labels(hq, 6, seed=n), seed=b + n)
+
+
+@pytest.mark.parametrize("b,hq,hkv", [(3, 6, 3), (1, 7, 1), (5, 4, 2)])
+def test_irregular_shapes_through_the_state(b, hq, hkv):
     """Unit counts B * Hkv = 9, 1, 10 (the XCD-ordered block mappings fall back to
     plain order when the block count is not a multiple of 8), N not a multiple of
-    the 64-token chunk, 2 to 7 query heads per KV head, and scan plans whose
-    segments do not divide the chunk count. N = 4165 is 66 chunks: the
-    denominator prefix scans take a full 64-chunk tile, then a tile of two."""
+    the 64-token chunk, and scan plans whose segments do not divide the chunk count."""
+    n = past_the_line(b, hq, hkv, 6, "bf16")
     _run(b, hq, hkv, n, _labels(hq, 6, seed=n), seed=b + n)
 
 

@@ -1,4 +1,5 @@
-"""The normalization floor on the GPU, both routes, against the oracle.
+"""The normalization floor on the GPU, in both precisions, over token pairs (512
+tokens) and through the state (1700), against the oracle.
 
 out = num / max(den, floor), and the VJP masks the output-gradient part of the
 denominator gradient where den < floor (reference
@@ -14,6 +15,7 @@ import pytest
 import torch
 
 from oracle import grouped_oracle as go
+from routes import takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -33,12 +35,14 @@ def rel(a, b):
 
 
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
-def test_floor_forward_and_backward_match_oracle(precision):
+@pytest.mark.parametrize("n,state", [(512, False), (1700, True)])
+def test_floor_forward_and_backward_match_oracle(precision, n, state):
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     dev = _dev()
     gen = torch.Generator().manual_seed(21)
-    b, hq, hkv, n, g = 1, 14, 2, 512, 8
+    b, hq, hkv, g = 1, 14, 2, 8
+    assert takes_state(b, hq, hkv, n, g, precision) == state
     q = torch.randn((b, hq, n, 64), generator=gen) * 0.5
     k = torch.randn((b, hkv, n, 64), generator=gen) * 0.5
     v = torch.randn((b, hkv, n, 64), generator=gen)

@@ -3,13 +3,15 @@ and replayed: the backward's second-stream fork and join (the intra-chunk VJP
 and the query-side fold on the second stream, events before the key-side fold
 and the reductions, the final join) are captured as event dependencies. Each
 replay follows other eager work and a synchronization, and must reproduce the
-eager results bitwise."""
+eager results bitwise. Short sequences (the direct route) have one stream to
+capture."""
 
 import pytest
 import torch
 
 from oal_amd import _native
 from oracle import grouped_oracle as go
+from routes import takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -21,10 +23,12 @@ def _dev():
 
 
 @pytest.mark.parametrize("precision", ["bf16", "fp32"])
-def test_captured_forward_backward_replays_match_eager(precision):
+@pytest.mark.parametrize("n,state", [(640, False), (1700, True)])
+def test_captured_forward_backward_replays_match_eager(precision, n, state):
     dev = _dev()
+    assert takes_state(1, 14, 2, n, 8, precision) == state
     gen = torch.Generator().manual_seed(41)
-    b, hq, hkv, n, g = 1, 14, 2, 640, 8
+    b, hq, hkv, g = 1, 14, 2, 8
     dt = torch.bfloat16
     q = (torch.randn(b, hq, n, 64, generator=gen) * 0.5).to(dt).to(dev)
     k = (torch.randn(b, hkv, n, 64, generator=gen) * 0.5).to(dt).to(dev)

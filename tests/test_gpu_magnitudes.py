@@ -1,4 +1,5 @@
-"""Operand magnitudes far from 1 on the bf16 matrix-core route, against the oracle.
+"""Operand magnitudes far from 1 in bf16 mode, against the oracle: over token pairs
+(512 tokens) and through the state (1500).
 
 The route rounds its chunk states, features and operands to bf16 and
 accumulates in fp32. These cases put the states, the query rows and the
@@ -13,6 +14,7 @@ import pytest
 import torch
 
 from oracle import grouped_oracle as go
+from routes import takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -45,13 +47,15 @@ def rel(a, b):
 
 
 @pytest.mark.parametrize("case", sorted(CASES))
-def test_scaled_operands_match_oracle(case):
+@pytest.mark.parametrize("n,state", [(512, False), (1500, True)])
+def test_scaled_operands_match_oracle(case, n, state):
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     mq, mk, mv, mf = CASES[case]
     dev = _dev()
     gen = torch.Generator().manual_seed(31)
-    b, hq, hkv, n, g = 1, 14, 2, 512, 8
+    b, hq, hkv, g = 1, 14, 2, 8
+    assert takes_state(b, hq, hkv, n, g, "bf16") == state
     q = (torch.randn((b, hq, n, 64), generator=gen) * 0.5 * mq).to(torch.bfloat16)
     k = (torch.randn((b, hkv, n, 64), generator=gen) * 0.5 * mk).to(torch.bfloat16)
     v = (torch.randn((b, hkv, n, 64), generator=gen) * mv).to(torch.bfloat16)

@@ -11,6 +11,7 @@ import pytest
 import torch
 
 from oracle import grouped_oracle as go
+from routes import past_the_line, takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -90,11 +91,14 @@ def test_reference_golden_fixtures_through_oal_attention(name):
 
 
 @pytest.mark.parametrize("upstream", ["dout", "dout_dnum_dden"])
-def test_fp32_forward_backward_ragged_gqa_matches_oracle(upstream):
+@pytest.mark.parametrize("state", [False, True])
+def test_fp32_forward_backward_ragged_gqa_matches_oracle(upstream, state):
+    """150 tokens over token pairs; the first ragged length that goes through the state."""
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     dev = _dev()
-    q, k, v, labels, c0, lam, gam = _random_grouped(2, 4, 2, 150, 3, seed=11)
+    n = past_the_line(2, 4, 2, 3, "fp32", torch.float32) if state else 150
+    q, k, v, labels, c0, lam, gam = _random_grouped(2, 4, 2, n, 3, seed=11)
     scale = 0.125
     qg, kg, vg = (t.to(dev).requires_grad_() for t in (q, k, v))
     c0g, lamg, gamg = (t.to(dev).requires_grad_() for t in (c0, lam, gam))
@@ -118,18 +122,20 @@ def test_fp32_forward_backward_ragged_gqa_matches_oracle(upstream):
         assert rel(got, want) <= FP32_TOL, (rel(got, want), got.shape)
 
 
-def test_fp32_state_scan_segments_match_oracle():
+@pytest.mark.parametrize("n", [1080, 2860])
+def test_fp32_state_scan_segments_match_oracle(n):
     """The fp32 route's backward state scan walks its chunks in segments when a
     geometry has few (feature slice, unit) blocks for a long chunk walk: at B=1,
-    Hq=8, Hkv=1, N=1080 (17 chunks, the last one ragged) it runs 9 segments of 2
-    chunks (the last of 1), then turns the segment totals into carries and adds
-    each chunk's carry. Outputs and every gradient must match the oracle to the
+    Hq=8, Hkv=1, N=2860 (45 chunks, the last one ragged) it runs 23 segments of 2
+    chunks (the last of 1), then turns the segment totals into carries and adds each
+    chunk's carry (1080 tokens go over token pairs). Outputs and every gradient must match the oracle to the
     fp32 bar, the coefficient gradients (formed from the per-item products inside
     the segments) included."""
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     dev = _dev()
-    q, k, v, labels, c0, lam, gam = _random_grouped(1, 8, 1, 1080, 4, seed=21)
+    assert takes_state(1, 8, 1, n, 4, "fp32", torch.float32) == (n == 2860)
+    q, k, v, labels, c0, lam, gam = _random_grouped(1, 8, 1, n, 4, seed=21)
     scale = 0.125
     qg, kg, vg = (t.to(dev).requires_grad_() for t in (q, k, v))
     c0g, lamg, gamg = (t.to(dev).requires_grad_() for t in (c0, lam, gam))
@@ -318,11 +324,13 @@ def test_matrix_core_layout_selftest():
     assert _native.selftest() == 0
 
 
-@pytest.mark.parametrize("n", [256, 200, 1024])
+@pytest.mark.parametrize("n", [256, 200, 1024, 1500])
 def test_bf16_matrix_core_forward_matches_fp32_oracle(n):
+    """1500 tokens go through the state, the shorter ones over token pairs."""
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     dev = _dev()
+    assert takes_state(1, 14, 2, n, 8, "bf16") == (n == 1500)
     inp = _bf16_case(1, n, seed=4)
     qb, kb, vb = (inp[nm].to(torch.bfloat16) for nm in ("q", "k", "v"))
     args = [t.to(dev) for t in (qb, kb, vb)] + [inp[nm].to(dev) for nm in ("groups", "c0", "lam", "gam")]
@@ -337,11 +345,14 @@ def test_bf16_matrix_core_forward_matches_fp32_oracle(n):
     assert e_num <= BF16_TOL and e_den <= BF16_TOL and e_out <= BF16_TOL
 
 
-@pytest.mark.parametrize("batch,n,upstream", [(1, 256, "dnum_dden"), (2, 200, "dout"), (1, 1024, "dout")])
+@pytest.mark.parametrize("batch,n,upstream", [(1, 256, "dnum_dden"), (2, 200, "dout"), (1, 1024, "dout"),
+                                              (1, 1500, "dnum_dden"), (1, 1500, "dout")])
 def test_bf16_matrix_core_backward_matches_fp32_oracle(batch, n, upstream):
+    """1500 tokens go through the state, the shorter ones over token pairs."""
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     dev = _dev()
+    assert takes_state(batch, 14, 2, n, 8, "bf16") == (n == 1500)
     inp = _bf16_case(batch, n, seed=6)
     qb, kb, vb = (inp[nm].to(torch.bfloat16).to(dev).requires_grad_() for nm in ("q", "k", "v"))
     c0, lam, gam = (inp[nm].to(dev).requires_grad_() for nm in ("c0", "lam", "gam"))
@@ -375,10 +386,11 @@ def test_bf16_matrix_core_backward_matches_fp32_oracle(batch, n, upstream):
     assert all(e <= BF16_TOL for e in errs.values()), errs
 
 
-@pytest.mark.parametrize("batch,n", [(1, 64), (4, 1088)])
+@pytest.mark.parametrize("batch,n", [(1, 64), (64, 115), (4, 1088)])
 def test_bf16_state_scan_segmentation_is_invisible(batch, n):
-    """Both chunk-state scans run in one pass (one segment: N = 64, a single
-    chunk) or in S segments: at B = 4, N = 1088 (17 chunks) the forward's
+    """Both chunk-state scans run in one pass (one segment: B = 64, N = 115, two
+    chunks of 128 units) or in S segments (one sequence of 64 tokens goes over
+    token pairs): at B = 4, N = 1088 (17 chunks) the forward's
     segment scratch (its num buffer) holds 3 segments, so it runs totals, carry
     and replay over 3 segments of 6, 6 and 5 chunks, and the backward runs one
     local pass over each of 3 segments of 6, 6 and 5 chunks, their carries, and
@@ -388,6 +400,7 @@ def test_bf16_state_scan_segmentation_is_invisible(batch, n):
     from oal_amd.hd_block_gemm_autograd import grouped_oal
 
     dev = _dev()
+    assert takes_state(batch, 14, 2, n, 8, "bf16") == (n > 64)
     segments = f"B={batch} N={n}"
     inp = _bf16_case(batch, n, seed=9)
     qb, kb, vb = (inp[nm].to(torch.bfloat16).to(dev).requires_grad_() for nm in ("q", "k", "v"))

@@ -5,6 +5,8 @@ most or all of the query-side fold onto a stream of the library's own, makes the
 stream recorded before the key-side fold and before the rest of the query-side
 fold and the coefficient reductions, and joins it back into the caller's stream
 before it returns.
+Short sequences (the direct route) use no second stream; each case says which side
+of that line it is on.
 These tests call it on caller-created streams (not the default one), from two
 streams in turn, and consume the gradients on the caller's stream right after
 the call with no synchronization in between. Every result must be bitwise
@@ -17,6 +19,7 @@ import torch
 
 from oal_amd import _native
 from oracle import grouped_oracle as go
+from routes import takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -52,12 +55,16 @@ def _step(inp, precision="bf16"):
     return [t.clone() for t in (out, num, den, *grads)]
 
 
-@pytest.mark.parametrize("precision", ["bf16", "fp32"])
-def test_backward_on_caller_streams_is_joined_before_the_next_work(precision):
+@pytest.mark.parametrize("precision,b,n,state", [
+    ("bf16", 2, 1000, False), ("fp32", 2, 1000, False), ("bf16", 2, 1300, True), ("bf16", 1, 1700, True),
+    ("fp32", 1, 1700, True), ("fp32", 2, 2600, True)])
+def test_backward_on_caller_streams_is_joined_before_the_next_work(precision, b, n, state):
     """bf16: the matrix-core backward's fork; fp32: the fp32 route's forward and
-    backward forks."""
+    backward forks, with the key side in slices (54 (chunk, unit) pairs) and whole
+    (164). Not state: the direct route, one stream throughout."""
     dev = _dev()
-    inp = _inputs(dev)
+    assert takes_state(b, 14, 2, n, 8, precision) == state
+    inp = _inputs(dev, n=n, b=b)
     ref = _step(inp, precision)
     torch.cuda.synchronize()
     streams = [torch.cuda.Stream(dev), torch.cuda.Stream(dev)]
@@ -105,18 +112,21 @@ def test_other_stream_arrangements_are_joined(n, b, groups):
         assert torch.equal(res[-1], ref[4].float().sum())
 
 
-def test_two_caller_streams_with_their_own_inputs():
+@pytest.mark.parametrize("precision,na,nb,state", [
+    ("bf16", 700, 900, False), ("bf16", 1300, 1500, True), ("fp32", 1300, 1500, True)])
+def test_two_caller_streams_with_their_own_inputs(precision, na, nb, state):
     dev = _dev()
-    inp_a, inp_b = _inputs(dev, n=700, seed=1), _inputs(dev, n=900, seed=2)
-    ref_a, ref_b = _step(inp_a), _step(inp_b)
+    assert all(takes_state(2, 14, 2, n, 8, precision) == state for n in (na, nb))
+    inp_a, inp_b = _inputs(dev, n=na, seed=1), _inputs(dev, n=nb, seed=2)
+    ref_a, ref_b = _step(inp_a, precision), _step(inp_b, precision)
     torch.cuda.synchronize()
     sa, sb = torch.cuda.Stream(dev), torch.cuda.Stream(dev)
     sa.wait_stream(torch.cuda.current_stream(dev))
     sb.wait_stream(torch.cuda.current_stream(dev))
     with torch.cuda.stream(sa):
-        res_a = _step(inp_a)
+        res_a = _step(inp_a, precision)
     with torch.cuda.stream(sb):
-        res_b = _step(inp_b)
+        res_b = _step(inp_b, precision)
     torch.cuda.synchronize()
     for a, r in zip(res_a, ref_a):
         assert torch.equal(a, r)

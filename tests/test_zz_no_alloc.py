@@ -6,7 +6,9 @@ contents), each compared with oal_backward on the same inputs and a
 caller-allocated workspace, bitwise (every reduction of both routes has a fixed
 order), for 8 groups, 12 groups and per-pair coefficients (64 groups), whose
 workspaces differ (the per-pair bf16 layout adds per-head dk partials and local
-slot partials; more than 8 groups run the fp32 route's scalar kernels). A geometry whose workspace
+slot partials; more than 8 groups run the fp32 route's scalar kernels; 8 groups
+on both sides of the direct route's line, the fp32 state's with its key side in
+slices). A geometry whose workspace
 exceeds the 256 MiB scratch is refused with an error before anything runs.
 """
 
@@ -17,6 +19,7 @@ import torch
 
 from oal_amd import _native
 from oracle import grouped_oracle as go
+from routes import takes_state
 
 pytestmark = pytest.mark.gpu
 
@@ -78,14 +81,16 @@ def _rel(a, b):
     return float((a.double() - b.double()).norm() / b.double().norm())
 
 
-@pytest.mark.parametrize("precision,dtype,gcount", [
-    ("bf16", torch.bfloat16, 8), ("fp32", torch.float32, 8), ("bf16", torch.bfloat16, 12),
-    ("fp32", torch.float32, 12), ("bf16", torch.bfloat16, 64), ("fp32", torch.float32, 64)])
-def test_noalloc_backward_matches_the_workspace_entry_point(precision, dtype, gcount):
+@pytest.mark.parametrize("precision,dtype,gcount,longest,shortest", [
+    ("bf16", torch.bfloat16, 8, 1024, 200), ("fp32", torch.float32, 8, 1024, 200),
+    ("bf16", torch.bfloat16, 8, 1900, 1600), ("fp32", torch.float32, 8, 1900, 1600),
+    ("bf16", torch.bfloat16, 12, 1024, 200), ("fp32", torch.float32, 12, 1024, 200),
+    ("bf16", torch.bfloat16, 64, 640, 130), ("fp32", torch.float32, 64, 640, 130)])
+def test_noalloc_backward_matches_the_workspace_entry_point(precision, dtype, gcount, longest, shortest):
     dev = _dev()
     lib = _native.load_library()
-    shapes = ((1, 1024, 3), (1, 200, 4)) if gcount <= 12 else ((1, 640, 3), (1, 130, 4))
-    for call, (b, n, seed) in enumerate(shapes):
+    for call, (b, n, seed) in enumerate(((1, longest, 3), (1, shortest, 4))):
+        assert takes_state(b, 14, 2, n, gcount, precision, dtype) == (gcount > 8 or n >= 1600)
         print(f"noalloc call {call}: precision={precision} groups={gcount} B={b} N={n}", flush=True)
         q, k, v, labels, c0, lam, gam, scale, dout, dden = _inputs(b, n, dtype, seed, dev, gcount)
         _, num, den, saved = _native.forward(q, k, v, labels, c0, lam, gam, scale=scale, floor=0.0,
