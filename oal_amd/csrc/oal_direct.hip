@@ -130,17 +130,6 @@ struct Lay {
   static __device__ __forceinline__ constexpr int in_block(int p) { return F32 ? 4 * (p & 3) + (p >> 2) : p; }
 };
 
-// The further windows of groups of more than 16 dimensions, in LDS: few heads
-// have any, and in scalar registers they displace the coefficients.
-struct More {
-  int group[kMore], at[kMore], count[kMore];  // group -1: none
-  __device__ __forceinline__ void put(int slot, const Window& w) {
-    group[slot] = w.group;
-    at[slot] = w.at;
-    count[slot] = w.count;
-  }
-};
-
 template <bool F32, int GP>
 struct Shared {
   using L = Lay<F32, GP>;
@@ -148,7 +137,7 @@ struct Shared {
   Elem<F32> natural[kWv][kM][L::LN];
   Elem<F32> fixed[kM][L::LS];
   uint8_t dim[16 * L::kWin];  // fp32: window and position -> dimension, 255 where there is none
-  More more;
+  uint32_t more[kMore];  // further windows (Window::word)
   float zrow[kWv][kM];
   float co[kWv][coef_count(GP)];
 };
@@ -162,13 +151,13 @@ struct Head {
   int pos;           // its LDS position
   float gam, lam;    // lane 8 g + h: scale^2 gam[g][h]; lane g: scale lam[g]
   int at[GP], count[GP];  // a group's first window and its dimensions in it
-  bool any_more;          // whether some group has further windows
+  bool any_more;          // whether there are further windows (groups of more than 16 dimensions)
 };
 
 template <bool F32, int GP>
 __device__ __forceinline__ Head<F32, GP> read_head(const int32_t* __restrict__ labels, const float* __restrict__ lam,
                                                    const float* __restrict__ gam, int G, int h, float scale, int l,
-                                                   More& mw) {
+                                                   uint32_t (&more)[kMore]) {
   using L = Lay<F32, GP>;
   Head<F32, GP> t;
   const int x = l >> 3, y = l & 7;
@@ -178,8 +167,8 @@ __device__ __forceinline__ Head<F32, GP> read_head(const int32_t* __restrict__ l
   t.gam = x < G && y < G ? scale * scale * gv : 0.f;
   t.lam = l < G ? scale * lv : 0.f;
   WindowWalk<F32, GP> walk;
+  Window slot[kMore];
   t.pos = 0;
-  if (threadIdx.x < kMore) mw.put(threadIdx.x, Window{});
 #pragma unroll
   for (int g = 0; g < GP; ++g) {
     const uint64_t in = __ballot(t.lab == g);
@@ -189,9 +178,11 @@ __device__ __forceinline__ Head<F32, GP> read_head(const int32_t* __restrict__ l
     const int i = __builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in, 0));
     const int w = i < 16 ? t.at[g] : walk.next() + (i & ~15) - 16;
     t.pos = t.lab == g ? w + L::in_block(i & 15) : t.pos;
-    if ((int)threadIdx.x < walk.extra(n)) mw.put(walk.more + threadIdx.x, walk.further(threadIdx.x, g, n));
-    walk.pass(n);
+    walk.pass(g, n, slot);
   }
+  // in LDS, since few heads have any and in scalar registers they displace the coefficients
+  if (threadIdx.x < kMore)
+    more[threadIdx.x] = threadIdx.x == 0 ? slot[0].word : threadIdx.x == 1 ? slot[1].word : slot[2].word;
   t.any_more = walk.more > 0;
   return t;
 }
@@ -281,6 +272,11 @@ __device__ __forceinline__ Blk<F32> read_at(const Elem<F32>* tile, int offset) {
   Blk<F32> b;
   b.v = *reinterpret_cast<const decltype(b.v)*>(tile + offset);
   return b;
+}
+__device__ __forceinline__ Window more_window(const uint32_t (&more)[kMore], int m) {
+  Window w;
+  w.word = __builtin_amdgcn_readfirstlane(more[m]);
+  return w;
 }
 // The fixed operand of a window: zero past the group's own dimensions.
 __device__ __forceinline__ Blk<false> fixed_window(const uint16_t* row, int at, int count, int l) {
@@ -650,14 +646,19 @@ __device__ __forceinline__ void tiles(const Args<T, F32>& a, Shared<F32, GP>& sh
 #pragma unroll
     for (int g = 0; g < GP; ++g) s[g] = mma(read_at<F32>(srt, wo[g]), f1[g], f32x4{});
     if (any_more) {
-#pragma unroll
-      for (int x = 0; x < kMore; ++x) {
-        const f32x4 e = mma(read_window<F32>(srt + lr * L::LS, sh.more.at[x], l),
-                            fixed_window(&sh.fixed[lr][0], sh.more.at[x], sh.more.count[x], l), f32x4{});
+      // A scalar branch a slot and a group. As selects of all groups over all slots,
+      // present or not, it was 190 VALU instructions a tile: B=2, N=1000, 14 heads, sizes
+      // 22 and seven of 6, forward 54 us, 44 now (37 with no group beyond 16 dimensions),
+      // fp32 forward and backward 664, 536 now. Unrolled, it takes 50 more registers.
+#pragma unroll 1
+      for (int m = 0; m < kMore; ++m) {
+        const Window w = more_window(sh.more, m);
+        if (!w.present()) continue;
+        const Blk<F32> a1 = read_window<F32>(srt + lr * L::LS, w.at(), l),
+                       b1 = fixed_window(&sh.fixed[lr][0], w.at(), w.count(), l);
 #pragma unroll
         for (int g = 0; g < GP; ++g)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) s[g][r] += sh.more.group[x] == g ? e[r] : 0.f;
+          if (w.group() == g) s[g] = mma(a1, b1, s[g]);
       }
     }
     // tiles off the diagonal and inside the sequence: every pair counts
@@ -732,7 +733,11 @@ __device__ __forceinline__ void tiles(const Args<T, F32>& a, Shared<F32, GP>& sh
     if constexpr (!kSums) {
       if (want_grad) {
         f32x4 kap = {2.f * cf.c0, 2.f * cf.c0, 2.f * cf.c0, 2.f * cf.c0};  // twice kappa
-        f32x4 xm[kMore] = {};  // the tiles of the groups that hold the further blocks
+        Window w[kMore];
+        if (any_more) {
+#pragma unroll
+          for (int m = 0; m < kMore; ++m) w[m] = more_window(sh.more, m);
+        }
 #pragma unroll
         for (int g = 0; g < GP; ++g) {
           f32x4 x;
@@ -747,15 +752,9 @@ __device__ __forceinline__ void tiles(const Args<T, F32>& a, Shared<F32, GP>& sh
           if (any_more) {
 #pragma unroll
             for (int m = 0; m < kMore; ++m)
-#pragma unroll
-              for (int r = 0; r < 4; ++r) xm[m][r] = sh.more.group[m] == g ? x[r] : xm[m][r];
+              if (w[m].group() == g)
+                gacc[GP + m] = mma(xa, rows_operand(srt, L::LS, 16 * (GP + m), L::in_block(lr), l), gacc[GP + m]);
           }
-        }
-        if (any_more) {
-#pragma unroll
-          for (int m = 0; m < kMore; ++m)
-            gacc[GP + m] = mma(as_operand<F32>(xm[m]), rows_operand(srt, L::LS, 16 * (GP + m), L::in_block(lr), l),
-                               gacc[GP + m]);
         }
         if constexpr (MODE == kDkv) {
           kap *= 0.5f;
@@ -891,7 +890,7 @@ struct SharedRoles {
   uint16_t fnat[kM][L::LN];  // dq: q
   float gz[kStep];           // dk: Gz of the step's rows
   int grp[kD];               // dq: group of a dimension
-  More more;
+  uint32_t more[kMore];
   float dc0[kWv];
 };
 
@@ -948,7 +947,21 @@ __device__ __forceinline__ void roles(const Args<T, false>& a, SharedRoles<GP>& 
     fo[x] = fixed_window(&sh.fixed[lr][0], at, n, l);
     wown[x] = window_offset<false, GP>(at, l);
   }
-  const bool any_more = hd.any_more;
+  // and the further windows: place among the wave's own groups, fixed operand, offset.
+  // They all fall to the waves whose groups are long while the others wait, so their
+  // reads go out together (one head of 2400 tokens, sizes 57 and seven of 1, forward and
+  // backward 288 us read one after the other, 217 so)
+  int xm[kMore], wm[kMore];
+  Blk<false> fm[kMore];
+  bool own_more = false;
+#pragma unroll
+  for (int m = 0; m < kMore; ++m) {
+    const Window w = more_window(sh.more, m);
+    xm[m] = w.group() - wave * kOwn;
+    own_more |= xm[m] >= 0 && xm[m] < kOwn;
+    fm[m] = fixed_window(&sh.fixed[lr][0], w.at(), w.count(), l);
+    wm[m] = window_offset<false, GP>(w.at(), l);
+  }
   f32x4 P[kOwn][4] = {}, Pl = {};
   float c0sum = 0.f;
   const int fc = row0 + lr;
@@ -1000,17 +1013,19 @@ __device__ __forceinline__ void roles(const Args<T, false>& a, SharedRoles<GP>& 
 #pragma unroll
         for (int x = 0; x < kOwn; ++x)
           s[x] = mma(read_at<false>(&sh.sorted[r0][0], wown[x]), fo[x], f32x4{});
-        if (any_more) {
+        if (own_more) {
+          Blk<false> a1[kMore];
+#pragma unroll
+          for (int m = 0; m < kMore; ++m) a1[m] = read_at<false>(&sh.sorted[r0][0], wm[m]);
 #pragma unroll
           for (int m = 0; m < kMore; ++m) {
-            const int mg = __builtin_amdgcn_readfirstlane(sh.more.group[m]);
-            if (mg < wave * kOwn || mg >= (wave + 1) * kOwn) continue;
-            const f32x4 v = mma(read_window<false>(&sh.sorted[r0 + lr][0], sh.more.at[m], l),
-                                fixed_window(&sh.fixed[lr][0], sh.more.at[m], sh.more.count[m], l), f32x4{});
+            const f32x4 e = mma(a1[m], fm[m], f32x4{});
 #pragma unroll
             for (int x = 0; x < kOwn; ++x)
+              if (xm[m] == x) {
 #pragma unroll
-              for (int r = 0; r < 4; ++r) s[x][r] += mg == wave * kOwn + x ? v[r] : 0.f;
+                for (int r = 0; r < 4; ++r) s[x][r] += e[r];
+              }
           }
         }
         float y[4] = {ds[0], ds[1], ds[2], ds[3]};

@@ -6,11 +6,14 @@ namespace oal {
 
 constexpr int kMore = 3;  // further windows of a head: 64 dimensions hold at most three beyond each group's first 16
 
-// A window of 16 LDS positions that holds dimensions of one group. An absent one
-// (group -1) is a valid empty window, since the token-pair kernels read every
-// slot and drop what no group claims.
+// A further window packed into a word: its group, first position and count of
+// dimensions. An absent one is group 255, an empty window at position 0.
 struct Window {
-  int group = -1, at = 0, count = 0;
+  unsigned word = 255u << 16;
+  constexpr int group() const { return (int)(word >> 16); }
+  constexpr int at() const { return (int)(word >> 8 & 255u); }
+  constexpr int count() const { return (int)(word & 255u); }
+  constexpr bool present() const { return group() != 255; }
 };
 
 // Positions of the token-pair kernels' sorted rows (Lay in oal_direct.hip): groups
@@ -19,18 +22,22 @@ template <bool F32, int GP>
 struct WindowWalk {
   // the last window may start at the end
   static constexpr int kPositions = F32 ? 16 * (GP + kMore) : 64 + 3 * (GP - 1) + 16;
+  static_assert(kPositions <= 256, "a position fits a byte");
   int start = 0, more = 0;  // bf16: the group's first position; further windows so far
 
   constexpr int first(int g) const { return F32 ? 16 * g : start; }
   constexpr int next() const { return F32 ? 16 * (GP + more) : start + 16; }
-  // A group of n dimensions has extra(n) further windows; number i of them goes into slot more + i.
-  static constexpr int extra(int n) { return n > 16 ? (n + 15) / 16 - 1 : 0; }
-  constexpr Window further(int i, int g, int n) const {
-    const int left = n - 16 * (i + 1);
-    return Window{g, next() + 16 * i, left < 16 ? left : 16};
-  }
-  constexpr void pass(int n) {
-    more += extra(n);
+  // Passes group g of n dimensions; its further windows go into the next slots.
+  constexpr void pass(int g, int n, Window (&slot)[kMore]) {
+    if (n > 16) {
+      const int extra = (n + 15) / 16 - 1;
+      for (int m = 0; m < kMore; ++m) {
+        const int i = m - more, left = n - 16 * (i + 1);
+        if (i >= 0 && i < extra)
+          slot[m].word = (unsigned)g << 16 | (unsigned)(next() + 16 * i) << 8 | (unsigned)(left < 16 ? left : 16);
+      }
+      more += extra;
+    }
     start += (n + 3) & ~3;
   }
 };

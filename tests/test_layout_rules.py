@@ -22,15 +22,12 @@ def _run(tmp_path, source):
 
 
 def test_every_window_slot_is_inside_the_sorted_row(tmp_path):
-    """The token-pair kernels read all kMore slots of further windows as LDS
-    positions, present or not: as a block leaves them in memory that held
-    anything, each is an aligned window inside the row, and the windows hold all
-    64 dimensions. Every size of up to three groups, and random sizes of all."""
+    """The token-pair kernels read further windows at LDS positions: every slot, present
+    or not, is an aligned window inside the row, and the windows hold all 64
+    dimensions. Every size of up to three groups, and random sizes of all."""
     _run(tmp_path, r"""
 #include <cstdio>
 #include <cstdlib>
-#include <cstring>
-#include <new>
 #include <random>
 #include <vector>
 #include "oal_layout.hpp"
@@ -39,29 +36,25 @@ using namespace oal;
 template <bool F32, int GP>
 void check(const std::vector<int>& sizes) {
   using Walk = WindowWalk<F32, GP>;
-  alignas(Window) unsigned char memory[sizeof(Window) * kMore];
-  std::memset(memory, 0x7f, sizeof memory);
-  Window* const table = reinterpret_cast<Window*>(memory);
+  Window table[kMore];
   int held = 0;
-  for (int x = 0; x < kMore; ++x) new (table + x) Window;  // as read_head does
   Walk walk;
   for (int g = 0; g < GP; ++g) {
-    const int n = g < (int)sizes.size() ? sizes[g] : 0;
+    const int n = g < (int)sizes.size() ? sizes[g] : 0, before = walk.more;
     if (walk.first(g) % 4 || walk.first(g) < 0 || walk.first(g) + 16 > Walk::kPositions) std::exit(1);
     held += n < 16 ? n : 16;
-    if (walk.more + walk.extra(n) > kMore) std::exit(2);
-    for (int i = 0; i < walk.extra(n); ++i) table[walk.more + i] = walk.further(i, g, n);
-    walk.pass(n);
+    walk.pass(g, n, table);
+    if (walk.more > kMore || walk.more - before != (n > 16 ? (n + 15) / 16 - 1 : 0)) std::exit(2);
   }
   for (int x = 0; x < kMore; ++x) {
     const Window& w = table[x];
-    const bool ok = w.at >= 0 && w.at % 4 == 0 && w.at + 16 <= Walk::kPositions && w.group >= -1 && w.group < GP &&
-                    (w.group < 0 ? w.count == 0 : w.count > 0 && w.count <= 16);
+    const bool ok = w.at() >= 0 && w.at() % 4 == 0 && w.at() + 16 <= Walk::kPositions && w.present() == (x < walk.more) &&
+                    (w.present() ? w.group() < GP && w.count() > 0 && w.count() <= 16 : w.count() == 0 && w.at() == 0);
     if (!ok) {
-      std::printf("F32=%d GP=%d: window %d %d %d\n", F32, GP, w.group, w.at, w.count);
+      std::printf("F32=%d GP=%d: window %d %d %d\n", F32, GP, w.group(), w.at(), w.count());
       std::exit(3);
     }
-    held += w.count;
+    held += w.count();
   }
   if (held != 64) std::exit(4);
 }
