@@ -12,36 +12,41 @@ namespace oal {
 constexpr int kDirectTile = 16;  // tokens per tile edge
 
 // Whether a call takes the direct route: where a model of both routes' forward
-// and backward time on MI355X (microseconds, kernels alone) says that it is the
-// shorter one. A function of the geometry alone, so that the size queries and
-// both directions agree. A direct call costs its launches and the longest row,
-// its 16 x 16 tiles and its blocks of 16 rows; the state route its longer chain
-// of launches (in bf16 with 30 us for what the host takes longer over them) and
-// its rows. Measured, bf16, 14/2 heads and 8 groups, direct against state: B=1
-// N=128 46 / 216, N=512 90 / 238, N=1024 177 / 257, N=1300 233 / 266, N=1600 299 /
-// 277; B=2 N=800 196 / 274, N=1000 272 / 270, N=1200 335 / 315; B=8 N=512 394 /
-// 315; B=64 N=128 404 / 437, N=256 1011 / 929. fp32: B=1 N=256 93 / 438, N=1024
-// 426 / 586, N=1536 766 / 663; B=4 N=512 502 / 800, N=1024 1394 / 1202; B=64 N=256
-// 2589 / 3814. Up to 4 groups: bf16 B=1 N=1600 228 / 280, B=4 N=1024 408 / 321;
-// fp32 B=1 N=2048 629 / 769, B=4 N=1024 755 / 1171.
-// All measured with the blocks numbered head by head. Longest rows of all heads
-// first, a forward and backward take up to a quarter less (bf16 B=1 N=1024 160 to
-// 130, B=2 N=1000 256 to 219, B=16 N=256 246 to 202; fp32 B=1 N=1024 382 to 274; no
-// size slower), so the line is on the safe side for the direct route.
+// and backward time on MI355X (microseconds of the library's calls in turn) says
+// that it is the shorter one. A function of the geometry alone, so that the size
+// queries and both directions agree. A direct call costs its launches and the longest
+// row, its 16 x 16 tiles and its blocks of 16 rows; the state route its longer
+// chain of launches (in bf16 with 30 us for what the host takes longer over them)
+// and its rows. Measured forward and backward, direct against state, at 14/2 heads
+// and, last of each list, at the line:
+//   bf16, 8 groups   B=1 N=712 84 / 239, N=1139 155 / 254, N=1424 207 / 262; B=2 N=1008
+//                    212 / 254; B=4 N=704 225 / 283; B=16 N=336 305 / 404; B=64 N=144 412 / 560
+//   bf16, 4 groups   B=1 N=848 82 / 246, N=1356 158 / 257, N=1696 205 / 265; B=16 N=416 301 / 475
+//   fp32, 8 groups   B=1 N=744 192 / 506, N=1190 349 / 617, N=1488 472 / 640; B=4 N=944
+//                    804 / 1098; B=16 N=688 1915 / 2664; B=64 N=592 6083 / 8994
+//   fp32, 4 groups   B=1 N=1144 201 / 548, N=1830 398 / 694, N=2288 568 / 791; B=16 N=1344 3437 / 4580
+// The host does not see the labels, so the line also holds for heads whose groups are
+// long (sizes 57 and seven of 1: bf16 B=1 N=1424 253 / 258, fp32 B=16 N=688 2377 / 2781;
+// 61, 1, 1, 1: bf16 B=1 N=1696 239 / 265, fp32 B=16 N=1344 4720 / 4679). For even groups it
+// is on the safe side. It does not know the number of KV heads, which the state's scans
+// run over (measured with 1 to 32, none slower), nor 64-token chunks: many
+// sequences of a few tokens, and calls without a backward, take its line as it is.
 inline bool direct_route(bool f32, int groups, int B, int Hq, int N) {
   if (groups > 8 || (long)B * Hq > 65535) return false;
   const double nt = (N + kDirectTile - 1) / kDirectTile, blocks = (double)B * Hq * nt, tiles = blocks * (nt + 1) / 2,
                rows = (double)B * Hq * N;
   const bool few = groups <= 4;
-  // One or two heads: the time is the longest row's chain, 61 ns a token and direction
-  // (50 up to 4 groups) against the state's 21, which the terms below do not hold. One
-  // head, 8 groups: N=3000 197 / 232, N=3600 237 / 245, N=3900 253 / 249, N=4390 285 /
-  // 262; without gradients of the coefficients N=4416 273 / 248; two heads of one
-  // unit N=3392 239 / 234. Up to 4 groups: N=4400 231 / 261, N=5000 270 / 277, without
-  // coefficients N=5088 266 / 260.
-  if (!f32 && N > (few ? 4500 : 3200)) return false;
-  if (f32) return 60 + 0.03 * N + (few ? 0.0042 : 0.0082) * tiles + (few ? 0.06 : 0.085) * blocks < 420 + 0.0145 * rows;
-  return 35 + 0.02 * N + (few ? 0.0018 : 0.0027) * tiles + (few ? 0.05 : 0.055) * blocks < 230 + 0.0028 * rows;
+  // Fewer than four groups hold one of more than 16 dimensions, whose further windows cost more.
+  const double tile = f32 ? (groups > 4 ? 0.0082 : groups == 4 ? 0.0044 : 0.0048)
+                          : (groups > 4 ? 0.0027 : groups == 4 ? 0.0019 : 0.0021);
+  // One or two heads in bf16: the time is the longest row's chain, which the terms
+  // below do not hold, 61 to 82 ns a token with 8 groups against the state's 20. One
+  // head, even groups: N=3000 197 / 232, N=3900 253 / 249, N=4390 285 / 262; sizes 57
+  // and seven of 1: N=2400 218 / 221, N=3200 284 / 236. Four groups: N=4199 even 232 /
+  // 261, sizes 61, 1, 1, 1 N=3149 223 / 238, N=4199 291 / 259.
+  if (!f32 && N > (few ? 3200 : 2400)) return false;
+  if (f32) return 60 + 0.03 * N + tile * tiles + (few ? 0.06 : 0.085) * blocks < 420 + 0.0145 * rows;
+  return 35 + 0.02 * N + tile * tiles + (few ? 0.05 : 0.055) * blocks < 230 + 0.0028 * rows;
 }
 
 // Workspace of a direct backward.

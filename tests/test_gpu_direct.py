@@ -27,6 +27,8 @@ SIZES = {
     "wide": (1, 17, 33, 13),
     "empty": (16, 0, 31, 0, 17),
     "tail": (15, 15, 15, 15, 1, 1, 1, 1),
+    "long": (57, 1, 1, 1, 1, 1, 1, 1),
+    "second": (6, 22, 6, 6, 6, 6, 6, 6),
 }
 
 
@@ -98,10 +100,11 @@ def test_tile_edges(precision, dtype, n):
 
 
 @pytest.mark.parametrize("precision", ["bf16", "fp32"])
-@pytest.mark.parametrize("sizes", ["one", "wide", "empty", "tail"])
+@pytest.mark.parametrize("sizes", ["one", "wide", "empty", "tail", "long", "second"])
 @pytest.mark.parametrize("hq,hkv", [(1, 1), (9, 1)])
 def test_group_windows(precision, sizes, hq, hkv):
-    """(9, 1): more query heads per KV head than the bf16 kernels serve, so fp32 arithmetic in both."""
+    """No further window of a group of more than 16 dimensions, one, two and three of
+    them, in one group and in several. (9, 1): more query heads per KV head than the bf16 kernels serve, so fp32 arithmetic in both."""
     case, got, grads, up = _run(1, hq, hkv, 83, SIZES[sizes], precision, torch.float32, seed=len(SIZES[sizes]) + hq)
     _check(case, got, grads, up, TOL["fp32" if hq > 8 else precision])
 

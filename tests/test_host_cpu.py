@@ -214,6 +214,6 @@ def test_long_rows_of_few_heads_take_the_state_route_in_bf16():
     def direct(heads, n, groups, codes):
         return size(1, heads, 1, n, groups, *codes) <= 256
 
-    assert direct(1, 3200, 8, bf16) and not direct(1, 3300, 8, bf16) and not direct(2, 3300, 8, bf16)
-    assert direct(1, 4500, 4, bf16) and not direct(1, 4600, 4, bf16)
-    assert direct(1, 4100, 8, fp32) and direct(1, 5500, 4, fp32)
+    assert direct(1, 2400, 8, bf16) and not direct(1, 2500, 8, bf16) and not direct(2, 2500, 8, bf16)
+    assert direct(1, 3200, 4, bf16) and not direct(1, 3300, 4, bf16)
+    assert direct(1, 4100, 8, fp32) and direct(1, 5200, 4, fp32)
