@@ -31,10 +31,10 @@
 // sixteenth of the bf16 depth). The bf16 backward is in direct_dq and
 // direct_dk_dv (roles). In short sequences what counts is the chain from the first
 // load to the first tile, so every wave works its group structure out for itself
-// without a barrier; N = 64 takes 16 us forward and 28 us backward with the
-// launches, against 48 and 155 through the state. At full load the waves' VALU and matrix-core cycles add up
-// to the time (they hardly overlap): a step of 64 rows of the bf16 dq is 293 VALU
-// and 50 matrix instructions a wave.
+// without a barrier; N = 64, 14 heads, takes 7 us forward and 31 forward and
+// backward, against 44 and 197 through the state. At full load the waves' VALU and
+// matrix-core cycles add up to the time (they hardly overlap): a step of 64 rows of
+// the bf16 dq is about 360 VALU and 52 matrix instructions a wave.
 //
 // The dimensions are sorted by group in LDS, a window of 16 positions for each
 // group's first 16 dimensions and at most three more in all. A group's sum is then
