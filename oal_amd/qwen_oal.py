@@ -104,9 +104,16 @@ def apply_rotary(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch
     return x * cos + rot * sin
 
 
+def _unrotated(d: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+    """The transpose of :func:`apply_rotary`."""
+    half, y = d.shape[-1] // 2, d * sin
+    return d * cos + torch.cat((y[..., half:], -y[..., :half]), dim=-1)
+
+
 class _RotaryHeads(torch.autograd.Function):
     """The operator's q, k, v from the projections' [B, N, heads * 64] (one kernel each
-    way, oal_adapter.hip): head-first, q and k rotated."""
+    way, oal_adapter.hip): head-first, q and k rotated. A backward that is itself
+    recorded goes through the torch operations."""
 
     @staticmethod
     def forward(ctx, q, k, v, cos, sin, q_heads: int, kv_heads: int):
@@ -117,11 +124,13 @@ class _RotaryHeads(torch.autograd.Function):
                                     back=False)
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, dq, dk, dv):
         if dq is None and dk is None and dv is None:
             return (None,) * 7
         cos, sin = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            turned = [t if t is None else _unrotated(t, cos, sin) for t in (dq, dk)]
+            return (*(t if t is None else t.transpose(1, 2).flatten(2) for t in (*turned, dv)), None, None, None, None)
         grads = tuple(None if t is None else t.contiguous() for t in (dq, dk, dv))
         return (*_native.rotary_heads(grads, cos, sin, *ctx.heads, back=True), None, None, None, None)
 
@@ -129,10 +138,10 @@ class _RotaryHeads(torch.autograd.Function):
 def rotary_heads(q, k, v, cos, sin, q_heads: int, kv_heads: int, head_dim: int):
     """Projections [B, N, heads * D] -> head-first q, k, v [B, heads, N, D], q and k
     rotated. One kernel for the operator's own types and head dimension with
-    tables that need no gradient; otherwise :func:`apply_rotary`."""
+    tables that need no gradient, in eager calls; otherwise :func:`apply_rotary`."""
     b, n, _ = q.shape
     if (
-        head_dim == _native.HEAD_DIM and q.device.type == "cuda" and torch.version.hip is not None
+        head_dim == _native.HEAD_DIM and _native.ordinary(q, k, v, cos, sin)
         and q.dtype in (torch.float32, torch.bfloat16)
         and all(t.dtype == q.dtype and t.device == q.device for t in (k, v, cos, sin))
         and cos.shape == sin.shape == (n, head_dim) and not (cos.requires_grad or sin.requires_grad)

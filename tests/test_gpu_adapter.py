@@ -129,6 +129,31 @@ def test_rotary_heads(dtype, b, n, hq, hkv):
         assert float((a.detach().cpu().double() - r.detach()).norm() / r.detach().norm()) <= tol
 
 
+def test_rotary_heads_under_tracers_and_twice():
+    """What replaces the module's attention may be traced or differentiated twice: the
+    rotation is linear, so its gradient's gradient is the rotation again."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from oal_amd.qwen_oal import rotary_heads, rotary_tables
+
+    dev, n = _dev(), 7
+    cos, sin = rotary_tables(n, 64, 1e6, dev, torch.float32)
+    one, two = ([torch.randn((2, n, h * 64), device=dev) for h in (4, 2, 2)] for _ in range(2))
+
+    def turn(q, k, v):
+        return rotary_heads(q, k, v, cos, sin, 4, 2, 64)
+
+    for a, r in zip(make_fx(turn)(*one)(*two), turn(*two)):
+        assert torch.allclose(a, r, rtol=1e-6, atol=1e-6)
+    leaves = [t.requires_grad_() for t in one]
+    up = [torch.randn_like(t).requires_grad_() for t in turn(*two)]
+    grads = torch.autograd.grad(turn(*leaves), leaves, up, create_graph=True)
+    plain = torch.autograd.grad(turn(*leaves), leaves, [t.detach() for t in up])
+    assert all(torch.allclose(a, r, rtol=1e-6, atol=1e-6) for a, r in zip(grads, plain))
+    for a, r in zip(torch.autograd.grad(grads, up, two), turn(*two)):
+        assert torch.allclose(a, r, rtol=1e-6, atol=1e-6)
+
+
 def _prefix(row, groups):
     used = sorted(set(row))
     return 1 if any(x < 0 or x >= groups for x in row) else 0 if used == list(range(len(used))) else 2

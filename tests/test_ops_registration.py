@@ -111,3 +111,13 @@ def test_make_fx_traces_the_factor_expansion():
         gm = make_fx(fwd, tracing_mode="fake")(q, k, v, labels, *small)
     inputs = [n for n in gm.graph.nodes if n.op == "placeholder"]
     assert all(n.users for n in inputs)  # none baked in
+
+
+def test_rotary_heads_of_fake_tensors():
+    """A traced layer with an attention of its own sees the rotation's operations."""
+    from oal_amd.qwen_oal import rotary_heads
+
+    with FakeTensorMode():
+        cos = torch.empty(20, 64, device="cuda")
+        turned = rotary_heads(*(torch.empty(2, 20, 64 * h, device="cuda") for h in (14, 2, 2)), cos, cos, 14, 2, 64)
+        assert [tuple(t.shape) for t in turned] == [(2, 14, 20, 64), (2, 2, 20, 64), (2, 2, 20, 64)]
